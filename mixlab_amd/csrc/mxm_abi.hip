@@ -183,8 +183,6 @@ struct MoeOp {
   bool dec16 = false;
   DevBuf d1, d1b, d2;
   int n_cu = 256;        // CUs of the op's device
-  int fam1 = 0, fam2 = 0;  // MFMA tile families of the up and down GEMMs
-  int fam_dh = 0;           // ... of the backward's dH = dY W_down^T (dX uses fam2)
   std::vector<char> have;
 
   // tile schedule of the forward (set at create from the op's parameters)
@@ -235,7 +233,7 @@ struct MoeOp {
   // bf16 ops of the MFMA family: bf16 intermediates of the MFMA backward and
   // the weights re-laid for its products (W_down [F][D], W1 [D][NC])
   bool bw_wbf_ready = false;
-  DevBuf bw_dhb, bw_gub, bw_dgub, bw_dxeb, bw_zero, bw_ms, bw_w2o, bw_w1u, bw_wscr,
+  DevBuf bw_dhb, bw_gub, bw_dgub, bw_dxeb, bw_zero, bw_w2o, bw_w1u, bw_wscr,
       bw_ddb, bw_gp, bw_dgp, bw_dlb, bw_dwr2;
   // the fp32 backward's products (run_backward_x3): bf16 planes of the
   // operands at the padded widths Dq x Fq, fp32 products
@@ -359,22 +357,17 @@ void set_schedule(MoeOp& o) {
   if (o.int8_kernels()) {
     o.bm1 = o.bm2 = 256;  // tile schedules are not used by the int8 kernels
   } else if (o.mfma) {
-    // Unless a family was requested: 256 x 256 tiles where the columns allow
-    // and the launch has at least two tiles per CU, else 128 x 128 (a grid
-    // of one 256 x 256 tile per CU spends its time in each tile's ramp and
-    // epilogue: C2's down projection 99 -> 92 us)
-    auto pick = [&](int ncols) {
-      if (o.family != MXM_TILE_AUTO) return o.family;
-      if (ncols % 256 != 0) return (int)MXM_TILE_128x128;
+    // Unless a family was requested, the scheduled kernel: it plans 256 x 256
+    // and 128 x 128 tiles from the experts' row counts.  bm is then the height
+    // that most rows run at: 256 where the columns allow and the launch has
+    // at least two such tiles per CU.
+    auto rows = [&](int ncols, int kd) {
       const int64_t tiles = ((int64_t)NK + 255) / 256 * (ncols / 256);
-      return tiles < 2 * (int64_t)o.n_cu ? (int)MXM_TILE_128x128 : (int)MXM_TILE_256x256;
+      if (o.family == MXM_TILE_AUTO && (ncols % 256 != 0 || tiles < 2 * (int64_t)o.n_cu)) return 128;
+      return mxm_mfma_tile_rows(ncols, kd, o.family);
     };
-    const int nc1 = glu ? 2 * o.Fk : o.Fk;
-    o.fam1 = pick(nc1);
-    o.fam2 = pick(o.Dk);
-    o.fam_dh = pick(o.Fk);
-    o.bm1 = mxm_mfma_tile_rows(nc1, o.Kx, o.fam1);
-    o.bm2 = mxm_mfma_tile_rows(o.Dk, o.hsplit ? 2 * o.Fk : o.Fk, o.fam2);
+    o.bm1 = rows(glu ? 2 * o.Fk : o.Fk, o.Kx);
+    o.bm2 = rows(o.Dk, o.hsplit ? 2 * o.Fk : o.Fk);
   } else {
     // 64 x 64 tiles where their grid covers every CU, else 32 x 32 (C1's
     // down projection: 72 tiles of 64 x 64 for 256 CUs); MXM_SIMT_TILE (32
@@ -443,7 +436,7 @@ void alloc_workspace(MoeOp& o) {
 // Refuse to launch a GEMM whose operands are not all allocated (a kernel
 // would otherwise read through a null pointer).
 void require_operands(const GemmArgs& g, bool second_matrix, bool scaled) {
-  if (!g.a || !g.b0 || !g.out || !g.offsets || !g.mstart || (second_matrix && !g.b1) ||
+  if (!g.a || !g.b0 || !g.out || !g.offsets || (second_matrix && !g.b1) ||
       (scaled && (!g.scale0 || (g.mode == MXM_GEMM_GLU && !g.scale1))) ||
       (g.mode != MXM_GEMM_DOWN && !g.perm))
     fail_rt("OP_MOE_FEED_FORWARD internal error: expert GEMM operand not allocated (mode %d)", g.mode);
@@ -636,7 +629,7 @@ void run_forward(MoeOp& o, const Workspace& w, const void* x, int x_dtype, float
   g1.max_mtiles = o.max_mtiles1;
   g1.simt_bm = o.bm1;
   g1.simt_vec = o.simt_vec;
-  g1.family = o.fam1;
+  g1.family = o.family;
   g1.expert_type = o.etype;
   g1.activation = o.act;
   g1.slope = o.slope;
@@ -708,7 +701,7 @@ void run_forward(MoeOp& o, const Workspace& w, const void* x, int x_dtype, float
   g2.max_mtiles = o.max_mtiles2;
   g2.simt_bm = o.bm2;
   g2.simt_vec = o.simt_vec;
-  g2.family = o.fam2;
+  g2.family = o.family;
   g2.expert_type = o.etype;
   g2.activation = o.act;
   g2.slope = o.slope;
@@ -1482,7 +1475,6 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
     o.bw_dxeb.alloc(NK * D * 2);
     o.bw_zero.alloc(512);  // 256 zero bf16: the weight gradients' rows past an expert's end
     HIPCK(hipMemsetAsync(o.bw_zero.p, 0, 512, st));
-    o.bw_ms.alloc(3 * ((size_t)E + 1) * 4);
     // the weight gradients' schedule and split-reduction partials (both
     // launches run in stream order and share it)
     o.bw_wscr.alloc(std::max({mxm_wgrad_scratch_bytes(D, NC), mxm_wgrad_scratch_bytes(Fk, D),
@@ -1515,13 +1507,8 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
   // gate on its left operand, so no per-slot dY = gate * dD is written)
   mxm_launch_dy_gate(b.d_delta, b.gates, b.slot_pos, o.N, D, o.K, ddb, nullptr,
                      o.bw_gp.as<float>(), st);
-  // families as the forward picks them for the same output width (dX has
-  // the down projection's, D)
-  auto product = [&](int which, const uint16_t* A, const void* W, uint16_t* out, int Kd, int Ncols,
-                     int family, bool gather) {
-    const int bm = mxm_mfma_tile_rows(Ncols, Kd, family);
-    int32_t* ms = o.bw_ms.as<int32_t>() + (size_t)which * (E + 1);
-    mxm_launch_tile_prefix(b.counts, E, bm, ms, st);
+  auto product = [&](const uint16_t* A, const void* W, uint16_t* out, int Kd, int Ncols,
+                     bool gather) {
     GemmArgs g{};
     g.no_off32 = o.force64;
     g.mode = MXM_GEMM_DOWN;
@@ -1529,12 +1516,10 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
     g.b0 = W;
     g.out = out;
     g.offsets = b.offsets;
-    g.mstart = ms;
     g.E = E;
     g.Kd = Kd;
     g.Ncols = Ncols;
-    g.max_mtiles = (int)((NK + bm - 1) / bm) + E;
-    g.family = family;
+    g.family = o.family;
     g.gather_a = gather;  // A rows = token rows through perm
     g.perm = b.perm;
     g.rows_total = (int)NK;
@@ -1544,7 +1529,7 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
   };
   // dH' = dD W_down^T for each slot's token, ungated: with H it gives the
   // gate gradients <dD, Y> = <dH', h>, and dH = gate * dH'
-  product(0, ddb, o.bw_w2o.p, dhb, D, Fk, o.fam_dh, true);
+  product(ddb, o.bw_w2o.p, dhb, D, Fk, true);
   // gub holds G|U from the forward (run_forward's pre_out)
   mxm_launch_act_bw_gated_bf16(gub, dhb, static_cast<uint16_t*>(o.ws.H), o.hsplit,
                                o.bw_gp.as<float>(), (int)NK, Fk, o.etype, o.act, o.slope, dgub,
@@ -1581,7 +1566,7 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
     mxm_launch_dwr_halves(o.bw_dwr2.as<float>(), D, E, Ep, b.dwr, st);
     HIPCK(hipGetLastError());
   }
-  product(2, dgub, o.bw_w1u.p, dxeb, NC, D, o.fam2, false);
+  product(dgub, o.bw_w1u.p, dxeb, NC, D, false);
   if (b.dxr)
     mxm_launch_dx_bf16(b.dxr, dxeb, b.slot_pos, o.N, D, o.K, dx, st);
   else
@@ -1641,15 +1626,6 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
   HIPCK(hipGetLastError());
 }
 
-// MFMA tile family for a product with Ncols output columns over `rows`
-// rows: 256 x 256 where the columns allow and there are at least two tiles
-// per CU, else 128 x 128 (as the forward's schedule picks them).
-int product_family(const MoeOp& o, int ncols, size_t rows) {
-  if (ncols % 256 != 0) return MXM_TILE_128x128;
-  const int64_t tiles = ((int64_t)rows + 255) / 256 * (ncols / 256);
-  return tiles < 2 * (int64_t)o.n_cu ? (int)MXM_TILE_128x128 : (int)MXM_TILE_256x256;
-}
-
 // The fp32 backward after the routing (fp32 compute, or the bf16 flow on
 // fp32 copies where the MFMA backward does not apply).  Every product of the
 // experts runs on the library's bf16 MFMA kernels as the product of the
@@ -1696,7 +1672,6 @@ void run_backward_x3(MoeOp& o, BackwardArgs& b, bool own_forward) {
       o.bw_zero.alloc(512);  // 256 zero bf16: the weight gradients' rows past an expert's end
       HIPCK(hipMemsetAsync(o.bw_zero.p, 0, 512, st));
     }
-    if (!o.bw_ms.p) o.bw_ms.alloc(3 * ((size_t)E + 1) * 4);
     o.bw_wscr.alloc(std::max(mxm_wgrad_scratch_bytes(Dq, NCq), mxm_wgrad_scratch_bytes(Fq, Dq)));
     o.bx_w_ready = false;
   }
@@ -1712,15 +1687,11 @@ void run_backward_x3(MoeOp& o, BackwardArgs& b, bool own_forward) {
   float *gu = o.bx_gu.as<float>(), *dh = o.bx_dh.as<float>(), *dxe = o.bx_dxe.as<float>();
   // grouped product out [NK][Ncols] fp32 = A [NK][Kd] (rows through perm when
   // gather) . B_e^T (B_e [Ncols][Kd] per expert)
-  auto product = [&](int which, const uint16_t* A, const uint16_t* W, float* out, int Kd,
-                     int Ncols, bool gather) {
-    const int family = product_family(o, Ncols, NK);
-    const int bm = mxm_mfma_tile_rows(Ncols, Kd, family);
-    if (bm <= 0)
+  auto product = [&](const uint16_t* A, const uint16_t* W, float* out, int Kd, int Ncols,
+                     bool gather) {
+    if (mxm_mfma_tile_rows(Ncols, Kd, MXM_TILE_AUTO) <= 0)
       fail("OP_MOE_FEED_FORWARD backward: a %d x %d expert product exceeds the MFMA tiles' "
            "addressing", Ncols, Kd);
-    int32_t* ms = o.bw_ms.as<int32_t>() + (size_t)which * (E + 1);
-    mxm_launch_tile_prefix(b.counts, E, bm, ms, st);
     GemmArgs g{};
     g.no_off32 = o.force64;
     g.mode = MXM_GEMM_DOWN;
@@ -1729,12 +1700,10 @@ void run_backward_x3(MoeOp& o, BackwardArgs& b, bool own_forward) {
     g.b0 = W;
     g.out = out;
     g.offsets = b.offsets;
-    g.mstart = ms;
     g.E = E;
     g.Kd = Kd;
     g.Ncols = Ncols;
-    g.max_mtiles = (int)((NK + bm - 1) / bm) + E;
-    g.family = family;
+    g.family = MXM_TILE_AUTO;
     g.gather_a = gather;
     g.perm = b.perm;
     g.rows_total = (int)NK;
@@ -1776,14 +1745,14 @@ void run_backward_x3(MoeOp& o, BackwardArgs& b, bool own_forward) {
     mxm_launch_gemm_simt(g, false, st);
     HIPCK(hipGetLastError());
   } else {
-    product(0, x3, o.bx_w1p.as<uint16_t>(), gu, 3 * Dq, NCq, true);
+    product(x3, o.bx_w1p.as<uint16_t>(), gu, 3 * Dq, NCq, true);
   }
   mxm_launch_hidden_planes3(gu, (int64_t)NK, Fq, o.etype, o.act, o.slope, h3, st);
   HIPCK(hipGetLastError());
   if (own_forward) {
     // the expert outputs Y = H W_down, which the gate gradients read
     float* y = static_cast<float*>(o.ws.Y);
-    product(1, h3, o.bx_w2p.as<uint16_t>(), Dq == D ? y : o.bx_y.as<float>(), 3 * Fq, Dq, false);
+    product(h3, o.bx_w2p.as<uint16_t>(), Dq == D ? y : o.bx_y.as<float>(), 3 * Fq, Dq, false);
     if (Dq != D) mxm_launch_rows_to_f32(o.bx_y.p, MXM_DTYPE_F32, (int64_t)NK, D, Dq, y, st);
     HIPCK(hipGetLastError());
   }
@@ -1791,10 +1760,10 @@ void run_backward_x3(MoeOp& o, BackwardArgs& b, bool own_forward) {
   HIPCK(hipGetLastError());
   // dH = dY W_down^T, the activation backward, dXe = dGU W1^T, dx
   mxm_launch_planes3(b.dy, (int64_t)NK, D, D, Dq, true, dy3, st);
-  product(1, dy3, o.bx_w2t.as<uint16_t>(), dh, 3 * Dq, Fq, false);
+  product(dy3, o.bx_w2t.as<uint16_t>(), dh, 3 * Dq, Fq, false);
   mxm_launch_act_bw_planes3(gu, dh, (int64_t)NK, Fq, o.etype, o.act, o.slope, dgu3, st);
   HIPCK(hipGetLastError());
-  product(2, dgu3, o.bx_w1t.as<uint16_t>(), dxe, 3 * NCq, Dq, false);
+  product(dgu3, o.bx_w1t.as<uint16_t>(), dxe, 3 * NCq, Dq, false);
   mxm_launch_dx_sum(b.dxr, dxe, Dq, b.slot_pos, o.N, D, o.K, b.dx, st);
   HIPCK(hipGetLastError());
   // weight gradients: dW1 = Xp^T dGU over the plane pairs (x hi, dGU hi),

@@ -838,19 +838,6 @@ int wgrad_router_chunks_impl(int N, int D, int E) {
   return (int)c;
 }
 
-// Row-tile prefix of a grouped GEMM family with tile height bm:
-// mstart[e] = sum over e' < e of ceil(counts[e'] / bm), e = 0..E.
-__global__ void tile_prefix_kernel(const int32_t* counts, int E, int bm, int32_t* mstart) {
-  if (threadIdx.x != 0) return;
-  int m = 0;
-  for (int e = 0; e < E; ++e) {
-    mstart[e] = m;
-    m += (counts[e] + bm - 1) / bm;
-  }
-  mstart[E] = m;
-}
-
-
 // ---- the fp32 backward's products on the bf16 MFMA kernels ----
 // An fp32 value v is carried as two bf16 planes, hi = bf16(v) and lo =
 // bf16(v - hi) (|v - hi - lo| <= 2^-18 |v|), and an fp32 product A . B as
@@ -1005,10 +992,6 @@ __global__ void dx_sum_kernel(const float* __restrict__ dxr, const float* __rest
 }  // namespace
 
 int wgrad_router_chunks(int N, int D, int E) { return wgrad_router_chunks_impl(N, D, E); }
-
-void mxm_launch_tile_prefix(const int32_t* counts, int E, int bm, int32_t* mstart, hipStream_t s) {
-  hipLaunchKernelGGL(tile_prefix_kernel, dim3(1), dim3(64), 0, s, counts, E, bm, mstart);
-}
 
 void mxm_launch_dx_fused_bf16(const float* dlogits, const float* wrt, int E, const uint16_t* dxe,
                               const int32_t* slot_pos, int N, int D, int K, float* dx,

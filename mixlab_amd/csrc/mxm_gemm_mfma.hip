@@ -16,31 +16,35 @@
 // the background.  With three or more stages the barrier of stage kt+1 is
 // taken before the last k step of stage kt, so it overlaps MFMA work.
 //
-// Tile families (flags select; the default is 256 x 256 where the columns
-// allow): 256 x 256 x 64 (8 waves as 2 x 4, each 128 x 64 = 4 x 2 MFMA tiles,
-// 2 stages), 256 x 128 x 32 (4 waves, 3 stages, 2 workgroups per CU) and
-// 128 x 128 x 64 (4 waves, 2 stages).  The GLU weight rows are interleaved in
-// groups of 32 (gate cols f..f+31, then up cols f..f+31), so a wave's two
-// column MFMA tiles hold gate and up for the same 32 hidden units and the
-// activation is applied straight from the accumulators.
+// Tile shapes: 256 x 256 x 64 (8 waves as 2 x 4, each 128 x 64 = 4 x 2 MFMA
+// tiles, 2 stages, one workgroup per CU), 256 x 128 x 32 (4 waves, 3 stages)
+// and 128 x 128 x 64 (4 waves, 2 stages; two workgroups per CU), and 128 x
+// 128 x 64 with four more waves that do the loading (4 stages).  By default a
+// launch mixes 256 x 256 and 128 x 128 tiles (gemm_sched_kernel) or takes 128
+// x 128 ones in pairs (mxm_launch_gemm_mfma); flags select one shape.  The
+// GLU weight rows are interleaved in groups of 32 (gate cols f..f+31, then up
+// cols f..f+31), so a wave's two column MFMA tiles hold gate and up for the
+// same 32 hidden units and the activation is applied straight from the
+// accumulators.
 //
-// Ragged experts: the scan kernel writes `mstart`, the prefix over experts of
-// ceil(count/BM) row tiles, so tile -> (expert, rows) is resolved on device
-// (one round of loads and a ballot) and tiles past the end are skipped.
+// Ragged experts: every workgroup computes the tiles of the launch from the
+// experts' offsets (prefixes of their row tiles in LDS), so a tile's expert
+// and rows are resolved without a launch or a memory lookup for it.
 //
 // The grid is persistent: as many workgroups as fit on the device at once,
-// each walking launch indices w, w + gridDim.x, ...; a CU goes from one
-// tile's epilogue straight to the next tile while the stores drain, instead
-// of waiting for the workgroup to retire and a new one to be dispatched.
+// each walking its places of the tile list; a CU goes from one tile's
+// epilogue straight to the next tile while the stores drain, instead of
+// waiting for the workgroup to retire and a new one to be dispatched.
 //
-// Tile order: the hardware hands workgroup L to XCD L % 8.  Row tiles are
-// grouped GM at a time with the column tiles of a group adjacent, and group g
-// is placed on XCD g % 8, so each XCD's L2 sees a GM x (N/BN) block of tiles
-// sharing A rows and B columns, and the empty tail tiles are spread over all
-// XCDs.  The epilogue applies the activation (hardware exp2 / rcp and bf16
-// conversion), stages each wave's bf16 tile through LDS (chunk-swizzled) and
-// writes 16-byte row segments.
+// Tile order: row tiles are grouped GM at a time with the column tiles of a
+// group adjacent, and each XCD (the hardware hands workgroup L to XCD L % 8)
+// takes a contiguous eighth of that list, so its L2 sees a GM x (N/BN) block
+// of tiles sharing A rows and B columns and every CU gets the same number of
+// tiles to within one.  The epilogue applies the activation (hardware exp2 /
+// rcp and bf16 conversion), stages each wave's bf16 tile through LDS
+// (chunk-swizzled) and writes 16-byte row segments.
 #include <algorithm>
+#include <type_traits>
 
 #include "mxm_kernels.h"
 
@@ -75,48 +79,6 @@ __device__ __forceinline__ int swz(int row, int kc) {
   return row * CH + swz_phys<CH>(row, kc);
 }
 
-__device__ __forceinline__ int find_expert(const int32_t* mstart, int E, int mtile) {
-  int lo = 0, hi = E - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (mstart[mid] <= mtile)
-      lo = mid;
-    else
-      hi = mid - 1;
-  }
-  return lo;
-}
-
-// Row tile mtile -> its expert e, first row row0 and the expert's row end.
-// Returns false for tiles past the last expert's.  For E <= 64 this is one
-// round of independent loads: lane l reads mstart[l + 1], offsets[l] and
-// offsets[l + 1]; since mstart is nondecreasing from mstart[0] = 0, e is the
-// number of i in 1..E-1 with mstart[i] <= mtile (a ballot), and the rest are
-// read from the lanes holding them.  A binary search would be log2(E)
-// dependent loads, each a full L2 round trip, before the tile's first
-// operand load could be issued.
-__device__ __forceinline__ bool locate_tile(const int32_t* mstart, const int32_t* offsets, int E,
-                                            int mtile, int BM, int& e, int& row0, int& rend) {
-  if (E <= 64) {
-    const int lane = threadIdx.x & 63;
-    const bool in = lane < E;
-    const int ms1 = in ? mstart[lane + 1] : 0x7fffffff;
-    const int of0 = in ? offsets[lane] : 0;
-    const int of1 = in ? offsets[lane + 1] : 0;
-    if (mtile >= __builtin_amdgcn_readlane(ms1, E - 1)) return false;
-    e = __popcll(__ballot(lane + 1 < E && ms1 <= mtile));
-    const int ms_e = e == 0 ? 0 : __builtin_amdgcn_readlane(ms1, e - 1);
-    row0 = __builtin_amdgcn_readlane(of0, e) + (mtile - ms_e) * BM;
-    rend = __builtin_amdgcn_readlane(of1, e);
-    return true;
-  }
-  if (mtile >= mstart[E]) return false;
-  e = find_expert(mstart, E, mtile);
-  row0 = offsets[e] + (mtile - mstart[e]) * BM;
-  rend = offsets[e + 1];
-  return true;
-}
-
 // Direct global->LDS load of 16 bytes per lane (global_load_lds_dwordx4):
 // lane l's data lands at LDS address `lds` + 16*l.  Issued as inline asm so
 // the compiler does not track it: its conservative tracking of LDS DMA would
@@ -148,30 +110,37 @@ __device__ __forceinline__ void stage_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
 }
 
+// The barrier of a wave with no loads in flight: its LDS reads are done.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
+}
+
 // Tile family: BM x BN workgroup tile, WM x WN waves, each wave
-// (BM/WM) x (BN/WN) = TM x TN MFMA 32x32 tiles.
-template <int BM, int BN, int WM, int WN, int WAVES_PER_SIMD, int NSTAGE, int BKK>
+// (BM/WM) x (BN/WN) = TM x TN MFMA 32x32 tiles.  With LOADERS, that many
+// more waves issue all the loads and the computing waves none.
+template <int BM, int BN, int WM, int WN, int WAVES_PER_SIMD, int NSTAGE, int BKK, int LOADERS = 0>
 struct Tile {
   static constexpr int NS = NSTAGE;
   static constexpr int BK = BKK;      // k per LDS stage
   static constexpr int CH = BKK / 8;  // 16-byte chunks per tile row
-  static constexpr int NT = 64 * WM * WN;
+  static constexpr int CW = WM * WN;  // computing waves
+  static constexpr int LW = LOADERS > 0 ? LOADERS : CW;  // waves that load
+  static constexpr int NT = 64 * (CW + LOADERS);
   static constexpr int TM = BM / WM / 32;
   static constexpr int TN = BN / WN / 32;
   static constexpr int A_CH = BM * CH;
   static constexpr int B_CH = BN * CH;
   static constexpr int BUF = A_CH + B_CH;
-  static constexpr int LA = A_CH / NT;
-  static constexpr int LB = B_CH / NT;
   static constexpr int WPS = WAVES_PER_SIMD;
   static_assert(TN % 2 == 0, "GLU epilogue pairs gate and up column tiles");
-  static_assert(A_CH % NT == 0 && B_CH % NT == 0, "whole chunks per thread");
+  static_assert(A_CH % (64 * LW) == 0 && B_CH % (64 * LW) == 0, "whole chunks per thread");
 };
 
+// One BM x BN tile: rows row0 .. row0 + rows - 1 of expert e (rows <= BM) by
+// columns n0 .. n0 + BN - 1, with the LDS ring (NS * BUF chunks) at lds.
 template <class TL, int BM, int BN, int WM, int WN, int EPI>
-__global__ __launch_bounds__(TL::NT, TL::WPS * 256 / TL::NT) void gemm_kernel(GemmArgs a,
-                                                                            int ngroups,
-                                                                            int nblocks) {
+__device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e, int row0,
+                                          int rows, int n0) {
   constexpr int MODE = Epi<EPI>::MODE;
   constexpr bool DOWN_SPLIT = Epi<EPI>::DOWN_SPLIT;  // A = [hi | lo] planes, y in fp32
   // 32-bit A offsets (when A fits) for the forward's up projections only:
@@ -181,32 +150,9 @@ __global__ __launch_bounds__(TL::NT, TL::WPS * 256 / TL::NT) void gemm_kernel(Ge
   constexpr bool H_SPLIT = Epi<EPI>::H_SPLIT;        // H stored as [hi | lo] planes
   constexpr int NT = TL::NT, TM = TL::TM, TN = TL::TN;
   constexpr int A_CH = TL::A_CH, BUF = TL::BUF;
-  constexpr int NW = NT / 64;
+  constexpr int NW = NT / 64, LW = TL::LW;
   constexpr int NS = TL::NS;  // LDS stages in the ring (NS-1 in flight)
   constexpr int BK = TL::BK, CH = TL::CH;
-  __shared__ u32x4_t lds[NS * BUF];
-
-  // XCD-aware grouped schedule (see the file comment).
-  const int ntile_n = a.Ncols / BN;
-  const int per_group = GM * ntile_n;
-  // The grid is persistent (as many workgroups as fit at once): workgroup w
-  // takes launch indices w, w + gridDim.x, ..., so the CU goes straight from
-  // one tile's epilogue to the next tile while the epilogue's stores drain.
-  // gridDim.x is a multiple of 8, so every index keeps the workgroup's XCD.
-  for (int L = blockIdx.x; L < nblocks; L += gridDim.x) {
-  // every wave has read the previous tile's epilogue staging out of LDS
-  // (plain s_barrier: no wait for that epilogue's stores)
-  if (L != (int)blockIdx.x) asm volatile("s_barrier" ::: "memory");
-  const int local = L >> 3;
-  const int g = (local / per_group) * 8 + (L & 7);
-  if (g >= ngroups) break;  // g only grows with L
-  const int rr = local % per_group;
-  const int mtile = g * GM + rr % GM;
-  const int ntile = rr / GM;
-  int e, row0, rend;
-  if (!locate_tile(a.mstart, a.offsets, a.E, mtile, BM, e, row0, rend)) continue;
-  const int rows = min(BM, rend - row0);
-  const int n0 = ntile * BN;
   const int Kd = a.Kd;
 
   const int tid = threadIdx.x;
@@ -246,30 +192,34 @@ __global__ __launch_bounds__(TL::NT, TL::WPS * 256 / TL::NT) void gemm_kernel(Ge
   // fetches the logical k-chunk stored there -- the swizzle is applied on the
   // global address.
   constexpr int RPW = 64 / CH;     // tile rows per wave-load
-  constexpr int QA = BM / RPW / NW;  // A wave-loads per wave per stage
-  constexpr int QB = BN / RPW / NW;
+  constexpr int QA = BM / RPW / LW;  // A wave-loads per wave per stage
+  constexpr int QB = BN / RPW / LW;
   constexpr int LDPS = QA + QB;      // direct-to-LDS loads per thread per stage
-  static_assert(QA * RPW * NW == BM && QB * RPW * NW == BN, "whole wave-loads");
+  static_assert(QA * RPW * LW == BM && QB * RPW * LW == BN, "whole wave-loads");
+  constexpr bool LOADERS = LW != NW;
+  // this wave's place among the loading waves (a computing wave of a tile
+  // with loaders: any)
+  const int lwave = LOADERS ? (wave >= TL::CW ? wave - TL::CW : 0) : wave;
   const int lrow = lane / CH;  // row within the wave-load group
   // Logical chunk of this lane's physical slot (the swizzle is an involution).
   // It depends on the tile row modulo 16; the row of load i is
-  // (wave + NW*i)*RPW + lrow, which is the same modulo 16 for every i because
-  // NW*RPW is a multiple of 16.
-  static_assert((NW * RPW) % 16 == 0, "swizzle phase is the same for every wave-load of a lane");
-  const int lkc = swz_phys<CH>(wave * RPW + lrow, lane % CH);
+  // (lwave + LW*i)*RPW + lrow, which is the same modulo 16 for every i because
+  // LW*RPW is a multiple of 16.
+  static_assert((LW * RPW) % 16 == 0, "swizzle phase is the same for every wave-load of a lane");
+  const int lkc = swz_phys<CH>(lwave * RPW + lrow, lane % CH);
   size_t aoff[QA];
 #pragma unroll
   for (int i = 0; i < QA; ++i) {
-    const int r = (wave + NW * i) * RPW + lrow;
+    const int r = (lwave + LW * i) * RPW + lrow;
     const int p = row0 + min(r, rows - 1);  // rows past the segment reload a valid row
     const int src = (MODE == MXM_GEMM_DOWN && !a.gather_a) ? p : a.perm[p];
     aoff[i] = 2 * ((size_t)src * Kd + lkc * 8);  // bytes
   }
-  const size_t bstep = (size_t)(NW * RPW) * Kb;
+  const size_t bstep = (size_t)(LW * RPW) * Kb;
   // the B loads as 32-bit byte offsets from the expert's matrix (one expert's
   // Ncols x Kb bf16 stays far below 4 GiB); the wave index in an SGPR keeps
   // every load's LDS destination scalar
-  const int wv = __builtin_amdgcn_readfirstlane(wave);
+  const int wv = __builtin_amdgcn_readfirstlane(lwave);
   const unsigned boff = (unsigned)(2 * ((size_t)(n0 + wv * RPW + lrow) * Kb + lkc * 8));
   const unsigned bstep_b = (unsigned)(2 * bstep);
 
@@ -281,18 +231,18 @@ __global__ __launch_bounds__(TL::NT, TL::WPS * 256 / TL::NT) void gemm_kernel(Ge
       ALOAD;                                                                                  \
     } else {                                                                                  \
       dma16s(B + (DOWN_SPLIT && (K0) >= Kb ? (K0) - Kb : (K0)), boff + (q_ - QA) * bstep_b,   \
-             STAGE + A_CH + (wv + NW * (q_ - QA)) * 64);                                      \
+             STAGE + A_CH + (wv + LW * (q_ - QA)) * 64);                                      \
     }                                                                                         \
   }
 #define MXM_DMA_PART(STAGE, K0, Q0, Q1)                                                       \
   do {                                                                                        \
     if (A_OFF32 && a.a_off32) {                                                               \
       MXM_DMA_LOOP(STAGE, K0, Q0, Q1,                                                         \
-                   dma16s(A + (K0), (unsigned)aoff[q_], STAGE + (wv + NW * q_) * 64))         \
+                   dma16s(A + (K0), (unsigned)aoff[q_], STAGE + (wv + LW * q_) * 64))         \
     } else {                                                                                  \
       MXM_DMA_LOOP(STAGE, K0, Q0, Q1,                                                         \
                    dma16(reinterpret_cast<const char*>(A + (K0)) + aoff[q_],                  \
-                         STAGE + (wv + NW * q_) * 64))                                        \
+                         STAGE + (wv + LW * q_) * 64))                                        \
     }                                                                                         \
   } while (0)
 #define MXM_DMA(STAGE, K0) MXM_DMA_PART(STAGE, K0, 0, LDPS)
@@ -388,6 +338,40 @@ __global__ __launch_bounds__(TL::NT, TL::WPS * 256 / TL::NT) void gemm_kernel(Ge
   constexpr int DSTEPS = (MXM_DMA_STEPS > 0 && MXM_DMA_STEPS < BK / 16) ? MXM_DMA_STEPS : BK / 16;
   constexpr int KS = BK / 16;
   const int nk = Kd / BK;
+  if constexpr (LOADERS) {
+    // Loading waves keep NS - 1 stages in flight; the computing waves only
+    // meet them at the stage barriers.  (With all waves loading, the loads of
+    // a stage queue up in every wave's way: a 128 x 128 x 64 stage takes the
+    // CU's load path about as long to accept as its MFMAs run.)  The barrier
+    // before a stage's last k step, as in the deep ring below.
+    static_assert(NS >= 3 && KS % 2 == 0, "a deep ring");
+    if (__builtin_amdgcn_readfirstlane(wave) >= TL::CW) {
+#pragma unroll
+      for (int st = 0; st < NS - 1; ++st)
+        if (st < nk) MXM_DMA(lds + st * BUF, st * BK);
+      MXM_STAGE_BARRIER(min(NS - 2, nk - 1));
+      for (int kt = 0; kt < nk - 1; ++kt) {
+        MXM_STAGE_BARRIER(min(NS - 3, nk - 2 - kt));
+        if (kt + NS - 1 < nk) MXM_DMA(lds + ((kt + NS - 1) % NS) * BUF, (kt + NS - 1) * BK);
+      }
+      MXM_STAGE_BARRIER(0);
+      return;
+    }
+    lds_barrier();
+    MXM_FRAGS(lds, 0, 0);
+    for (int kt = 0; kt < nk - 1; ++kt) {
+      const u32x4_t* cur = lds + (kt % NS) * BUF;
+#pragma unroll
+      for (int ks = 0; ks < KS - 1; ++ks) MXM_KSTEP(ks & 1, cur, ks + 1, true);
+      lds_barrier();
+      MXM_KSTEP((KS - 1) & 1, lds + ((kt + 1) % NS) * BUF, 0, true);
+    }
+    const u32x4_t* cur = lds + ((nk - 1) % NS) * BUF;
+#pragma unroll
+    for (int ks = 0; ks < KS - 1; ++ks) MXM_KSTEP(ks & 1, cur, ks + 1, true);
+    MXM_KSTEP((KS - 1) & 1, cur, 0, false);
+    lds_barrier();
+  } else {
   // first stage: the weight rows go out first, they do not wait for perm
   if (nk > 0) {
     MXM_DMA_PART(lds, 0, QA, LDPS);
@@ -432,6 +416,7 @@ __global__ __launch_bounds__(TL::NT, TL::WPS * 256 / TL::NT) void gemm_kernel(Ge
     }
   }
   MXM_STAGE_BARRIER(0);  // every wave is done reading before the staging reuse
+  }
 #undef MXM_DMA
 #undef MXM_DMA_PART
 #undef MXM_STAGE_BARRIER
@@ -465,7 +450,7 @@ __global__ __launch_bounds__(TL::NT, TL::WPS * 256 / TL::NT) void gemm_kernel(Ge
                                         yo + (size_t)(row0 + lr) * a.Ncols + ycol + j * 32);
         }
       }
-    continue;
+    return;
   }
   // ---- epilogue: activation, bf16, per-wave LDS staging, 16-byte stores ----
   // 32x32 accumulator layout: register r of lane l holds
@@ -543,9 +528,7 @@ __global__ __launch_bounds__(TL::NT, TL::WPS * 256 / TL::NT) void gemm_kernel(Ge
       if (grow + 1 < rows)
         *reinterpret_cast<u32x4_t*>(rout + (size_t)(row0 + grow + 1) * a.Ncols + c0r) = hi;
     }
-    // every wave's staging reads are done before the next tile's loads
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    continue;  // no hidden: the backward's activation pass derives it
+    return;  // no hidden: the backward's activation pass derives it
   }
   // kinds whose hidden is fp32 store it as two bf16 planes (hi, then lo =
   // bf16(h - hi)) through the same staging, one plane after the other
@@ -629,9 +612,13 @@ __global__ __launch_bounds__(TL::NT, TL::WPS * 256 / TL::NT) void gemm_kernel(Ge
   const int c0 = n0 / (MODE == MXM_GEMM_GLU ? 2 : 1) + wn * C + plane * hcols;
   uint16_t* __restrict__ out = static_cast<uint16_t*>(a.out);
   constexpr int SEGS = C / 8;  // 8-column segments per row pair
+  // (each plane computes its own addresses: kept from one to the next they
+  // would spill)
+  int ln = lane;
+  if constexpr (H_SPLIT) asm volatile("" : "+v"(ln));
 #pragma unroll
   for (int it = 0; it < (WROWS / 2) * SEGS / 64; ++it) {
-    const int q = lane + 64 * it;
+    const int q = ln + 64 * it;
     const int kp = q / SEGS, sg = q % SEGS;
     const u32x4_t w0 = *reinterpret_cast<const u32x4_t*>(stage + word_at(kp, sg * 8));
     const u32x4_t w1 = *reinterpret_cast<const u32x4_t*>(stage + word_at(kp, sg * 8 + 4));
@@ -657,7 +644,215 @@ __global__ __launch_bounds__(TL::NT, TL::WPS * 256 / TL::NT) void gemm_kernel(Ge
     }
   }
   }  // plane loop
-  }  // tile loop
+}
+
+// ---- the scheduled kernel: 256 x 256 tiles, what is left in 128 x 128 ------
+//
+// A CU holds one 256 x 256 tile at a time, so a launch of T such tiles takes
+// ceil(T / 256) rounds however few tiles the last one has, and an expert's
+// last row tile costs a whole tile however few rows it has.  This kernel
+// plans its own work from the experts' row counts: 256-row tiles where they
+// are full or more than half full, 128 x 128 tiles (8 waves, four LDS stages
+// of 64 k: the same 128 KB of LDS with three stages in flight instead of
+// one) for an expert's last 128 rows or fewer, for the columns past a
+// multiple of 256, and for the big tiles of a last round that would leave
+// most CUs idle.  Every output is one tile's sum over k in ascending order
+// whichever shape it falls in, so the plan changes no result.
+//
+// The plan is a function of the counts only, computed by every workgroup in
+// LDS (prefixes over the experts of the big and the small row tiles), so it
+// needs neither a launch before it nor a lookup in memory per tile.  Each XCD
+// (workgroup L runs on XCD L % 8) takes a contiguous eighth of the big tiles,
+// in groups of GM row tiles by all column tiles, then of the small ones; the
+// workgroups that have one big tile fewer start the small ones.
+//
+// Measured against one tile shape per launch (16384 tokens of D 512 / E 8 / K
+// 2 / ffn 2048): gate+up 163 -> 147 us, down (272 tiles of 256 x 256, or 1056
+// of 128 x 128) 89 -> 72 us, 0.95 PFLOP/s of the 1.2 that this card reaches
+// on a large dense product; 4096 tokens of D 2048 / E 64 / K 8 / ffn 1408
+// gate+up 502 -> 455 us.
+using BigTile = Tile<256, 256, 2, 4, 2, 2, 64>;
+using SmallTile = Tile<128, 128, 2, 2, 2, 4, 64, 4>;
+constexpr int SMALL_PER_BIG = 3;  // small tiles in the time of a big one
+
+struct SchedLds {
+  int big[MXM_MAX_EXPERTS + 1];    // first big row tile of expert e
+  int small[MXM_MAX_EXPERTS + 1];  // first small row tile (an expert has one or none)
+  int off[MXM_MAX_EXPERTS + 1];    // offsets
+  int wsum[2][MXM_MAX_EXPERTS / 64];
+};
+
+// Prefixes of the experts' row tiles of BM rows: (count + rnd) / BM big ones,
+// and a small one for rows left over (rnd = BM - 1 leaves none).
+template <int BM>
+__device__ __forceinline__ void sched_build(SchedLds& S, const int32_t* offsets, int E, int rnd) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  static_assert(MXM_MAX_EXPERTS % 64 == 0 && MXM_MAX_EXPERTS <= 256, "one expert per thread");
+  const int o0 = tid < E ? offsets[tid] : 0;
+  const int o1 = tid < E ? offsets[tid + 1] : 0;
+  const int nb = (o1 - o0 + rnd) / BM, ns = o1 - o0 > nb * BM ? 1 : 0;
+  int ib = nb, is = ns;
+#pragma unroll
+  for (int sh = 1; sh < 64; sh <<= 1) {
+    const int vb = __shfl_up(ib, sh, 64), vs = __shfl_up(is, sh, 64);
+    if (lane >= sh) {
+      ib += vb;
+      is += vs;
+    }
+  }
+  if (lane == 63 && wave < MXM_MAX_EXPERTS / 64) {
+    S.wsum[0][wave] = ib;
+    S.wsum[1][wave] = is;
+  }
+  __syncthreads();
+  if (tid < MXM_MAX_EXPERTS) {
+    for (int w = 0; w < wave; ++w) {
+      ib += S.wsum[0][w];
+      is += S.wsum[1][w];
+    }
+    if (tid < E) {
+      S.big[tid + 1] = ib;
+      S.small[tid + 1] = is;
+      S.off[tid + 1] = o1;
+      if (tid == 0) S.big[0] = S.small[0] = S.off[0] = 0;
+    }
+  }
+  __syncthreads();
+}
+
+// The expert of row tile t: the number of e in 1 .. E-1 with pre[e] <= t.
+__device__ __forceinline__ int sched_find(const int* pre, int E, int t) {
+  const int lane = threadIdx.x & 63;
+  int e = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int i = e0 + lane + 1;
+    e += __popcll(__ballot(i < E && pre[i] <= t));
+  }
+  return e;
+}
+
+// Row tile and column tile of place q in the list of a launch's tiles: groups
+// of GM row tiles (of `nrow`), a group's `ncol` column tiles one after the
+// other.
+__device__ __forceinline__ void sched_place(int q, int nrow, int ncol, int& mt, int& nt) {
+  const int g = q / (GM * ncol), rr = q - g * (GM * ncol);
+  const int rig = min(GM, nrow - g * GM);
+  mt = g * GM + rr % rig;
+  nt = rr / rig;
+}
+
+template <int EPI>
+__global__ __launch_bounds__(512, 1) void gemm_sched_kernel(GemmArgs a, int whole) {
+  static_assert(BigTile::NS * BigTile::BUF == SmallTile::NS * SmallTile::BUF &&
+                    BigTile::NT == 512 && SmallTile::NT == 512,
+                "both shapes share the ring and the workgroup");
+  __shared__ u32x4_t lds[BigTile::NS * BigTile::BUF];
+  __shared__ SchedLds S;
+  const int E = a.E;
+  // whole: 256 x 256 tiles only (Ncols a multiple of 256)
+  sched_build<256>(S, a.offsets, E, whole ? 255 : 127);
+  auto uni = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+  const int BR = uni(S.big[E]), SR = uni(S.small[E]);
+  const int ncb = a.Ncols / 256, ncs = a.Ncols / 128;  // column tiles
+  const int G = gridDim.x;
+  // big tiles B, small tiles S0 whatever becomes of the last round; that
+  // round's `rem` big tiles are cut in four each where all the small tiles
+  // then take fewer rounds of CUs than the two kinds apart
+  const int B = BR * ncb;
+  const int S0 = SR * ncs + (ncs & 1) * 2 * BR;
+  const int rem = B % G;
+  int Bm = B;
+  if (!whole && rem > 0) {
+    const int cut = (4 * rem + S0 + G - 1) / G;
+    const int left = max(0, S0 - (G - rem) * SMALL_PER_BIG);
+    const int keep = SMALL_PER_BIG + (left + G - 1) / G;
+    if (cut < keep) Bm = B - rem;
+  }
+  const int Ns = S0 + 4 * (B - Bm);
+  // this XCD's part of both lists, and this workgroup's place in it
+  const int xcd = blockIdx.x & 7, s = blockIdx.x >> 3, W = G >> 3;
+  const int lo = (int)((int64_t)Bm * xcd / 8), hi = (int)((int64_t)Bm * (xcd + 1) / 8);
+  const int slo = (int)((int64_t)Ns * xcd / 8), sn = (int)((int64_t)Ns * (xcd + 1) / 8) - slo;
+  bool first = true;
+  for (int p = lo + s; p < hi; p += W) {
+    // every wave has read the previous tile's epilogue staging out of LDS
+    // (plain s_barrier: no wait for that epilogue's stores)
+    if (!first) asm volatile("s_barrier" ::: "memory");
+    first = false;
+    int mt, nt;
+    sched_place(p, BR, ncb, mt, nt);
+    const int e = uni(sched_find(S.big, E, mt));
+    const int row0 = uni(S.off[e] + (mt - S.big[e]) * 256);
+    const int rows = min(256, uni(S.off[e + 1]) - row0);
+    gemm_tile<BigTile, 256, 256, 2, 4, EPI>(a, lds, e, row0, rows, nt * 256);
+  }
+  if (whole) return;
+  const int odd = (hi - lo) % W;              // workgroups with one big tile more
+  const int idle = odd > 0 ? W - odd : 0;     // ... and the rest, which start
+  const int ahead = SMALL_PER_BIG * idle;
+  for (int k = (idle > 0 && s >= odd) ? 0 : SMALL_PER_BIG;; ++k) {
+    const int i = k < SMALL_PER_BIG ? s - odd + k * idle : ahead + s + (k - SMALL_PER_BIG) * W;
+    if (i >= sn) {
+      if (k < SMALL_PER_BIG) continue;
+      break;
+    }
+    if (!first) asm volatile("s_barrier" ::: "memory");
+    first = false;
+    int t = slo + i, e, row0, rows, n0;
+    if (t < SR * ncs) {
+      // an expert's last rows
+      const int sr = t / ncs;
+      e = uni(sched_find(S.small, E, sr));
+      row0 = uni(S.off[e] + (S.big[e + 1] - S.big[e]) * 256);
+      rows = uni(S.off[e + 1]) - row0;
+      n0 = (t - sr * ncs) * 128;
+    } else {
+      int mt, half;
+      if (t < S0) {
+        // the last 128 columns of the big row tiles
+        t -= SR * ncs;
+        mt = t >> 1;
+        half = t & 1;
+        n0 = ncb * 256;
+      } else {
+        // a quarter of a big tile of the last round
+        t -= S0;
+        int nt;
+        sched_place(Bm + (t >> 2), BR, ncb, mt, nt);
+        half = (t >> 1) & 1;
+        n0 = nt * 256 + (t & 1) * 128;
+      }
+      e = uni(sched_find(S.big, E, mt));
+      row0 = uni(S.off[e] + (mt - S.big[e]) * 256) + half * 128;
+      rows = min(128, uni(S.off[e + 1]) - row0);
+    }
+    gemm_tile<SmallTile, 128, 128, 2, 2, EPI>(a, lds, e, row0, rows, n0);
+  }
+}
+
+// Tiles of one shape, two workgroups of 4 waves on a CU: the requested
+// families, and launches of up to two 128 x 128 tiles per CU, whose second
+// round of single tiles would leave most CUs idle on the kernel above.
+template <class TL, int BM, int BN, int WM, int WN, int EPI>
+__global__ __launch_bounds__(TL::NT, TL::WPS * 256 / TL::NT) void gemm_kernel(GemmArgs a) {
+  __shared__ u32x4_t lds[TL::NS * TL::BUF];
+  __shared__ SchedLds S;
+  const int E = a.E;
+  sched_build<BM>(S, a.offsets, E, BM - 1);
+  auto uni = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+  const int BR = uni(S.big[E]), ncol = a.Ncols / BN;
+  const int64_t T = (int64_t)BR * ncol;
+  const int xcd = blockIdx.x & 7, s = blockIdx.x >> 3, W = gridDim.x >> 3;
+  const int lo = (int)(T * xcd / 8), hi = (int)(T * (xcd + 1) / 8);
+  for (int p = lo + s; p < hi; p += W) {
+    if (p != lo + s) asm volatile("s_barrier" ::: "memory");  // as above
+    int mt, nt;
+    sched_place(p, BR, ncol, mt, nt);
+    const int e = uni(sched_find(S.big, E, mt));
+    const int row0 = uni(S.off[e] + (mt - S.big[e]) * BM);
+    gemm_tile<TL, BM, BN, WM, WN, EPI>(a, lds, e, row0, min(BM, uni(S.off[e + 1]) - row0),
+                                       nt * BN);
+  }
 }
 
 // Workgroups resident at once on the current device: CUs x workgroups per
@@ -677,70 +872,68 @@ static int persistent_grid(int per_cu) {
   return std::max(8, ncu[dev] * per_cu / 8 * 8);
 }
 
-template <int BM, int BN, int WM, int WN, int WPS, int NSTG, int BKK, int EPI>
-void launch_epi(const GemmArgs& a, hipStream_t s, int blocks, int ngroups) {
-  using TL = Tile<BM, BN, WM, WN, WPS, NSTG, BKK>;
-  // workgroups per CU: what the launch bounds allow, capped by LDS
-  constexpr int lds_bytes = NSTG * TL::BUF * 16;
-  constexpr int per_cu = std::min(TL::WPS * 256 / TL::NT, 160 * 1024 / lds_bytes);
-  const int grid = std::min(blocks, persistent_grid(std::max(1, per_cu)));
-  hipLaunchKernelGGL((gemm_kernel<TL, BM, BN, WM, WN, EPI>), dim3(grid), dim3(TL::NT), 0, s, a,
-                     ngroups, blocks);
-}
-
-template <int BM, int BN, int WM, int WN, int WPS, int NSTG, int BKK>
-void launch_family(const GemmArgs& a, hipStream_t s);
-
-// An up projection that also keeps its raw projections (GemmArgs::out2),
-// or whose weights are int8 integers with per-column scales (scale0).
-template <int BM, int BN, int WM, int WN, int WPS, int NSTG, int BKK, int EPI>
-void launch_up(const GemmArgs& a, hipStream_t s, int blocks, int ngroups) {
-  if (a.out2)
-    launch_epi<BM, BN, WM, WN, WPS, NSTG, BKK, EPI_KEEP + EPI>(a, s, blocks, ngroups);
-  else if (a.scale0)
-    launch_epi<BM, BN, WM, WN, WPS, NSTG, BKK, EPI_SCALE + EPI>(a, s, blocks, ngroups);
-  else
-    launch_epi<BM, BN, WM, WN, WPS, NSTG, BKK, EPI>(a, s, blocks, ngroups);
-}
-
-template <int BM, int BN, int WM, int WN, int WPS, int NSTG, int BKK>
-void launch_family(const GemmArgs& a, hipStream_t s) {
-  const int ngroups = (a.max_mtiles + GM - 1) / GM;
-  const int per_group = GM * (a.Ncols / BN);
-  const int blocks = ((ngroups + 7) / 8) * 8 * per_group;
+// Calls f with the epilogue kind of these arguments as a constant: an up
+// projection may keep its raw projections (GemmArgs::out2), and weights may
+// be int8 integers with per-column scales (scale0).
+template <class F>
+void with_epi(const GemmArgs& a, F&& f) {
+  auto up = [&](auto kind) {
+    constexpr int K = decltype(kind)::value;
+    if (a.out2)
+      f(std::integral_constant<int, EPI_KEEP + K>{});
+    else if (a.scale0)
+      f(std::integral_constant<int, EPI_SCALE + K>{});
+    else
+      f(kind);
+  };
   if (a.mode == MXM_GEMM_DOWN) {
     if (a.scale0 && a.h_split)
-      launch_epi<BM, BN, WM, WN, WPS, NSTG, BKK, EPI_SCALE + EPI_DOWN_F32>(a, s, blocks, ngroups);
+      f(std::integral_constant<int, EPI_SCALE + EPI_DOWN_F32>{});
     else if (a.scale0)
-      launch_epi<BM, BN, WM, WN, WPS, NSTG, BKK, EPI_SCALE + EPI_DOWN>(a, s, blocks, ngroups);
+      f(std::integral_constant<int, EPI_SCALE + EPI_DOWN>{});
     else if (a.h_split)
-      launch_epi<BM, BN, WM, WN, WPS, NSTG, BKK, EPI_DOWN_F32>(a, s, blocks, ngroups);
+      f(std::integral_constant<int, EPI_DOWN_F32>{});
     else if (a.f32_out)
-      launch_epi<BM, BN, WM, WN, WPS, NSTG, BKK, EPI_F32>(a, s, blocks, ngroups);
+      f(std::integral_constant<int, EPI_F32>{});
     else
-      launch_epi<BM, BN, WM, WN, WPS, NSTG, BKK, EPI_DOWN>(a, s, blocks, ngroups);
+      f(std::integral_constant<int, EPI_DOWN>{});
     return;
   }
   switch (mxm_epi_kind(a.expert_type, a.activation)) {
     case EPI_GEGLU:
-      launch_up<BM, BN, WM, WN, WPS, NSTG, BKK, EPI_GEGLU>(a, s, blocks, ngroups);
-      break;
+      return up(std::integral_constant<int, EPI_GEGLU>{});
     case EPI_MLP_SILU:
-      launch_up<BM, BN, WM, WN, WPS, NSTG, BKK, EPI_MLP_SILU>(a, s, blocks, ngroups);
-      break;
+      return up(std::integral_constant<int, EPI_MLP_SILU>{});
     case EPI_MLP_GELU:
-      launch_up<BM, BN, WM, WN, WPS, NSTG, BKK, EPI_MLP_GELU>(a, s, blocks, ngroups);
-      break;
+      return up(std::integral_constant<int, EPI_MLP_GELU>{});
     case EPI_MLP_RELU:
-      launch_up<BM, BN, WM, WN, WPS, NSTG, BKK, EPI_MLP_RELU>(a, s, blocks, ngroups);
-      break;
+      return up(std::integral_constant<int, EPI_MLP_RELU>{});
     case EPI_MLP_LEAKY:
-      launch_up<BM, BN, WM, WN, WPS, NSTG, BKK, EPI_MLP_LEAKY>(a, s, blocks, ngroups);
-      break;
+      return up(std::integral_constant<int, EPI_MLP_LEAKY>{});
     default:
-      launch_up<BM, BN, WM, WN, WPS, NSTG, BKK, EPI_SWIGLU>(a, s, blocks, ngroups);
-      break;
+      return up(std::integral_constant<int, EPI_SWIGLU>{});
   }
+}
+
+template <int BM, int BN, int WM, int WN, int WPS, int NSTG, int BKK>
+void launch_family(const GemmArgs& a, hipStream_t s) {
+  using TL = Tile<BM, BN, WM, WN, WPS, NSTG, BKK>;
+  // workgroups per CU: what the launch bounds allow, capped by LDS
+  constexpr int lds_bytes = NSTG * TL::BUF * 16 + (int)sizeof(SchedLds);
+  constexpr int per_cu = std::min(TL::WPS * 256 / TL::NT, 160 * 1024 / lds_bytes);
+  static_assert(per_cu == 2, "two workgroups per CU");
+  with_epi(a, [&](auto epi) {
+    hipLaunchKernelGGL((gemm_kernel<TL, BM, BN, WM, WN, decltype(epi)::value>),
+                       dim3(persistent_grid(per_cu)), dim3(TL::NT), 0, s, a);
+  });
+}
+
+// The scheduled kernel: one workgroup per CU.  whole: 256 x 256 tiles only.
+void launch_sched(const GemmArgs& a, hipStream_t s, int whole) {
+  with_epi(a, [&](auto epi) {
+    hipLaunchKernelGGL((gemm_sched_kernel<decltype(epi)::value>), dim3(persistent_grid(1)),
+                       dim3(512), 0, s, a, whole);
+  });
 }
 
 }  // namespace
@@ -757,30 +950,46 @@ int mxm_mfma_tile_rows(int Ncols, int Kd, int family) {
       return f128 ? 128 : 0;
     case MXM_TILE_256x256:
       return f256 ? 256 : 0;
-    default:  // auto: 256 x 256 where it tiles, else 128 x 128
+    default:  // auto and the scheduled kernel
       return f256 ? 256 : f128 ? 128 : 0;
   }
 }
 
-// Family chosen for these dimensions (auto resolved).
-static int resolve_family(const GemmArgs& a) {
-  if (a.family != MXM_TILE_AUTO) return a.family;
-  return a.Ncols % 256 == 0 ? MXM_TILE_256x256 : MXM_TILE_128x128;
-}
-
 void mxm_launch_gemm_mfma(const GemmArgs& args, hipStream_t s) {
-  if (args.max_mtiles <= 0) return;
+  if (args.rows_total <= 0) return;
   GemmArgs a = args;
   a.a_off32 = !a.no_off32 && (size_t)a.rows_total * a.Kd * 2 < ((size_t)1 << 32);
-  switch (resolve_family(a)) {
+  int family = a.family;
+  if (family == MXM_TILE_AUTO) {
+    // 128 x 128 tiles of a launch with evenly loaded experts, the last tile
+    // of each half full.  Between one and two of them per CU the pairs run
+    // them in one round (2000 tokens of D 1024 / E 16 / K 2 / ffn 2734, down:
+    // 312 tiles 43 us, 48 on the scheduled kernel; 6000 of D 512 / E 16 / ffn
+    // 1024: 407 tiles 17.2 / 20.2 us); below, the scheduled kernel's deeper
+    // ring is faster (219 tiles of 64 stages: 48 / 34 us), above, its big
+    // tiles (527: 29.7 / 26.8, 1040: 85 / 71).  A pair also overlaps one
+    // tile's epilogue with the other's products, which counts where tiles
+    // have few stages (6 and fewer: 20000 tokens of D 256, up 36.0 / 38.3 us,
+    // 12000 of D 384 52.4 / 54.9; at 8 stages 161 / 147), and 128 columns
+    // hold no big tile (23433 tokens, D 128: 15.7 / 18.5 us).
+    const int64_t tiles =
+        ((int64_t)a.rows_total + 64 * (int64_t)a.E) / 128 * (a.Ncols / 128);
+    const int n_cu = persistent_grid(1);
+    if (a.Ncols < 256 || a.Kd <= 384 || (tiles > n_cu && tiles <= 2 * n_cu))
+      family = MXM_TILE_128x128;
+  }
+  switch (family) {
     case MXM_TILE_256x128:
       launch_family<256, 128, 2, 2, 2, 3, 32>(a, s);
       break;
     case MXM_TILE_128x128:
       launch_family<128, 128, 2, 2, 2, 2, 64>(a, s);
       break;
+    case MXM_TILE_256x256:
+      launch_sched(a, s, 1);
+      break;
     default:
-      launch_family<256, 256, 2, 4, 2, 2, 64>(a, s);
+      launch_sched(a, s, 0);
       break;
   }
 }

@@ -175,9 +175,9 @@ struct GemmArgs {
                           // ld2 apart (out may then be null: no hidden stored)
   int ld2;
   const int32_t* offsets; // [E + 1]
-  const int32_t* mstart;  // [E + 1]
+  const int32_t* mstart;  // [E + 1] (SIMT and int8 families; the MFMA kernels plan their own)
   int E, Kd, Ncols;       // reduction length, output columns (per matrix)
-  int max_mtiles;         // grid bound on row tiles
+  int max_mtiles;         // grid bound on row tiles (SIMT family)
   int expert_type, activation;
   float slope;
   bool y_bf16;            // SIMT down: round y to bf16
@@ -509,8 +509,6 @@ void mxm_launch_hidden_from_raw_bf16(const uint16_t* gu, int rows, int F, int et
 void mxm_launch_act_bw_gated_bf16(const uint16_t* gu, const uint16_t* dhr, uint16_t* Hg,
                                   bool hsplit, const float* gp, int rows, int F, int etype, int act,
                                   float slope, uint16_t* dgu, float* dgp, hipStream_t s);
-// Row-tile prefix of counts for tile height bm (mstart[0..E]).
-void mxm_launch_tile_prefix(const int32_t* counts, int E, int bm, int32_t* mstart, hipStream_t s);
 
 // fp32 products on the bf16 MFMA kernels (the fp32 backward): fp32 values
 // as bf16 planes hi = bf16(v), lo = bf16(v - hi), concatenated along k as
