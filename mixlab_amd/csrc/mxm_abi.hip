@@ -99,11 +99,10 @@ struct DevBuf {
 };
 
 // Every device buffer a forward writes besides its outputs.  layout_workspace
-// places the pieces at 256-byte aligned offsets from one base; the two
-// tickets share the first piece and must be zero between calls (the kernels
-// that take them leave them zero).
+// places the pieces at 256-byte aligned offsets from one base; the ticket is
+// the first and must be zero between calls (the kernel that takes it leaves
+// it zero).
 struct Workspace {
-  int32_t* scan_ticket = nullptr;  // [1] scan kernel (N > 1024)
   int32_t* ticket = nullptr;       // [1] one-launch router (decode sizes)
   void* xcast = nullptr;           // [N, D] bf16 copy of fp32 x (bf16 compute)
   int32_t* top_idx = nullptr;      // [N*K]
@@ -111,18 +110,18 @@ struct Workspace {
   int32_t* slot_rank = nullptr;    // [N*K]
   int32_t* slot_pos = nullptr;     // [N*K]
   int32_t* perm = nullptr;         // [N*K]
-  int32_t* tile_counts = nullptr;  // [E, ntiles]
-  float* tile_psum = nullptr;      // [E, ntiles]
+  int32_t* tile_counts = nullptr;  // [ntiles, E]
+  float* tile_psum = nullptr;      // [ntiles, E]
   float* tile_ent = nullptr;       // [ntiles]
-  int32_t* tile_base = nullptr;    // [E, ntiles]
+  int32_t* group_counts = nullptr; // [groups, E] (batches with many tiles)
+  float* group_psum = nullptr;     // [groups, E]
+  float* group_ent = nullptr;      // [groups]
   int32_t* counts = nullptr;       // [E]
   int32_t* offsets = nullptr;      // [E + 1]
   int32_t* mstart1 = nullptr;      // [E + 1]
   int32_t* mstart2 = nullptr;      // [E + 1]
   float* aux = nullptr;            // [1] when the caller passes none
   float* ent = nullptr;            // [1]
-  int32_t* expert_count = nullptr; // [E]
-  float* expert_pmean = nullptr;   // [E]
   void* xpad = nullptr;            // [N, Kx] bf16 x padded to the up projection's reduction
   void* H = nullptr;               // [N*K, Fk] (split hidden: [N*K, 2Fk])
   void* Y = nullptr;               // [N*K, Dk]
@@ -160,9 +159,9 @@ struct MoeOp {
   // up (GLU) fp32 [E][D][F], w2 = down fp32 [E][F][D].  MFMA family: w1 =
   // bf16 [E][2F or F][D] (GLU interleaved), w2 = bf16 [E][D][F].
   DevBuf router, w1, w1b, w2;
-  // decode-sized batches, and the tiled router's matrix-core logits (E >
-  // 32): router_w lane-interleaved (RouteSmallArgs::wr_t)
-  bool small_route = false, mf_router = false;
+  // decode-sized batches, and the tiled router's matrix-core logits:
+  // router_w lane-interleaved (RouteSmallArgs::wr_t)
+  bool small_route = false, mf_router = true;
   int ldw = 0;
   DevBuf router_t;
   // int8 family: q1 = gate (GLU) or up (MLP), q1b = up (GLU), q2 = down, in
@@ -186,6 +185,7 @@ struct MoeOp {
   std::vector<char> have;
 
   // tile schedule of the forward (set at create from the op's parameters)
+  int tile_tokens = MXM_ROUTER_TM;  // of the tiled router
   int ntiles = 0, bm1 = 0, bm2 = 0, max_mtiles1 = 0, max_mtiles2 = 0;
   int simt_tile = 0;  // MXM_SIMT_TILE at creation: the SIMT family's tile (0 picks)
   int simt_vec = 0;   // MXM_SIMT_MFMA=0 at creation: 64 x 64 SIMT tiles on the vector unit
@@ -352,7 +352,7 @@ bool dec16_pays(int N, int E, int K) { return (int64_t)N * K < DEC16_MAX_RPE * (
 // the op's parameters only.
 void set_schedule(MoeOp& o) {
   const size_t NK = (size_t)o.N * o.K;
-  o.ntiles = (int)(((size_t)o.N + MXM_ROUTER_TM - 1) / MXM_ROUTER_TM);
+  o.ntiles = (o.N + o.tile_tokens - 1) / o.tile_tokens;
   const bool glu = o.etype != MXM_EXPERT_MLP;
   if (o.int8_kernels()) {
     o.bm1 = o.bm2 = 256;  // tile schedules are not used by the int8 kernels
@@ -391,9 +391,7 @@ Workspace layout_workspace(const MoeOp& o, char* base) {
     off += (bytes + 255) / 256 * 256;
     return p;
   };
-  char* tickets = take(8);
-  w.scan_ticket = reinterpret_cast<int32_t*>(tickets);
-  w.ticket = base ? reinterpret_cast<int32_t*>(tickets + 4) : nullptr;
+  w.ticket = reinterpret_cast<int32_t*>(take(4));
   if (o.bf16) w.xcast = take(N * o.D * 2);
   w.top_idx = reinterpret_cast<int32_t*>(take(NK * 4));
   w.gates = reinterpret_cast<float*>(take(NK * 4));
@@ -403,15 +401,17 @@ Workspace layout_workspace(const MoeOp& o, char* base) {
   w.tile_counts = reinterpret_cast<int32_t*>(take(E * T * 4));
   w.tile_psum = reinterpret_cast<float*>(take(E * T * 4));
   w.tile_ent = reinterpret_cast<float*>(take(T * 4));
-  w.tile_base = reinterpret_cast<int32_t*>(take(E * T * 4));
+  if (const size_t G = (size_t)mxm_dispatch_groups(o.ntiles, o.E)) {
+    w.group_counts = reinterpret_cast<int32_t*>(take(E * G * 4));
+    w.group_psum = reinterpret_cast<float*>(take(E * G * 4));
+    w.group_ent = reinterpret_cast<float*>(take(G * 4));
+  }
   w.counts = reinterpret_cast<int32_t*>(take(E * 4));
   w.offsets = reinterpret_cast<int32_t*>(take((E + 1) * 4));
   w.mstart1 = reinterpret_cast<int32_t*>(take((E + 1) * 4));
   w.mstart2 = reinterpret_cast<int32_t*>(take((E + 1) * 4));
   w.aux = reinterpret_cast<float*>(take(4));
   w.ent = reinterpret_cast<float*>(take(4));
-  w.expert_count = reinterpret_cast<int32_t*>(take(E * 4));
-  w.expert_pmean = reinterpret_cast<float*>(take(E * 4));
   const size_t esz = (o.mfma || o.q8) ? 2 : 4;
   if ((o.mfma || o.q8) && o.Kx != o.D) w.xpad = take(N * (size_t)o.Kx * 2);
   w.H = take(NK * (size_t)o.Fk * esz * (o.hsplit ? 2 : 1));
@@ -429,7 +429,7 @@ void alloc_workspace(MoeOp& o) {
   const size_t bytes = layout_workspace(o, nullptr).bytes;
   o.wsbuf.alloc(bytes);
   o.ws = layout_workspace(o, o.wsbuf.as<char>());
-  HIPCK(hipMemsetAsync(o.ws.scan_ticket, 0, 8, o.stream));  // both tickets
+  HIPCK(hipMemsetAsync(o.ws.ticket, 0, 4, o.stream));
   o.ws_ready = true;
 }
 
@@ -507,16 +507,17 @@ void run_forward(MoeOp& o, const Workspace& w, const void* x, int x_dtype, float
 
   mark(0);
   float* probs_keep = o.keep_probs ? o.bw_probs.as<float>() : w.probs;
-  ScanArgs sa{};
-  sa.counts = w.counts;
-  sa.offsets = w.offsets;
-  sa.mstart1 = w.mstart1;
-  sa.mstart2 = w.mstart2;
-  ScatterArgs sc{};
-  sc.perm = w.perm;
-  sc.slot_pos = w.slot_pos;
+  // the up projection reads x's rows Kx long: a zero-padded copy when D is
+  // not a multiple of 64 (the tiled router reads it too: whole 16-byte pieces)
+  const void* xg = xin;
+  if (w.xpad) {
+    for (int rep = 0; rep < reps; ++rep)
+      mxm_launch_pad_rows_bf16(static_cast<const uint16_t*>(xin), o.N, o.D, o.Kx,
+                               static_cast<uint16_t*>(w.xpad), st);
+    xg = w.xpad;
+  }
   if (o.small_route) {
-    // one launch: router, scan and scatter (stages 1 and 2 are empty)
+    // one launch: router and dispatch (stages 1 and 2 are empty)
     RouteSmallArgs rs{};
     rs.x = xin;
     rs.wr_t = o.router_t.p;
@@ -531,12 +532,12 @@ void run_forward(MoeOp& o, const Workspace& w, const void* x, int x_dtype, float
     rs.gates = w.gates;
     rs.probs = probs_keep ? probs_keep : w.small_probs;
     rs.tok_ent = w.tok_ent;
-    rs.counts = sa.counts;
-    rs.offsets = sa.offsets;
-    rs.mstart1 = sa.mstart1;
-    rs.mstart2 = sa.mstart2;
-    rs.perm = sc.perm;
-    rs.slot_pos = sc.slot_pos;
+    rs.counts = w.counts;
+    rs.offsets = w.offsets;
+    rs.mstart1 = w.mstart1;
+    rs.mstart2 = w.mstart2;
+    rs.perm = w.perm;
+    rs.slot_pos = w.slot_pos;
     rs.aux = aux_p;
     rs.entropy = ent_p;
     rs.aux_weight = blk ? blk->aux_weight : 1.0f;
@@ -549,13 +550,16 @@ void run_forward(MoeOp& o, const Workspace& w, const void* x, int x_dtype, float
     mark(1);
     mark(2);
   } else {
+    const bool padded = w.xpad && o.mf_router;
     RouterArgs ra{};
-    ra.x = xin;
+    ra.x = padded ? w.xpad : xin;
+    ra.ldx = ra.Dx = padded ? o.Kx : o.D;
     ra.wr = o.router.p;
     ra.N = o.N;
     ra.D = o.D;
     ra.E = o.E;
     ra.K = o.K;
+    ra.tile_tokens = o.tile_tokens;
     ra.top_idx = w.top_idx;
     ra.gates = w.gates;
     ra.slot_rank = w.slot_rank;
@@ -569,60 +573,50 @@ void run_forward(MoeOp& o, const Workspace& w, const void* x, int x_dtype, float
     HIPCK(hipGetLastError());
 
     mark(1);
-    sa.tile_counts = ra.tile_counts;
-    sa.tile_psum = ra.tile_psum;
-    sa.tile_ent = ra.tile_ent;
-    sa.N = o.N;
-    sa.E = o.E;
-    sa.K = o.K;
-    sa.ntiles = o.ntiles;
-    sa.bm1 = o.bm1;
-    sa.bm2 = o.bm2;
-    sa.tile_base = w.tile_base;
-    sa.aux = aux_p;
-    sa.entropy = ent_p;
-    sa.aux_weight = blk ? blk->aux_weight : 1.0f;
-    sa.aux_scaled = blk ? blk->aux_scaled : nullptr;
-    sa.expert_count = w.expert_count;
-    sa.expert_pmean = w.expert_pmean;
-    sa.ticket = w.scan_ticket;
-    for (int rep = 0; rep < reps; ++rep) mxm_launch_scan(sa, o.bf16, st);
+    DispatchArgs da{};
+    da.tile_counts = w.tile_counts;
+    da.tile_psum = w.tile_psum;
+    da.tile_ent = w.tile_ent;
+    da.top_idx = w.top_idx;
+    da.slot_rank = w.slot_rank;
+    da.N = o.N;
+    da.E = o.E;
+    da.K = o.K;
+    da.ntiles = o.ntiles;
+    da.tile_tokens = o.tile_tokens;
+    da.bm1 = o.bm1;
+    da.bm2 = o.bm2;
+    da.group_counts = w.group_counts;
+    da.group_psum = w.group_psum;
+    da.group_ent = w.group_ent;
+    da.counts = w.counts;
+    da.offsets = w.offsets;
+    da.mstart1 = w.mstart1;
+    da.mstart2 = w.mstart2;
+    da.perm = w.perm;
+    da.slot_pos = w.slot_pos;
+    da.aux = aux_p;
+    da.entropy = ent_p;
+    da.aux_weight = blk ? blk->aux_weight : 1.0f;
+    da.aux_scaled = blk ? blk->aux_scaled : nullptr;
+    for (int rep = 0; rep < reps; ++rep) mxm_launch_dispatch(da, o.bf16, st);
     HIPCK(hipGetLastError());
-
-    mark(2);
-    sc.top_idx = ra.top_idx;
-    sc.slot_rank = ra.slot_rank;
-    sc.tile_base = sa.tile_base;
-    sc.offsets = sa.offsets;
-    sc.N = o.N;
-    sc.K = o.K;
-    sc.ntiles = o.ntiles;
-    for (int rep = 0; rep < reps; ++rep) mxm_launch_scatter(sc, st);
-    HIPCK(hipGetLastError());
+    mark(2);  // (the scatter stage is part of the dispatch launch)
   }
 
   mark(3);
   if (o.route_only) return;
   const bool glu = o.etype != MXM_EXPERT_MLP;
-  // the up projection reads x's rows Kx long: a zero-padded copy when D is
-  // not a multiple of 64
-  const void* xg = xin;
-  if (w.xpad) {
-    for (int rep = 0; rep < reps; ++rep)
-      mxm_launch_pad_rows_bf16(static_cast<const uint16_t*>(xin), o.N, o.D, o.Kx,
-                               static_cast<uint16_t*>(w.xpad), st);
-    xg = w.xpad;
-  }
   GemmArgs g1{};
   g1.no_off32 = o.force64;
   g1.mode = glu ? MXM_GEMM_GLU : MXM_GEMM_MLP;
   g1.a = xg;
-  g1.perm = sc.perm;
+  g1.perm = w.perm;
   g1.b0 = o.w1.p;
   g1.b1 = o.w1b.p;
   g1.out = w.H;
-  g1.offsets = sa.offsets;
-  g1.mstart = sa.mstart1;
+  g1.offsets = w.offsets;
+  g1.mstart = w.mstart1;
   g1.E = o.E;
   g1.Kd = o.Kx;
   g1.Ncols = (o.mfma && glu && !stream) ? 2 * o.Fk : o.Fk;
@@ -691,8 +685,8 @@ void run_forward(MoeOp& o, const Workspace& w, const void* x, int x_dtype, float
   g2.a = w.H;
   g2.b0 = o.w2.p;
   g2.out = w.Y;
-  g2.offsets = sa.offsets;
-  g2.mstart = sa.mstart2;
+  g2.offsets = w.offsets;
+  g2.mstart = w.mstart2;
   g2.E = o.E;
   // the split MFMA down projection reduces over both planes of H
   g2.Kd = (o.hsplit && o.mfma && !stream) ? 2 * o.Fk : o.Fk;
@@ -739,7 +733,7 @@ void run_forward(MoeOp& o, const Workspace& w, const void* x, int x_dtype, float
   ca.y = w.Y;
   ca.top_idx = w.top_idx;
   ca.gates = w.gates;
-  ca.slot_pos = sc.slot_pos;
+  ca.slot_pos = w.slot_pos;
   ca.N = o.N;
   ca.D = o.D;
   ca.ldy = o.Dk;
@@ -924,7 +918,7 @@ std::mutex g_scratch_mu;
 char* g_scratch[kMaxDevices] = {};
 
 // This device's scratch address.  The first call on a device looks it up and
-// clears the tickets (the first 256 bytes of every workspace layout; the
+// clears the ticket (the first 256 bytes of every workspace layout; the
 // kernels leave them zero after each call) with a fill kernel, then waits for
 // the device, so it must not run under stream capture: mxm_init does it
 // before any capture.
@@ -1135,15 +1129,28 @@ int64_t mxm_moe_create(const float* float_params, int n_float_params, const int3
     const size_t DE = (size_t)o->D * o->E, DF = (size_t)o->D * o->F, EE = (size_t)o->E;
     const size_t F1 = (size_t)o->Kx * o->Fk, F2 = (size_t)o->Fk * o->Dk;  // padded matrices
     o->router.alloc(DE * (o->bf16 ? 2 : 4));
-    o->mf_router = o->E > 32;
-    if (const char* v = std::getenv("MXM_ROUTER_MFMA")) o->mf_router = o->mf_router && std::atoi(v) != 0;
+    if (const char* v = std::getenv("MXM_ROUTER_MFMA")) o->mf_router = std::atoi(v) != 0;
     // (the launcher also wants x 16-byte aligned; D decides it for the choice)
-    const bool mf_logits = o->mf_router && o->D % (o->bf16 ? 8 : 4) == 0 && o->D <= (1 << 24);
+    const bool mf_logits =
+        o->mf_router && o->E > 32 && o->D % (o->bf16 ? 8 : 4) == 0 && o->D <= (1 << 24);
     o->small_route = mxm_route_small_fits(o->N, o->D, o->E, o->K) &&
                      (o->int8_kernels() || o->dec16 ||
                       small_route_pays(o->N, o->D, o->E, mf_logits));
     if (const char* v = std::getenv("MXM_SMALL_ROUTE"))
       o->small_route = std::atoi(v) != 0 && mxm_route_small_fits(o->N, o->D, o->E, o->K);
+    // Tiles of 16 tokens, their reduction split over the workgroup's waves,
+    // up to MXM_ROUTER_SPLIT_N tokens (mxm_router.hip).  Their four times as
+    // many histograms must not take an op past the scratch of the
+    // no-allocation forward that fits it with tiles of 64.
+    if (o->N <= MXM_ROUTER_SPLIT_N) {
+      o->tile_tokens = 16;
+      set_schedule(*o);
+      if (layout_workspace(*o, nullptr).bytes > (size_t)MXM_NOALLOC_MAX_BYTES)
+        o->tile_tokens = MXM_ROUTER_TM;
+      set_schedule(*o);
+      if (layout_workspace(*o, nullptr).bytes > (size_t)MXM_NOALLOC_MAX_BYTES)
+        o->tile_tokens = 16;  // past it either way
+    }
     set_schedule(*o);
     if (o->small_route || o->mf_router) {
       o->ldw = (o->D + MXM_LOGIT_CHUNK - 1) / MXM_LOGIT_CHUNK * MXM_LOGIT_CHUNK;
@@ -2137,7 +2144,7 @@ int mxm_moe_info(int64_t h, int64_t* info, int n) {
   const int64_t flow = !op->have_last ? -1 : op->last_decode ? 2 : op->small_route ? 1 : 0;
   const int64_t vals[8] = {op->q8_mfma ? 3 : op->q8 ? 2 : op->dec16 ? 4 : op->mfma ? 1 : 0,
                            (int64_t)layout_workspace(*op, nullptr).bytes, (int64_t)op->bm1,
-                           (int64_t)((op->N + MXM_ROUTER_TM - 1) / MXM_ROUTER_TM),
+                           (int64_t)op->ntiles,
                            (int64_t)op->Fk, (int64_t)op->Dk, (int64_t)op->Kx, flow};
   int w = 0;
   for (; w < n && w < 8; ++w) info[w] = vals[w];

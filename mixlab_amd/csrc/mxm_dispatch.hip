@@ -8,10 +8,9 @@
 //   counts[e]      = #{n : e in top_idx[n, :]}
 //   offsets        = exclusive scan of counts (offsets[E] = N*K)
 //   perm[offsets[e] + r] = the r-th such token
-// The router leaves per-tile counts and per-slot in-tile ranks; the scan
-// kernel below turns the counts into offsets and per-(expert, tile) bases
-// (one workgroup per expert), and the scatter kernel places every slot.  Nothing here uses atomics, so
-// the result does not depend on scheduling.
+// The router leaves per-tile counts and per-slot in-tile ranks; the dispatch
+// kernel below turns the counts into offsets and per-(tile, expert) bases and
+// places every slot.  The result does not depend on scheduling.
 //
 // The combine sums, per token, gate * y over its K slots in ascending expert
 // id, multiply then add in fp32, starting from 0 -- the accumulation order of
@@ -35,135 +34,209 @@ __device__ __forceinline__ float wave_sum_fixed(float v) {
   return v;
 }
 
-constexpr int SCAN_NT = 256;
+// Sums of the tiles' histograms and partial sums over groups of
+// MXM_DISPATCH_GROUP tiles, one workgroup per group (large batches: every
+// workgroup of the dispatch reads this table, so it is kept short).
+__global__ __launch_bounds__(256) void dispatch_group_kernel(DispatchArgs a) {
+  const int g = blockIdx.x, t0 = g * MXM_DISPATCH_GROUP;
+  const int t1 = min(a.ntiles, t0 + MXM_DISPATCH_GROUP);
+  const int e = threadIdx.x;
+  if (e < a.E) {
+    int c = 0;
+    float p = 0.0f;
+    for (int t = t0; t < t1; ++t) {
+      c += a.tile_counts[(size_t)t * a.E + e];
+      p = p + a.tile_psum[(size_t)t * a.E + e];
+    }
+    a.group_counts[(size_t)g * a.E + e] = c;
+    a.group_psum[(size_t)g * a.E + e] = p;
+  }
+  if (e < 64) {
+    float s = t0 + e < t1 && e < MXM_DISPATCH_GROUP ? a.tile_ent[t0 + e] : 0.0f;
+    s = wave_sum_fixed(s);
+    if (e == 0) a.group_ent[g] = s;
+  }
+}
 
-// Workgroup e < E: expert e's total, its mean probability and the exclusive
-// prefix of its per-tile counts (relative to the expert's first row);
-// workgroup E: the entropy.  The last expert workgroup to finish (agent-scope
-// release fence, atomic ticket; agent-scope acquire) computes counts,
-// offsets, both row-tile prefixes and aux from the per-expert totals and
-// resets the ticket.  No workgroup waits for another, so the grid always
-// drains.  The floating-point sums keep one fixed order: per expert (and for
-// the entropy) lane-strided sequential partial sums over the tiles, then an
-// xor butterfly over the wave; aux over experts in ascending order.
+// Dispatch in one launch: every workgroup adds up the table of histograms
+// (tiles' or groups') for itself -- all of it for the experts' totals, hence
+// the offsets, and the rows before its own tiles for those tiles' bases --
+// and places its tiles' slots.  Nothing is exchanged between workgroups: the
+// table is a few to a few hundred KB, read from L2 by 1024 threads with
+// several loads in flight, where a scan of its own with a ticket's release
+// and acquire, and a launch for the slots after it, took 12-30 us (16384
+// tokens of E 8: 7.7 + 4.0 us, 4096 of E 64: 23 + 5).  The last workgroup
+// computes aux and entropy instead.  Sums of floats keep a fixed order:
+// thread (group, e) adds the rows group, group + groups, ... ascending, the
+// groups of a wave and the experts meet in butterflies, the waves in order.
+constexpr int DP_NT = 1024;
+constexpr int DP_TPW = 16;  // most tiles per workgroup
+
 template <bool BF16>
-__global__ __launch_bounds__(SCAN_NT) void scan_kernel(ScanArgs a) {
-  __shared__ int wtot[SCAN_NT / 64];
-  __shared__ int s_last;
-  __shared__ int scount[MXM_MAX_EXPERTS];
-  __shared__ float spmean[MXM_MAX_EXPERTS];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int T = a.ntiles;
-  const int e = blockIdx.x;
-  constexpr int SB = 16;  // loads per lane issued together
-
-  if (e == a.E) {
-    if (wave == 0) {
+__global__ __launch_bounds__(DP_NT) void dispatch_kernel(DispatchArgs a, int table_rows, int rows_per,
+                                                         int tpw) {
+  __shared__ int tot[MXM_MAX_EXPERTS], bef[MXM_MAX_EXPERTS];
+  __shared__ int wsum[3][MXM_MAX_EXPERTS / 64];
+  __shared__ int base[DP_TPW][MXM_MAX_EXPERTS];
+  __shared__ float fpart[DP_NT], wterm[MXM_MAX_EXPERTS / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int E = a.E, K = a.K;
+  // table rows: tiles, or groups of rows_per tiles
+  const int32_t* __restrict__ tab = rows_per > 1 ? a.group_counts : a.tile_counts;
+  int lg = 2;  // experts padded to a power of two, one per thread of a group
+  while ((1 << lg) < E) ++lg;
+  const int Ep = 1 << lg, NG = DP_NT >> lg, e = tid & (Ep - 1), grp = tid >> lg;
+  const bool aux_wg = blockIdx.x == gridDim.x - 1;
+  const int t0 = blockIdx.x * tpw;                     // this workgroup's first tile
+  const int r0 = aux_wg ? 0 : t0 / rows_per;           // table rows before it
+  if (tid < MXM_MAX_EXPERTS) tot[tid] = bef[tid] = 0;
+  __syncthreads();
+  int vt = 0, vb = 0;
+  constexpr int U = 8;
+  for (int r = grp; r < table_rows; r += NG * U) {
+    int v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = r + u * NG;
+      v[u] = q < table_rows && e < E ? tab[(size_t)q * E + e] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      vt += v[u];
+      if (r + u * NG < r0) vb += v[u];
+    }
+  }
+  // rows of the same expert within a wave, then over the waves (integers:
+  // any order)
+  for (int o = Ep; o < 64; o <<= 1) {
+    vt += __shfl_xor(vt, o, 64);
+    vb += __shfl_xor(vb, o, 64);
+  }
+  if (e < E && (Ep >= 64 || lane < Ep)) {
+    atomicAdd(&tot[e], vt);
+    atomicAdd(&bef[e], vb);
+  }
+  __syncthreads();
+  // exclusive prefixes over the experts: rows, and the row tiles of both GEMMs
+  int c = 0, u1 = 0, u2 = 0, i0 = 0, i1 = 0, i2 = 0;
+  if (tid < MXM_MAX_EXPERTS) {
+    c = tid < E ? tot[tid] : 0;
+    u1 = (c + a.bm1 - 1) / a.bm1;
+    u2 = (c + a.bm2 - 1) / a.bm2;
+    i0 = c;
+    i1 = u1;
+    i2 = u2;
+#pragma unroll
+    for (int sh = 1; sh < 64; sh <<= 1) {
+      const int v0 = __shfl_up(i0, sh, 64), v1 = __shfl_up(i1, sh, 64), v2 = __shfl_up(i2, sh, 64);
+      if (lane >= sh) {
+        i0 += v0;
+        i1 += v1;
+        i2 += v2;
+      }
+    }
+    if (lane == 63) {
+      wsum[0][wave] = i0;
+      wsum[1][wave] = i1;
+      wsum[2][wave] = i2;
+    }
+  }
+  __syncthreads();
+  int off = 0;
+  if (tid < MXM_MAX_EXPERTS) {
+    for (int w = 0; w < wave; ++w) {
+      i0 += wsum[0][w];
+      i1 += wsum[1][w];
+      i2 += wsum[2][w];
+    }
+    off = i0 - c;
+    if (blockIdx.x == 0 && tid < E) {
+      a.counts[tid] = c;
+      a.offsets[tid] = off;
+      a.mstart1[tid] = i1 - u1;
+      a.mstart2[tid] = i2 - u2;
+      if (tid == E - 1) {
+        a.offsets[E] = i0;
+        a.mstart1[E] = i1;
+        a.mstart2[E] = i2;
+      }
+    }
+  }
+  if (aux_wg) {
+    const float* __restrict__ ps = rows_per > 1 ? a.group_psum : a.tile_psum;
+    float s = 0.0f;
+    for (int r = grp; r < table_rows; r += NG * U) {
+      float v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = r + u * NG;
+        v[u] = q < table_rows && e < E ? ps[(size_t)q * E + e] : 0.0f;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) s = s + v[u];
+    }
+    // the groups of a wave by a butterfly, then the waves in order
+    for (int o = Ep; o < 64; o <<= 1) s = s + __shfl_xor(s, o, 64);
+    const int ways = Ep < 64 ? DP_NT / 64 : NG, wd = Ep < 64 ? 64 : Ep;
+    fpart[tid] = s;
+    __syncthreads();
+    if (tid < MXM_MAX_EXPERTS) {
+      float term = 0.0f;
+      if (tid < E) {
+        s = fpart[tid];
+        for (int g = 1; g < ways; ++g) s = s + fpart[g * wd + tid];
+        const float mean = s / (float)a.N;
+        const float frac = ((float)c / (float)K) / (float)a.N;
+        term = (BF16 ? mxm_rbf(mean) : mean) * frac;
+      }
+      term = wave_sum_fixed(term);
+      if (lane == 0) wterm[wave] = term;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      float aux = wterm[0];
+#pragma unroll
+      for (int w = 1; w < MXM_MAX_EXPERTS / 64; ++w) aux = aux + wterm[w];
+      const float raw = aux * (float)E;
+      a.aux[0] = raw;
+      if (a.aux_scaled) a.aux_scaled[0] = raw * a.aux_weight;
+    }
+    if (wave == 1) {
+      const float* __restrict__ en = rows_per > 1 ? a.group_ent : a.tile_ent;
       float sum = 0.0f;
-      for (int t0 = lane; t0 < T; t0 += 64 * SB) {
-        float ev[SB];
+      for (int r = lane; r < table_rows; r += 64 * U) {
+        float v[U];
 #pragma unroll
-        for (int b = 0; b < SB; ++b) ev[b] = t0 + 64 * b < T ? a.tile_ent[t0 + 64 * b] : 0.0f;
+        for (int u = 0; u < U; ++u) v[u] = r + 64 * u < table_rows ? en[r + 64 * u] : 0.0f;
 #pragma unroll
-        for (int b = 0; b < SB; ++b)
-          if (t0 + 64 * b < T) sum = sum + ev[b];
+        for (int u = 0; u < U; ++u) sum = sum + v[u];
       }
       sum = wave_sum_fixed(sum);
       if (lane == 0) a.entropy[0] = -(sum / (float)a.N);
     }
     return;
   }
-
-  const int32_t* tc = a.tile_counts + (size_t)e * T;
-  if (wave == 0) {
-    const float* tp = a.tile_psum + (size_t)e * T;
-    float ps = 0.0f;
-    for (int t0 = lane; t0 < T; t0 += 64 * SB) {
-      float pv[SB];
-#pragma unroll
-      for (int b = 0; b < SB; ++b) pv[b] = t0 + 64 * b < T ? tp[t0 + 64 * b] : 0.0f;
-#pragma unroll
-      for (int b = 0; b < SB; ++b)
-        if (t0 + 64 * b < T) ps = ps + pv[b];
-    }
-    ps = wave_sum_fixed(ps);
-    if (lane == 0) {
-      const float mean = ps / (float)a.N;
-      a.expert_pmean[e] = BF16 ? mxm_rbf(mean) : mean;
+  // the bases of this workgroup's tiles
+  if (tid < E) {
+    int b = off + bef[tid];
+    for (int t = r0 * rows_per; t < t0; ++t) b += a.tile_counts[(size_t)t * E + tid];
+    const int nt = min(tpw, a.ntiles - t0);
+    for (int j = 0; j < nt; ++j) {
+      base[j][tid] = b;
+      if (j + 1 < nt) b += a.tile_counts[(size_t)(t0 + j) * E + tid];
     }
   }
-  // thread i owns tiles [i*R, i*R + R): its run total, the workgroup's
-  // exclusive scan of the run totals, then the tiles' bases
-  const int R = (T + SCAN_NT - 1) / SCAN_NT;
-  const int t_lo = min(T, tid * R), t_hi = min(T, t_lo + R);
-  int run = 0;
-  for (int t = t_lo; t < t_hi; ++t) run += tc[t];
-  int incl = run;
-#pragma unroll
-  for (int sh = 1; sh < 64; sh <<= 1) {
-    const int up = __shfl_up(incl, sh, 64);
-    if (lane >= sh) incl += up;
-  }
-  if (lane == 63) wtot[wave] = incl;
   __syncthreads();
-  int base = incl - run;
-  for (int w = 0; w < wave; ++w) base += wtot[w];
-  for (int t = t_lo; t < t_hi; ++t) {
-    a.tile_base[(size_t)e * T + t] = base;
-    base += tc[t];
+  const int n0 = t0 * a.tile_tokens;
+  const int nn = min(a.N - n0, tpw * a.tile_tokens);
+  const size_t s0 = (size_t)n0 * K;
+  const int shift = a.tile_tokens == 16 ? 4 : 6;
+  for (int i = tid; i < nn * K; i += DP_NT) {
+    const int ln = i / K;
+    const int pos = base[ln >> shift][a.top_idx[s0 + i]] + a.slot_rank[s0 + i];
+    a.perm[pos] = n0 + ln;
+    a.slot_pos[s0 + i] = pos;
   }
-  if (tid == SCAN_NT - 1) a.expert_count[e] = base;  // the expert's total
-
-  // ---- ticket: the last expert workgroup continues ----
-  __threadfence();
-  __syncthreads();
-  if (tid == 0) s_last = atomicAdd(a.ticket, 1) == a.E - 1;
-  __syncthreads();
-  if (!s_last) return;
-  __threadfence();
-  // every expert's total read in one round of loads
-  for (int x = tid; x < a.E; x += SCAN_NT) {
-    scount[x] = a.expert_count[x];
-    spmean[x] = a.expert_pmean[x];
-  }
-  __syncthreads();
-  if (tid == 0) {
-    int o = 0, m1 = 0, m2 = 0;
-    float aux = 0.0f;
-    for (int x = 0; x < a.E; ++x) {
-      const int c = scount[x];
-      a.offsets[x] = o;
-      a.counts[x] = c;
-      a.mstart1[x] = m1;
-      a.mstart2[x] = m2;
-      o += c;
-      m1 += (c + a.bm1 - 1) / a.bm1;
-      m2 += (c + a.bm2 - 1) / a.bm2;
-      const float frac = ((float)c / (float)a.K) / (float)a.N;
-      const float term = spmean[x] * frac;
-      aux = (x == 0) ? term : aux + term;
-    }
-    a.offsets[a.E] = o;
-    a.mstart1[a.E] = m1;
-    a.mstart2[a.E] = m2;
-    const float raw = aux * (float)a.E;
-    a.aux[0] = raw;
-    if (a.aux_scaled) a.aux_scaled[0] = raw * a.aux_weight;
-    __hip_atomic_store(a.ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-}
-
-__global__ __launch_bounds__(256) void scatter_kernel(ScatterArgs a) {
-  const int64_t s = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (s >= (int64_t)a.N * a.K) return;
-  const int n = (int)(s / a.K);
-  const int e = a.top_idx[s];
-  const int tile = n / MXM_ROUTER_TM;
-  const int pos = a.offsets[e] + a.tile_base[(size_t)e * a.ntiles + tile] + a.slot_rank[s];
-  a.perm[pos] = n;
-  a.slot_pos[s] = pos;
 }
 
 template <typename TY>
@@ -404,17 +477,25 @@ __global__ __launch_bounds__(256) void combine_tm_kernel(CombineArgs a) {
 
 }  // namespace
 
-void mxm_launch_scan(const ScanArgs& a, bool bf16, hipStream_t s) {
-  if (bf16)
-    hipLaunchKernelGGL(scan_kernel<true>, dim3(a.E + 1), dim3(SCAN_NT), 0, s, a);
-  else
-    hipLaunchKernelGGL(scan_kernel<false>, dim3(a.E + 1), dim3(SCAN_NT), 0, s, a);
+int mxm_dispatch_groups(int ntiles, int E) {
+  return (int64_t)ntiles * E > MXM_DISPATCH_TABLE
+             ? (ntiles + MXM_DISPATCH_GROUP - 1) / MXM_DISPATCH_GROUP
+             : 0;
 }
 
-void mxm_launch_scatter(const ScatterArgs& a, hipStream_t s) {
-  const int64_t slots = (int64_t)a.N * a.K;
-  const int blocks = (int)((slots + 255) / 256);
-  if (blocks > 0) hipLaunchKernelGGL(scatter_kernel, dim3(blocks), dim3(256), 0, s, a);
+void mxm_launch_dispatch(const DispatchArgs& a, bool bf16, hipStream_t s) {
+  const int groups = mxm_dispatch_groups(a.ntiles, a.E);
+  if (groups > 0) hipLaunchKernelGGL(dispatch_group_kernel, dim3(groups), dim3(256), 0, s, a);
+  // up to 256 workgroups of whole tiles (more past DP_TPW tiles each); tiles
+  // per workgroup a power of two, so that one lies within a group
+  int tpw = 1;
+  while (tpw < DP_TPW && (a.ntiles + tpw - 1) / tpw > 256) tpw *= 2;
+  const dim3 grid((a.ntiles + tpw - 1) / tpw + 1);
+  const int rows = groups > 0 ? groups : a.ntiles, per = groups > 0 ? MXM_DISPATCH_GROUP : 1;
+  if (bf16)
+    hipLaunchKernelGGL(dispatch_kernel<true>, grid, dim3(DP_NT), 0, s, a, rows, per, tpw);
+  else
+    hipLaunchKernelGGL(dispatch_kernel<false>, grid, dim3(DP_NT), 0, s, a, rows, per, tpw);
 }
 
 void mxm_launch_combine(const CombineArgs& a, bool y_bf16, hipStream_t s) {

@@ -10,6 +10,8 @@
 // Tokens per router tile; the dispatch bitmasks are two 32-bit words per
 // expert and tile, so this is fixed at 64.
 #define MXM_ROUTER_TM 64
+// Batches of up to this many tokens take tiles of 16 on the tiled router.
+#define MXM_ROUTER_SPLIT_N 16384
 // Largest expert count the router supports (4 experts per lane).
 #define MXM_MAX_EXPERTS 256
 
@@ -52,16 +54,18 @@ struct RouterArgs {
   const void* x;   // [N, D], bf16 bits or fp32
   const void* wr;  // [D, E], same dtype
   int N, D, E, K;
+  int ldx, Dx;           // x's row stride and columns (D, or more with zeros past D)
+  int tile_tokens;       // tokens per tile, 16 or 64
   int32_t* top_idx;      // [N, K]
   float* gates;          // [N, K]
   int32_t* slot_rank;    // [N, K] rank of the slot among the tile's tokens on that expert
-  int32_t* tile_counts;  // [E, ntiles]
-  float* tile_psum;      // [E, ntiles] sum of probabilities over the tile
+  int32_t* tile_counts;  // [ntiles, E]
+  float* tile_psum;      // [ntiles, E] sum of probabilities over the tile
   float* tile_ent;       // [ntiles] sum over the tile of sum_e p log max(p, 1e-12)
   float* probs_out;      // optional [N, E]
   // optional: router_w lane-interleaved as RouteSmallArgs::wr_t (ldw a
-  // multiple of 64 >= D); for E > 32 the logits then run on the fp32 matrix
-  // cores (same bits)
+  // multiple of 64 >= D); the logits then run on the fp32 matrix cores (same
+  // bits)
   const void* wr_t;
   int ldw;
 };
@@ -110,37 +114,38 @@ void mxm_launch_route_small(const RouteSmallArgs& a, bool bf16, hipStream_t s);
 // (one workgroup) from the per-token results already written.
 void mxm_launch_route_dispatch(const RouteSmallArgs& a, bool bf16, hipStream_t s);
 
-struct ScanArgs {
-  const int32_t* tile_counts;  // [E, ntiles]
-  const float* tile_psum;      // [E, ntiles]
+// Dispatch of the tiled router's batches: per-expert counts, offsets and
+// row-tile prefixes, the stable permutation, aux and entropy from the tiles'
+// histograms and sums.
+struct DispatchArgs {
+  const int32_t* tile_counts;  // [ntiles, E]
+  const float* tile_psum;      // [ntiles, E]
   const float* tile_ent;       // [ntiles]
-  int N, E, K, ntiles;
+  const int32_t* top_idx;      // [N, K]
+  const int32_t* slot_rank;    // [N, K]
+  int N, E, K, ntiles, tile_tokens;
   int bm1, bm2;         // row-tile heights of the two grouped GEMMs
+  // sums over groups of MXM_DISPATCH_GROUP tiles, where the batch has more
+  // than MXM_DISPATCH_TABLE histogram entries (mxm_dispatch_groups)
+  int32_t* group_counts;  // [groups, E]
+  float* group_psum;      // [groups, E]
+  float* group_ent;       // [groups]
   int32_t* counts;      // [E]
   int32_t* offsets;     // [E + 1]
-  int32_t* tile_base;   // [E, ntiles] first position of the tile's rows on e, relative to offsets[e]
   int32_t* mstart1;     // [E + 1] prefix of ceil(counts / bm1)
   int32_t* mstart2;     // [E + 1] prefix of ceil(counts / bm2)
+  int32_t* perm;        // [N*K] permuted position -> token
+  int32_t* slot_pos;    // [N*K] slot (n, k) -> permuted position
   float* aux;           // [1]
   float* entropy;       // [1]
   float aux_weight;     // block level: aux_scaled = aux * aux_weight
   float* aux_scaled;    // [1] or null
-  int32_t* expert_count;  // [E] scratch: each workgroup's expert total
-  float* expert_pmean;    // [E] scratch: each workgroup's mean probability
-  int32_t* ticket;        // [1], zero between calls (the last workgroup resets it)
 };
-void mxm_launch_scan(const ScanArgs& a, bool bf16, hipStream_t s);
-
-struct ScatterArgs {
-  const int32_t* top_idx;
-  const int32_t* slot_rank;
-  const int32_t* tile_base;  // relative to offsets[e]
-  const int32_t* offsets;
-  int N, K, ntiles;
-  int32_t* perm;      // [N*K] permuted position -> token
-  int32_t* slot_pos;  // [N*K] slot (n, k) -> permuted position
-};
-void mxm_launch_scatter(const ScatterArgs& a, hipStream_t s);
+#define MXM_DISPATCH_GROUP 32
+#define MXM_DISPATCH_TABLE (1 << 18)
+// Groups of tiles whose sums the dispatch keeps (0: it reads the tiles').
+int mxm_dispatch_groups(int ntiles, int E);
+void mxm_launch_dispatch(const DispatchArgs& a, bool bf16, hipStream_t s);
 
 // aux and entropy of a decode batch from its per-token results (the int8
 // decode flow computes them in one more workgroup of its gate+up launch).

@@ -2,20 +2,19 @@
 // (gpu/ir.cpp:1106-1111), fused with the per-tile pieces of dispatch and of
 // the aux / entropy outputs (gpu/ir.cpp:1150-1162).
 //
-// One workgroup owns a tile of MXM_ROUTER_TM consecutive tokens and all E
-// experts.  Phase 1 computes the logits in their summation order
-// (mxm_numerics.h): per 64-d chunk of d, a partial by fmaf over the chunk's
-// d ascending from +0, added to the logit in chunk order -- the order the
-// CPU restatement uses, so logits are bit-identical.  For E > 32 the fmaf
-// chains run on the fp32 matrix cores (logits_mfma, a pass per group of 64
-// experts), otherwise as a register-tiled SIMT product on the vector unit.
-// Phase 2
-// gives each wavefront 16 tokens: one lane per expert (lane l holds experts
-// l, l+64, ...), softmax with a fixed xor-butterfly sum, top-k by K rounds of
-// a wave-wide argmax under the total order (p desc, expert asc), i.e. the
-// order of a stable argsort(-p).  Phase 3 writes, per tile, the per-expert
+// One workgroup owns a tile of 64 or 16 consecutive tokens and all E experts.
+// Phase 1 computes the logits in their summation order (mxm_numerics.h): per
+// 64-d chunk of d, a partial by fmaf over the chunk's d ascending from +0,
+// added to the logit in chunk order -- the order the CPU restatement uses, so
+// logits are bit-identical.  The fmaf chains run on the fp32 matrix cores
+// (router_mf_kernel), or, for rows that are not whole 16-byte pieces, as a
+// register-tiled SIMT product on the vector unit.  Phase 2 gives each
+// wavefront a quarter of the tokens: one lane per expert (lane l holds experts
+// l, l+64, ...; E <= 32 several tokens at once), softmax with a fixed
+// xor-butterfly sum, top-k under the total order (p desc, expert asc), i.e.
+// the order of a stable argsort(-p).  Phase 3 writes, per tile, the per-expert
 // token bitmasks' popcounts (the tile histogram) and each slot's rank among
-// the tile's tokens routed to the same expert; the scan kernel turns these
+// the tile's tokens routed to the same expert; the dispatch kernel turns these
 // into the stable permutation.
 //
 // Decode-sized batches take route_small_kernel instead (one launch for the
@@ -270,7 +269,7 @@ __device__ __forceinline__ float route_token_seg(float v, int lane, int E, int K
 // Phase 2 of the tiled router for E <= SEG: the wave's TPW tokens, 64 / SEG at
 // a time.  The per-expert probability sums (lane e) and the entropy sum take
 // the tokens one by one in token order, as the one-token-per-pass loop does.
-template <bool BF16, int SEG, int TPW, int LGS, int EPP>
+template <bool BF16, int SEG, int TPW, int LGS>
 __device__ __forceinline__ void route_tile_seg(const float* lg, int wave, int lane, int n0, int N,
                                                int E, int K, float* probs_out, int32_t* top_idx,
                                                float* gates, uint32_t (*mask)[2], RankScratch* rsc,
@@ -304,31 +303,28 @@ __device__ __forceinline__ void route_tile_seg(const float* lg, int wave, int la
       }
     }
   }
-  (void)EPP;
 }
 
-// ---- logits on the fp32 matrix cores (E in 33..64) -------------------------
+// ---- logits on the fp32 matrix cores ---------------------------------------
 // v_mfma_f32_16x16x1_4b_f32 is four 16 x 16 blocks of fused multiply-adds
 // with one product each: D = C + A B rounded once, to nearest even,
 // denormals kept -- the fmaf of the logits' summation order, bit for bit
 // (checked on the part against fmaf chains over bf16-valued, fp32, wide-
 // exponent, denormal, signed-zero and cancelling operands).  A chain of them
-// over a chunk's d from +0 is therefore the SIMT path's chunk partial, at
-// twice the rate of the non-packed fp32 FMA.
+// over a chunk's d from +0 is therefore a chunk's partial.
 //
-// A wave computes 16 tokens x 64 experts.  A = tokens, broadcast to the four
-// blocks from lane group k = lane / 16 (cbsz 2, abid k); B = experts, lane l
-// holding expert l (blocks b = experts 16 b .. 16 b + 15).  The output's
-// register 4 b + q in lane l is token (l / 16) * 4 + q, expert 16 b + l % 16.
-// A round is 32 d: lane group k loads its token's d0 + 8k .. d0 + 8k + 7
-// from x (one 16-byte piece in bf16, two in fp32), and every lane its
-// expert's 32 d from the lane-interleaved router copy (4 or 8 pieces).
+// A wave computes 16 tokens x 16 G experts (G = 1, 2, 4).  The blocks take
+// the G groups of 16 experts and 4 / G chunks at once, each block its own
+// chunk's chain: lane l works on token l % 16, expert group b % G (b = l / 16)
+// and chunk c + b / G, and holds those operands itself.  Register 4 b + q of
+// lane l of the result is token (l / 16) * 4 + q, expert l % 16 of its group,
+// so a token's partials of the round's chunks are in one lane, in registers.
 typedef float mxm_lg16 __attribute__((ext_vector_type(16)));
 
 template <typename TX>
-struct LgRound {
+struct LgHalf {  // 32 d of a chunk
   static constexpr int P = 16 / (int)sizeof(TX);  // values per 16-byte piece
-  uint4 xu[8 / P];
+  uint4 xu[32 / P];
   uint4 wu[32 / P];
 };
 
@@ -341,390 +337,372 @@ __device__ __forceinline__ float lg_val(const uint4& u, int j) {
   else return mxm_u2f(w);
 }
 
-// x through a buffer descriptor over the wave's 16 token rows: the loads
-// are unconditional (a range check in the load returns zeros), so every
-// path leaves the same loads in flight and the wait before a round counts
-// only the older round's.  Word 3 of a gfx9 raw buffer descriptor: 32-bit
+// Operands through buffer descriptors (the wave's 16 token rows; a group of
+// 64 experts of the router copy): the loads are unconditional, a range check
+// in the load returns zeros.  Word 3 of a gfx9 raw buffer descriptor: 32-bit
 // data format, no swizzle.
 constexpr int LG_RSRC_W3 = 0x00020000;
-constexpr int LG_OUT_OF_RANGE = 0x7ffffff0;  // above any wave's record count
+constexpr int LG_OUT_OF_RANGE = 0x7ffffff0;  // above any record count
 typedef uint32_t lg_u4 __attribute__((ext_vector_type(4)));
 
-// Round r's pieces.  x pieces at or past D (D % P == 0, so a piece is wholly
-// in or out) take an offset past the records and tokens past N lie past
-// them, so both load as zeros; the router copy is zero past D up to its
-// ldw, a multiple of 64 >= 32 * rounds.
 template <typename TX>
-__device__ __forceinline__ void lg_load(LgRound<TX>& R, __amdgpu_buffer_rsrc_t xs, int xoff, int D,
-                                        const uint4* wt, int lane, int r) {
-  constexpr int P = LgRound<TX>::P;
-  const int d0 = 32 * r + 8 * (lane >> 4);
+struct LgSrc {
+  __amdgpu_buffer_rsrc_t xs, ws;
+  int xoff;   // this lane's token row
+  int woff;   // this lane's expert
+  int D;
+};
+
+// d0 .. d0 + 31 of the lane's token and expert.  x pieces at or past D (its columns, D % P
+// == 0, so a piece is wholly in or out) take an offset past the records and
+// tokens past N lie past them, so both load as zeros; the router copy is
+// zero from D to its end, past which its pieces load as zeros too.
+template <typename TX>
+__device__ __forceinline__ void lg_load(LgHalf<TX>& R, const LgSrc<TX>& S, int d0) {
+  constexpr int P = LgHalf<TX>::P;
 #pragma unroll
-  for (int h = 0; h < 8 / P; ++h) {
+  for (int h = 0; h < 32 / P; ++h) {
     const int d = d0 + P * h;
-    const int off = d < D ? xoff + d * (int)sizeof(TX) : LG_OUT_OF_RANGE;
-    const lg_u4 v = __builtin_amdgcn_raw_buffer_load_b128(xs, off, 0, 0);
+    const int off = d < S.D ? S.xoff + d * (int)sizeof(TX) : LG_OUT_OF_RANGE;
+    const lg_u4 v = __builtin_amdgcn_raw_buffer_load_b128(S.xs, off, 0, 0);
     R.xu[h] = make_uint4(v.x, v.y, v.z, v.w);
-  }
-  const uint4* wp = wt + (size_t)(32 / P) * r * 64 + lane;
-#pragma unroll
-  for (int c = 0; c < 32 / P; ++c) R.wu[c] = wp[c * 64];
-}
-
-// the 8 d of lane group KK: d0 + 8 KK + t, t ascending
-template <typename TX, int KK, bool FIRST>
-__device__ __forceinline__ void lg_group(const LgRound<TX>& R, mxm_lg16& c) {
-  constexpr int P = LgRound<TX>::P;
-#pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    const float a = lg_val<TX>(R.xu[t / P], t % P);
-    const float b = lg_val<TX>(R.wu[(8 * KK + t) / P], (8 * KK + t) % P);
-    if (FIRST && t == 0)
-      c = __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, mxm_lg16{}, 2, KK, 0);
-    else
-      c = __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, c, 2, KK, 0);
+    const lg_u4 w = __builtin_amdgcn_raw_buffer_load_b128(S.ws, S.woff + (d / P) * 1024, 0, 0);
+    R.wu[h] = make_uint4(w.x, w.y, w.z, w.w);
   }
 }
 
-// a round's 32 d in ascending order; FIRST starts the chunk partial at +0
+// The 32 d in ascending order; FIRST starts the chunk partials at +0.
 template <typename TX, bool FIRST>
-__device__ __forceinline__ void lg_round(const LgRound<TX>& R, mxm_lg16& c) {
-  lg_group<TX, 0, FIRST>(R, c);
-  lg_group<TX, 1, false>(R, c);
-  lg_group<TX, 2, false>(R, c);
-  lg_group<TX, 3, false>(R, c);
+__device__ __forceinline__ void lg_half(const LgHalf<TX>& R, mxm_lg16& c) {
+  constexpr int P = LgHalf<TX>::P;
+#pragma unroll
+  for (int t = 0; t < 32; ++t) {
+    const float a = lg_val<TX>(R.xu[t / P], t % P);
+    const float b = lg_val<TX>(R.wu[t / P], t % P);
+    if (FIRST && t == 0)
+      c = __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, mxm_lg16{}, 0, 0, 0);
+    else
+      c = __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, c, 0, 0, 0);
+  }
 }
 
-// The logits of tokens n0w .. n0w + 15 against the 64 (padded) experts: per
-// 64-d chunk (two rounds) a partial from +0, added to the logit (from +0) in
-// chunk order.  Both rounds of the last chunk run: past D the x pieces and
-// the router copy (zero up to ldw) are zeros, and fma(0, 0, c) = c except
-// that a -0 partial (a product that underflowed to -0) becomes +0, which
-// the logit's addition absorbs (the logit, a sum from +0, is never -0, and
-// adding either zero leaves it as it is).  The next round's
-// pieces are loaded while a round computes (after the last chunk, its
-// second round again, unused).  Needs 16 D sizeof(TX) < 2^30 (the launcher
-// checks).
-template <typename TX>
-__device__ __forceinline__ mxm_lg16 logits_mfma(const TX* x, const TX* wr_t, int N, int D,
-                                                int n0w, int lane) {
+// Sources of a wave for tokens n0w .. n0w + 15 and the experts 64 g .. a
+// group of 64 of the router copy, [ldw / P][64][P] (1024 bytes per P values of
+// d).
+template <typename TX, int G>
+__device__ __forceinline__ LgSrc<TX> lg_source(const TX* x, int ldx, const TX* wr_t, int ldw, int N,
+                                               int Dx, int n0w, int lane) {
   // (readfirstlane: the clamp is computed on the vector unit, and a
   // descriptor in vector registers would be taken apart lane by lane)
   const int rows = __builtin_amdgcn_readfirstlane(N - n0w >= 16 ? 16 : N - n0w > 0 ? N - n0w : 0);
-  const __amdgpu_buffer_rsrc_t xs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<TX*>(rows > 0 ? x + (size_t)n0w * D : x), (short)0, rows * D * (int)sizeof(TX),
+  LgSrc<TX> S;
+  S.xs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<TX*>(rows > 0 ? x + (size_t)n0w * ldx : x), (short)0, rows * ldx * (int)sizeof(TX),
       LG_RSRC_W3);
-  const int xoff = (lane & 15) * D * (int)sizeof(TX);
-  const uint4* wt = reinterpret_cast<const uint4*>(wr_t);
-  const int nch = (D + 63) / 64;
-  mxm_lg16 lgt = {};
-  LgRound<TX> ra, rb;
-  // (the scheduling barriers keep each round's loads issued before the
-  // other round's products instead of next to their own uses)
-  lg_load<TX>(ra, xs, xoff, D, wt, lane, 0);
-  for (int ch = 0; ch < nch; ++ch) {
-    lg_load<TX>(rb, xs, xoff, D, wt, lane, 2 * ch + 1);
-    __builtin_amdgcn_sched_barrier(0);
-    mxm_lg16 part;
-    lg_round<TX, true>(ra, part);
-    __builtin_amdgcn_sched_barrier(0);
-    lg_load<TX>(ra, xs, xoff, D, wt, lane, min(2 * ch + 2, 2 * nch - 1));
-    __builtin_amdgcn_sched_barrier(0);
-    lg_round<TX, false>(rb, part);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) lgt[i] = lgt[i] + part[i];
-  }
-  return lgt;
+  S.ws = __builtin_amdgcn_make_buffer_rsrc(const_cast<TX*>(wr_t), (short)0,
+                                           ldw * 64 * (int)sizeof(TX), LG_RSRC_W3);
+  S.xoff = (lane & 15) * ldx * (int)sizeof(TX);
+  S.woff = (((lane >> 4) % G) * 16 + (lane & 15)) * 16;
+  S.D = Dx;
+  return S;
 }
 
-// EPT = experts per thread in phase 1 (E padded to 16*EPT).  MF: phase 1 on
-// the fp32 matrix cores (EPT 4, 8 or 16; wr_t is the lane-interleaved router
-// copy [EPT/4][ldw/P][64][P], x 16-byte aligned with D % P == 0).
-template <typename TX, bool BF16, int EPT, bool VEC, bool MF = false>
-__global__ __launch_bounds__(NT) void router_kernel(
-    const TX* __restrict__ x, const TX* __restrict__ wr, int N, int D, int E, int K,
-    int32_t* __restrict__ top_idx, float* __restrict__ gates, int32_t* __restrict__ slot_rank,
-    int32_t* __restrict__ tile_counts, float* __restrict__ tile_psum, float* __restrict__ tile_ent,
-    float* __restrict__ probs_out, int ntiles,
-    const TX* __restrict__ wr_t, int ldw) {
-  constexpr int EP = 16 * EPT;
-  constexpr int NJ = (EP + 63) / 64;  // experts per lane in phase 2
-  constexpr int LG_STRIDE = EP + 1;
-  constexpr int STAGE_FLOATS = BK * TM + BK * EP;
-  constexpr int LG_FLOATS = TM * LG_STRIDE;
-  constexpr int SMEM_FLOATS = MF ? LG_FLOATS : STAGE_FLOATS > LG_FLOATS ? STAGE_FLOATS : LG_FLOATS;
-  __shared__ __attribute__((aligned(16))) float smem[SMEM_FLOATS];
-  __shared__ uint32_t mask[EP][2];
-  constexpr int THREADS = NT;
-  constexpr int NWAVE = THREADS / 64;
-  __shared__ float wave_psum[NWAVE][EP];
-  __shared__ float wave_ent[NWAVE];
-  __shared__ __attribute__((aligned(16))) RankScratch rank_scr[NWAVE];
+// ---- phases 2 and 3 of a tile ------------------------------------------------
+// Per-workgroup scratch of a tile of TT tokens (EP: E padded to the kernel's
+// expert count).
+template <int EP>
+struct TileScratch {
+  uint32_t mask[EP][2];
+  float wave_psum[NT / 64][EP];
+  float wave_ent[NT / 64];
+  __attribute__((aligned(16))) RankScratch rank[NT / 64];
+};
 
-  float* xs = smem;            // [BK][TM]
-  float* ws = smem + BK * TM;  // [BK][EP]
-  float* lg = smem;            // [TM][LG_STRIDE] after phase 1
-
-  const int tid = threadIdx.x;
-  const int tile = blockIdx.x;
-  const int n0 = tile * TM;
-  for (int i = tid; i < EP * 2; i += THREADS) (&mask[0][0])[i] = 0u;
-
-  // ---- phase 1: logits --------------------------------------------------
-  if constexpr (MF) {
-    // one pass of 64 experts per group of the lane-interleaved copy (its
-    // groups lie ldw * 64 elements apart); each pass reads the wave's x rows
-    // again
-    static_assert(EP % 64 == 0, "the matrix-core logits cover groups of 64 experts");
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), ln = tid & 63;  // wv: uniform
-    for (int g = 0; g < EP / 64; ++g) {
-      const mxm_lg16 v = logits_mfma<TX>(x, wr_t + (size_t)g * ldw * 64, N, D, n0 + 16 * wv, ln);
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int t = 16 * wv + (ln >> 4) * 4 + q;
-          lg[t * LG_STRIDE + 64 * g + 16 * b + (ln & 15)] =
-              BF16 ? mxm_rbf(v[4 * b + q]) : v[4 * b + q];
-        }
-    }
-    __syncthreads();
-  } else {
-    const int ty = tid >> 4;  // tokens ty*4 .. ty*4+3
-    const int tx = tid & 15;  // experts tx*EPT .. tx*EPT+EPT-1
-    float acc[4][EPT];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < EPT; ++j) acc[i][j] = 0.0f;
-
-    // products of one BK chunk held in LDS (BK is the logits' 64-d summation
-    // chunk): a partial from +0, then added to the logit
-    static_assert(BK == MXM_LOGIT_CHUNK, "one LDS chunk per summation chunk");
-    auto compute = [&]() {
-      float part[4][EPT];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < EPT; ++j) part[i][j] = 0.0f;
-#pragma unroll 4
-      for (int dd = 0; dd < BK; ++dd) {
-        const float4 xv = *reinterpret_cast<const float4*>(&xs[dd * TM + ty * 4]);
-        float wv[EPT];
-#pragma unroll
-        for (int j = 0; j < EPT; ++j) wv[j] = ws[dd * EP + tx * EPT + j];
-#pragma unroll
-        for (int j = 0; j < EPT; ++j) {
-          part[0][j] = __builtin_fmaf(xv.x, wv[j], part[0][j]);
-          part[1][j] = __builtin_fmaf(xv.y, wv[j], part[1][j]);
-          part[2][j] = __builtin_fmaf(xv.z, wv[j], part[2][j]);
-          part[3][j] = __builtin_fmaf(xv.w, wv[j], part[3][j]);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < EPT; ++j) acc[i][j] = acc[i][j] + part[i][j];
-    };
-    if constexpr (VEC) {
-      // 16-byte pieces of x (token-fastest across lanes, so the transposed LDS
-      // store is conflict-free) and of router_w rows.  The next chunk's pieces
-      // are loaded into registers while the current chunk's products run;
-      // pieces outside [N, D] x [D, E] are loaded from a valid address and
-      // zeroed when stored.
-      constexpr int PER = 16 / (int)sizeof(TX);
-      constexpr int XPC = TM * BK / PER;  // x pieces per chunk
-      constexpr int WPC = BK * EP / PER;  // router_w pieces per chunk
-      constexpr int XP = (XPC + NT - 1) / NT, WP = (WPC + NT - 1) / NT;
-      static_assert(WP <= 32 && XP <= 32, "validity masks are 32 bits");
-      uint4 xr[XP], wrr[WP];
-      uint32_t xok = 0u, wok = 0u;
-      auto load = [&](int d0) {
-        xok = 0u;
-        wok = 0u;
-#pragma unroll
-        for (int p = 0; p < XP; ++p) {
-          const int i = tid + p * NT;
-          const int t = i % TM, dc = i / TM;
-          const int n = n0 + t, d = d0 + dc * PER;
-          const bool ok = i < XPC && n < N && d < D;
-          xr[p] = *reinterpret_cast<const uint4*>(x + (ok ? (size_t)n * D + d : 0));
-          xok |= ok ? (1u << p) : 0u;
-        }
-#pragma unroll
-        for (int p = 0; p < WP; ++p) {
-          const int j = tid + p * NT;
-          const int dd = j / (EP / PER), ec = (j % (EP / PER)) * PER;
-          const int d = d0 + dd;
-          const bool ok = j < WPC && d < D && ec < E;
-          wrr[p] = *reinterpret_cast<const uint4*>(wr + (ok ? (size_t)d * E + ec : 0));
-          wok |= ok ? (1u << p) : 0u;
-        }
-      };
-      auto store = [&]() {
-#pragma unroll
-        for (int p = 0; p < XP; ++p) {
-          const int i = tid + p * NT;
-          if (i < XPC) {
-            const int t = i % TM, dc = i / TM;
-            float f[PER];
-            unpack16<TX>(xr[p], f);
-            const bool ok = (xok >> p) & 1u;
-#pragma unroll
-            for (int q = 0; q < PER; ++q) xs[(dc * PER + q) * TM + t] = ok ? f[q] : 0.0f;
-          }
-        }
-#pragma unroll
-        for (int p = 0; p < WP; ++p) {
-          const int j = tid + p * NT;
-          if (j < WPC) {
-            const int dd = j / (EP / PER), ec = (j % (EP / PER)) * PER;
-            float f[PER];
-            unpack16<TX>(wrr[p], f);
-            const bool ok = (wok >> p) & 1u;
-#pragma unroll
-            for (int q = 0; q < PER; q += 4)
-              *reinterpret_cast<float4*>(&ws[dd * EP + ec + q]) =
-                  ok ? make_float4(f[q], f[q + 1], f[q + 2], f[q + 3]) : make_float4(0.f, 0.f, 0.f, 0.f);
-          }
-        }
-      };
-      load(0);
-      for (int d0 = 0; d0 < D; d0 += BK) {
-        __syncthreads();  // the previous chunk's products are done with LDS
-        store();
-        __syncthreads();
-        if (d0 + BK < D) load(d0 + BK);
-        compute();
-      }
-    } else {
-      for (int d0 = 0; d0 < D; d0 += BK) {
-        __syncthreads();
-        for (int i = tid; i < TM * BK; i += NT) {
-          const int t = i % TM, dd = i / TM;
-          const int n = n0 + t, d = d0 + dd;
-          xs[dd * TM + t] = (n < N && d < D) ? ld_as_f32<TX>(x + (size_t)n * D + d) : 0.0f;
-        }
-        for (int i = tid; i < BK * EP; i += NT) {
-          const int dd = i / EP, e = i % EP;
-          const int d = d0 + dd;
-          ws[i] = (d < D && e < E) ? ld_as_f32<TX>(wr + (size_t)d * E + e) : 0.0f;
-        }
-        __syncthreads();
-        compute();
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < EPT; ++j) {
-        const float v = acc[i][j];
-        lg[(ty * 4 + i) * LG_STRIDE + tx * EPT + j] = BF16 ? mxm_rbf(v) : v;
-      }
-    __syncthreads();
-  }
-
-  // ---- phase 2: softmax, top-k, gates -----------------------------------
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
+// Softmax, top-k and gates of tokens n0 .. n0 + TT - 1 from their logits
+// lg[t][LGS] in LDS, then the tile's histogram, slot ranks and aux partials.
+// All NT threads; starts and ends with the scratch and lg free of readers.
+template <bool BF16, int EP, int TT, int LGS>
+__device__ __forceinline__ void route_tile(const float* lg, TileScratch<EP>& sc, int n0, int tile,
+                                           const RouterArgs& a) {
+  constexpr int NJ = (EP + 63) / 64;  // experts per lane
+  constexpr int NWAVE = NT / 64, TPW = TT / NWAVE;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int N = a.N, E = a.E, K = a.K;
+  for (int i = tid; i < EP * 2; i += NT) (&sc.mask[0][0])[i] = 0u;
+  __syncthreads();  // the logits are written, the masks cleared
   float psum[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; ++j) psum[j] = 0.0f;
   float ent_acc = 0.0f;
-
-  // E <= 32 (the EPT 1 and 2 instantiations): several tokens on one wave at
-  // once, a lane segment each
+  // E <= 32: several tokens on one wave at once, a lane segment each (no
+  // more than the wave has)
   bool seg_done = false;
-  if constexpr (EPT <= 2) {
-    if (E <= 32) {
-      float ps = 0.0f;
-      constexpr int TPW = TM / NWAVE;
-      if (E <= 4)
-        route_tile_seg<BF16, 4, TPW, LG_STRIDE, EP>(lg, wave, lane, n0, N, E, K, probs_out, top_idx,
-                                                    gates, mask, &rank_scr[wave], ps, ent_acc);
-      else if (E <= 8)
-        route_tile_seg<BF16, 8, TPW, LG_STRIDE, EP>(lg, wave, lane, n0, N, E, K, probs_out, top_idx,
-                                                    gates, mask, &rank_scr[wave], ps, ent_acc);
-      else if (E <= 16)
-        route_tile_seg<BF16, 16, TPW, LG_STRIDE, EP>(lg, wave, lane, n0, N, E, K, probs_out,
-                                                     top_idx, gates, mask, &rank_scr[wave], ps,
-                                                     ent_acc);
-      else
-        route_tile_seg<BF16, 32, TPW, LG_STRIDE, EP>(lg, wave, lane, n0, N, E, K, probs_out,
-                                                     top_idx, gates, mask, &rank_scr[wave], ps,
-                                                     ent_acc);
-      psum[0] = ps;
-      seg_done = true;
-    }
+  if constexpr (EP <= 32) {
+    auto seg = [&](auto w) {
+      constexpr int SEG = decltype(w)::value;
+      route_tile_seg<BF16, SEG, TPW, LGS>(lg, wave, lane, n0, N, E, K, a.probs_out, a.top_idx,
+                                          a.gates, sc.mask, &sc.rank[wave], psum[0], ent_acc);
+    };
+    if (TT >= 64 && E <= 4) seg(std::integral_constant<int, (TT >= 64 ? 4 : 16)>{});
+    else if (TT >= 64 && E <= 8) seg(std::integral_constant<int, (TT >= 64 ? 8 : 16)>{});
+    else if (E <= 16) seg(std::integral_constant<int, 16>{});
+    else seg(std::integral_constant<int, 32>{});
+    seg_done = true;
   }
-  for (int tt = 0; tt < TM / NWAVE && !seg_done; ++tt) {
-    const int t = wave * (TM / NWAVE) + tt;
+  for (int tt = 0; tt < TPW && !seg_done; ++tt) {
+    const int t = wave * TPW + tt;
     const int n = n0 + t;
     if (n >= N) break;
     float v[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       const int e = lane + 64 * j;
-      v[j] = (e < E) ? lg[t * LG_STRIDE + e] : -__builtin_inff();
+      v[j] = (e < E) ? lg[t * LGS + e] : -__builtin_inff();
     }
     float p[NJ], pick_g[NJ];
     int pick_e[NJ];
-    ent_acc = ent_acc + route_token<BF16, NJ>(v, lane, E, K, p, pick_e, pick_g, &rank_scr[wave]);
+    ent_acc = ent_acc + route_token<BF16, NJ>(v, lane, E, K, p, pick_e, pick_g, &sc.rank[wave]);
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       const int e = lane + 64 * j;
       if (e < E) {
         psum[j] = psum[j] + p[j];
-        if (probs_out) probs_out[(size_t)n * E + e] = p[j];
+        if (a.probs_out) a.probs_out[(size_t)n * E + e] = p[j];
       }
     }
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       const int k = lane + 64 * j;
       if (k < K) {
-        top_idx[(size_t)n * K + k] = pick_e[j];
-        gates[(size_t)n * K + k] = pick_g[j];
-        atomicOr(&mask[pick_e[j]][t >> 5], 1u << (t & 31));
+        a.top_idx[(size_t)n * K + k] = pick_e[j];
+        a.gates[(size_t)n * K + k] = pick_g[j];
+        atomicOr(&sc.mask[pick_e[j]][t >> 5], 1u << (t & 31));
       }
     }
   }
 
-  if (lane == 0) wave_ent[wave] = ent_acc;
+  if (lane == 0) sc.wave_ent[wave] = ent_acc;
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     const int e = lane + 64 * j;
-    if (e < EP) wave_psum[wave][e] = psum[j];
+    if (e < EP) sc.wave_psum[wave][e] = psum[j];
   }
   __syncthreads();
 
-  // ---- phase 3: tile histogram, slot ranks, aux partials -----------------
-  for (int e = tid; e < E; e += THREADS) {
-    tile_counts[(size_t)e * ntiles + tile] = __popc(mask[e][0]) + __popc(mask[e][1]);
-    float ps = wave_psum[0][e];
+  for (int e = tid; e < E; e += NT) {
+    a.tile_counts[(size_t)tile * E + e] = __popc(sc.mask[e][0]) + __popc(sc.mask[e][1]);
+    float ps = sc.wave_psum[0][e];
 #pragma unroll
-    for (int w = 1; w < NWAVE; ++w) ps = ps + wave_psum[w][e];
-    tile_psum[(size_t)e * ntiles + tile] = ps;
+    for (int w = 1; w < NWAVE; ++w) ps = ps + sc.wave_psum[w][e];
+    a.tile_psum[(size_t)tile * E + e] = ps;
   }
   if (tid == 0) {
-    float en = wave_ent[0];
+    float en = sc.wave_ent[0];
 #pragma unroll
-    for (int w = 1; w < NWAVE; ++w) en = en + wave_ent[w];
-    tile_ent[tile] = en;
+    for (int w = 1; w < NWAVE; ++w) en = en + sc.wave_ent[w];
+    a.tile_ent[tile] = en;
   }
-  for (int i = tid; i < TM * K; i += THREADS) {
+  for (int i = tid; i < TT * K; i += NT) {
     const int t = i / K;
     const int n = n0 + t;
     if (n >= N) continue;
-    const int e = top_idx[(size_t)n * K + (i % K)];
-    const uint32_t lo = mask[e][0], hi = mask[e][1];
+    const int e = a.top_idx[(size_t)n * K + (i % K)];
+    const uint32_t lo = sc.mask[e][0], hi = sc.mask[e][1];
     int r;
     if (t < 32)
       r = __popc(lo & ((1u << t) - 1u));
     else
       r = __popc(lo) + __popc(hi & ((1u << (t - 32)) - 1u));
-    slot_rank[(size_t)n * K + (i % K)] = r;
+    a.slot_rank[(size_t)n * K + (i % K)] = r;
   }
+  __syncthreads();
+}
+
+// The tiled router, logits on the matrix cores (x rows 16-byte aligned, D a
+// multiple of a 16-byte piece).  TT tokens per workgroup of four waves:
+//   TT = 64: wave w computes tokens 16 w .. 16 w + 15 over all of D, the
+//     partials added in registers;
+//   TT = 16: the four waves take every fourth round of chunks of the same 16
+//     tokens and leave the partials in LDS, where each thread adds its logits'
+//     in chunk order -- for batches whose 64-token tiles would leave most
+//     SIMDs without a wave, where a wave's chain of dependent rounds is the
+//     time (see MXM_ROUTER_SPLIT_N).
+// EP = 16 G experts, or 64 NP for E > 64 (passes of 64, G = 4).
+// Bound by the chain of rounds (a round of 64 k = 1 products is 2048 clocks of
+// the matrix core) and, in large batches, by the products themselves.
+// Measured, against 64-token tiles on the vector unit (E <= 32) or with 64
+// experts a round from broadcast x: 1999 tokens of D 1024 / E 16 37.5 -> 6.9
+// us, 4096 of D 2048 / E 64 89 -> 34 us, 16384 of D 512 / E 8 24 -> 11 us, 65536
+// of D 1024 / E 16 (tiles of 64) 79 -> 47 us, of D 2048 / E 64 unchanged at 225.
+template <typename TX, bool BF16, int G, int NP, int TT>
+__global__ __launch_bounds__(NT) void router_mf_kernel(RouterArgs a) {
+  constexpr int EP = 16 * G * NP, LGS = EP + 1;
+  constexpr int CPR = 4 / G;  // chunks per round
+  constexpr bool SPLIT = TT == 16;
+  __shared__ float lg[TT * LGS];
+  __shared__ TileScratch<EP> sc;
+  __shared__ float part[SPLIT ? 2 * 4 * 16 * 64 : 1];  // [buffer][wave][register][lane]
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = blockIdx.x * TT;
+  const int nch = (a.D + 63) / 64, nr = (nch + CPR - 1) / CPR;
+  const int lc = (lane >> 4) / G;  // this lane's chunk of a round
+  for (int pass = 0; pass < NP; ++pass) {
+    const LgSrc<TX> S = lg_source<TX, G>(
+        static_cast<const TX*>(a.x), a.ldx,
+        static_cast<const TX*>(a.wr_t) + (size_t)pass * a.ldw * 64, a.ldw, a.N, a.Dx,
+        n0 + (SPLIT ? 0 : 16 * wave), lane);
+    auto d_of = [&](int r, int half) { return ((r * CPR + lc) * 2 + half) * 32; };
+    LgHalf<TX> ra, rb;
+    mxm_lg16 acc;
+    if constexpr (SPLIT) {
+      float lgt[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) lgt[g] = 0.0f;
+      lg_load<TX>(ra, S, d_of(wave, 0));
+      for (int r0 = 0, buf = 0; r0 < nr; r0 += 4, buf ^= 1) {
+        const int r = r0 + wave;
+        float* pb = part + buf * (4 * 16 * 64);
+        if (r < nr) {
+          lg_load<TX>(rb, S, d_of(r, 1));
+          __builtin_amdgcn_sched_barrier(0);
+          lg_half<TX, true>(ra, acc);
+          __builtin_amdgcn_sched_barrier(0);
+          lg_load<TX>(ra, S, d_of(r + 4, 0));  // (past the end: zeros, unused)
+          __builtin_amdgcn_sched_barrier(0);
+          lg_half<TX, false>(rb, acc);
+#pragma unroll
+          for (int i = 0; i < 16; ++i) pb[(wave * 16 + i) * 64 + lane] = acc[i];
+        }
+        __syncthreads();
+        // (the buffer is written again two rounds on, after the next barrier)
+        for (int w = 0; w < 4 && r0 + w < nr; ++w)
+#pragma unroll
+          for (int cc = 0; cc < CPR; ++cc)
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+              lgt[g] = lgt[g] + pb[(w * 16 + 4 * (cc * G + g) + wave) * 64 + lane];
+      }
+      const int t = (lane >> 4) * 4 + wave;
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        lg[t * LGS + (pass * G + g) * 16 + (lane & 15)] = BF16 ? mxm_rbf(lgt[g]) : lgt[g];
+      if (pass + 1 < NP) __syncthreads();  // the partials' buffers are free
+    } else {
+      float lgt[4 * G];
+#pragma unroll
+      for (int i = 0; i < 4 * G; ++i) lgt[i] = 0.0f;
+      lg_load<TX>(ra, S, d_of(0, 0));
+      // (the scheduling barriers keep each half's loads issued before the
+      // other half's products instead of next to their own uses)
+      for (int r = 0; r < nr; ++r) {
+        lg_load<TX>(rb, S, d_of(r, 1));
+        __builtin_amdgcn_sched_barrier(0);
+        lg_half<TX, true>(ra, acc);
+        __builtin_amdgcn_sched_barrier(0);
+        lg_load<TX>(ra, S, d_of(r + 1, 0));  // (past the end: zeros, unused)
+        __builtin_amdgcn_sched_barrier(0);
+        lg_half<TX, false>(rb, acc);
+        // chunks past the last are +0 partials, which change no logit (a sum
+        // from +0, never -0)
+#pragma unroll
+        for (int cc = 0; cc < CPR; ++cc)
+#pragma unroll
+          for (int i = 0; i < 4 * G; ++i) lgt[i] = lgt[i] + acc[4 * G * cc + i];
+      }
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int t = 16 * wave + (lane >> 4) * 4 + q;
+          const float v = lgt[4 * g + q];
+          lg[t * LGS + (pass * G + g) * 16 + (lane & 15)] = BF16 ? mxm_rbf(v) : v;
+        }
+    }
+  }
+  route_tile<BF16, EP, TT, LGS>(lg, sc, n0, blockIdx.x, a);
+}
+
+// The same on the vector unit, for rows that are not whole 16-byte pieces:
+// 64 tokens per workgroup, each thread 4 tokens x EPT experts over 64-d
+// chunks staged in LDS, then the tiles of TT tokens one after the other.
+template <typename TX, bool BF16, int EPT, int TT>
+__global__ __launch_bounds__(NT) void router_kernel(RouterArgs a) {
+  constexpr int EP = 16 * EPT;
+  constexpr int LGS = EP + 1;
+  constexpr int STAGE_FLOATS = BK * TM + BK * EP;
+  constexpr int LG_FLOATS = TM * LGS;
+  constexpr int SMEM_FLOATS = STAGE_FLOATS > LG_FLOATS ? STAGE_FLOATS : LG_FLOATS;
+  __shared__ __attribute__((aligned(16))) float smem[SMEM_FLOATS];
+  __shared__ TileScratch<EP> sc;
+  const TX* __restrict__ x = static_cast<const TX*>(a.x);
+  const TX* __restrict__ wr = static_cast<const TX*>(a.wr);
+  const int N = a.N, D = a.D, E = a.E;
+
+  float* xs = smem;            // [BK][TM]
+  float* ws = smem + BK * TM;  // [BK][EP]
+  float* lg = smem;            // [TM][LGS] after the products
+  const int tid = threadIdx.x;
+  const int n0 = blockIdx.x * TM;
+  const int ty = tid >> 4;  // tokens ty*4 .. ty*4+3
+  const int tx = tid & 15;  // experts tx*EPT .. tx*EPT+EPT-1
+  float acc[4][EPT];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < EPT; ++j) acc[i][j] = 0.0f;
+
+  // products of one BK chunk held in LDS (BK is the logits' 64-d summation
+  // chunk): a partial from +0, then added to the logit
+  static_assert(BK == MXM_LOGIT_CHUNK, "one LDS chunk per summation chunk");
+  for (int d0 = 0; d0 < D; d0 += BK) {
+    __syncthreads();
+    for (int i = tid; i < TM * BK; i += NT) {
+      const int t = i % TM, dd = i / TM;
+      const int n = n0 + t, d = d0 + dd;
+      xs[dd * TM + t] = (n < N && d < D) ? ld_as_f32<TX>(x + (size_t)n * a.ldx + d) : 0.0f;
+    }
+    for (int i = tid; i < BK * EP; i += NT) {
+      const int dd = i / EP, e = i % EP;
+      const int d = d0 + dd;
+      ws[i] = (d < D && e < E) ? ld_as_f32<TX>(wr + (size_t)d * E + e) : 0.0f;
+    }
+    __syncthreads();
+    float part[4][EPT];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < EPT; ++j) part[i][j] = 0.0f;
+#pragma unroll 4
+    for (int dd = 0; dd < BK; ++dd) {
+      const float4 xv = *reinterpret_cast<const float4*>(&xs[dd * TM + ty * 4]);
+      float wv[EPT];
+#pragma unroll
+      for (int j = 0; j < EPT; ++j) wv[j] = ws[dd * EP + tx * EPT + j];
+#pragma unroll
+      for (int j = 0; j < EPT; ++j) {
+        part[0][j] = __builtin_fmaf(xv.x, wv[j], part[0][j]);
+        part[1][j] = __builtin_fmaf(xv.y, wv[j], part[1][j]);
+        part[2][j] = __builtin_fmaf(xv.z, wv[j], part[2][j]);
+        part[3][j] = __builtin_fmaf(xv.w, wv[j], part[3][j]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < EPT; ++j) acc[i][j] = acc[i][j] + part[i][j];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < EPT; ++j) {
+      const float v = acc[i][j];
+      lg[(ty * 4 + i) * LGS + tx * EPT + j] = BF16 ? mxm_rbf(v) : v;
+    }
+  for (int sub = 0; sub < TM / TT && n0 + sub * TT < N; ++sub)
+    route_tile<BF16, EP, TT, LGS>(lg + sub * TT * LGS, sc, n0 + sub * TT,
+                                  blockIdx.x * (TM / TT) + sub, a);
 }
 
 // Decode-sized batches: routing in one launch.  Workgroup n owns token n.
@@ -1112,45 +1090,38 @@ void launch_route_small_dt(const RouteSmallArgs& a, hipStream_t s) {
     launch_route_small_t<TX, BF16, 4>(a, s);
 }
 
-template <typename TX, bool BF16, int EPT>
-void launch_router_t(const RouterArgs& a, hipStream_t s) {
-  const int ntiles = (a.N + TM - 1) / TM;
+template <typename TX, bool BF16, int TT>
+void launch_router_tt(const RouterArgs& a, hipStream_t s) {
   constexpr int PER = 16 / (int)sizeof(TX);
-  const bool xvec = a.D % PER == 0 && (reinterpret_cast<uintptr_t>(a.x) % 16) == 0;
-  const bool vec = xvec && a.E % PER == 0 && (reinterpret_cast<uintptr_t>(a.wr) % 16) == 0;
-  const TX* x = static_cast<const TX*>(a.x);
-  const TX* wr = static_cast<const TX*>(a.wr);
-  const TX* wr_t = static_cast<const TX*>(a.wr_t);
-  if constexpr (EPT >= 4) {
-    if (wr_t && xvec && a.E > 32 && a.D <= (1 << 24)) {
-      hipLaunchKernelGGL((router_kernel<TX, BF16, EPT, true, true>), dim3(ntiles), dim3(NT), 0, s,
-                         x, wr, a.N, a.D, a.E, a.K, a.top_idx, a.gates, a.slot_rank,
-                         a.tile_counts, a.tile_psum, a.tile_ent, a.probs_out, ntiles, wr_t, a.ldw);
-      return;
-    }
-  }
-  if (vec)
-    hipLaunchKernelGGL((router_kernel<TX, BF16, EPT, true>), dim3(ntiles), dim3(NT), 0, s, x, wr,
-                       a.N, a.D, a.E, a.K, a.top_idx, a.gates, a.slot_rank, a.tile_counts,
-                       a.tile_psum, a.tile_ent, a.probs_out, ntiles, nullptr, 0);
-  else
-    hipLaunchKernelGGL((router_kernel<TX, BF16, EPT, false>), dim3(ntiles), dim3(NT), 0, s, x, wr,
-                       a.N, a.D, a.E, a.K, a.top_idx, a.gates, a.slot_rank, a.tile_counts,
-                       a.tile_psum, a.tile_ent, a.probs_out, ntiles, nullptr, 0);
+  // whole 16-byte pieces, and 32-bit byte offsets into 16 rows of x and a
+  // group of the router copy
+  const bool mf = a.wr_t && a.Dx % PER == 0 && a.ldx % PER == 0 &&
+                  reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && a.ldx <= (1 << 22) &&
+                  a.ldw <= (1 << 22);
+  const dim3 grid((a.N + TT - 1) / TT), grid64((a.N + TM - 1) / TM);
+  auto go = [&](auto g, auto np) {
+    constexpr int G = decltype(g)::value, NP = decltype(np)::value;
+    if (mf)
+      hipLaunchKernelGGL((router_mf_kernel<TX, BF16, G, NP, TT>), grid, dim3(NT), 0, s, a);
+    else
+      hipLaunchKernelGGL((router_kernel<TX, BF16, G * NP, TT>), grid64, dim3(NT), 0, s, a);
+  };
+  using std::integral_constant;
+  const integral_constant<int, 1> one{};
+  const integral_constant<int, 4> four{};
+  if (a.E <= 16) go(one, one);
+  else if (a.E <= 32) go(integral_constant<int, 2>{}, one);
+  else if (a.E <= 64) go(four, one);
+  else if (a.E <= 128) go(four, integral_constant<int, 2>{});
+  else go(four, four);
 }
 
 template <typename TX, bool BF16>
 void launch_router_dt(const RouterArgs& a, hipStream_t s) {
-  if (a.E <= 16)
-    launch_router_t<TX, BF16, 1>(a, s);
-  else if (a.E <= 32)
-    launch_router_t<TX, BF16, 2>(a, s);
-  else if (a.E <= 64)
-    launch_router_t<TX, BF16, 4>(a, s);
-  else if (a.E <= 128)
-    launch_router_t<TX, BF16, 8>(a, s);
+  if (a.tile_tokens == 16)
+    launch_router_tt<TX, BF16, 16>(a, s);
   else
-    launch_router_t<TX, BF16, 16>(a, s);
+    launch_router_tt<TX, BF16, 64>(a, s);
 }
 
 }  // namespace
