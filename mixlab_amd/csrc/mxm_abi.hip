@@ -436,7 +436,7 @@ void alloc_workspace(MoeOp& o) {
 // Refuse to launch a GEMM whose operands are not all allocated (a kernel
 // would otherwise read through a null pointer).
 void require_operands(const GemmArgs& g, bool second_matrix, bool scaled) {
-  if (!g.a || !g.b0 || !g.out || !g.offsets || (second_matrix && !g.b1) ||
+  if (!g.a || !g.b0 || (!g.out && !g.out2) || !g.offsets || (second_matrix && !g.b1) ||
       (scaled && (!g.scale0 || (g.mode == MXM_GEMM_GLU && !g.scale1))) ||
       (g.mode != MXM_GEMM_DOWN && !g.perm))
     fail_rt("OP_MOE_FEED_FORWARD internal error: expert GEMM operand not allocated (mode %d)", g.mode);
@@ -455,7 +455,7 @@ struct BlockIO {
 
 // pre_out (MFMA family only): also keep the up projections' pre-activation
 // products [N*K, NC] bf16 there (the backward's activation gradient reads
-// them); H is then derived from them with the same activation code.
+// them).
 // w is the workspace the forward writes (the op's own, or the device
 // scratch of the no-allocation entry point); with events = false no
 // profiling events are recorded (they are created on demand).
@@ -661,16 +661,14 @@ void run_forward(MoeOp& o, const Workspace& w, const void* x, int x_dtype, float
     require_operands(g1, glu, o.q8);
     for (int rep = 0; rep < reps; ++rep) mxm_launch_gemm_q8(g1, st);
   } else if (o.mfma) {
-    g1.out2 = pre_out;  // the backward keeps the raw projections (and no hidden)
+    g1.out2 = pre_out;  // the backward keeps the raw projections
+    if (o.up_only) g1.out = nullptr;  // ... and its own forward no hidden
     if (o.q8_mfma) {
       g1.scale0 = o.s1.as<float>();
       g1.scale1 = glu ? o.s1b.as<float>() : nullptr;
     }
     require_operands(g1, false, o.q8_mfma);
     for (int rep = 0; rep < reps; ++rep) mxm_launch_gemm_mfma(g1, st);
-    if (pre_out && !o.up_only)  // a kept forward: the hidden from them, as the epilogue would
-      mxm_launch_hidden_from_raw_bf16(pre_out, o.N * o.K, o.Fk, o.etype, o.act, o.slope, o.hsplit,
-                                      static_cast<uint16_t*>(w.H), st);
   } else {
     require_operands(g1, glu, false);
     for (int rep = 0; rep < reps; ++rep) mxm_launch_gemm_simt(g1, o.bf16, st);

@@ -468,8 +468,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
   constexpr int WROWS = TM * 32;
   constexpr int C = (MODE == MXM_GEMM_GLU) ? TN * 16 : TN * 32;  // output columns per wave
   static_assert(C == 32 || C == 64, "staging swizzle covers 32 or 64 columns per wave");
-  static_assert(NW * WROWS * C * 2 <= (int)sizeof(u32x4_t) * NS * BUF, "staging fits in LDS");
-  uint32_t* stage = reinterpret_cast<uint32_t*>(lds) + (size_t)wave * (WROWS / 2) * C;
+  // words of staging per row pair and wave: the widest of the tile's stores
+  constexpr int CS = Epi<EPI>::KEEP_RAW && TN * 32 > C ? TN * 32 : C;
+  static_assert(NW * WROWS * CS * 2 <= (int)sizeof(u32x4_t) * NS * BUF, "staging fits in LDS");
+  uint32_t* stage = reinterpret_cast<uint32_t*>(lds) + (size_t)wave * (WROWS / 2) * CS;
   auto word_at = [](int kp, int c) -> int {
     const int b1 = (kp >> 1) & 1;
     if constexpr (C == 64) {
@@ -486,9 +488,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
     // as W1's rows) to out2, through the same staging with 64 columns per
     // wave, before the activation overwrites the accumulators
     constexpr int CR = TN * 32;
-    static_assert(CR == 64 && NW * WROWS * CR * 2 <= (int)sizeof(u32x4_t) * NS * BUF,
-                  "raw staging fits in LDS");
-    uint32_t* rst = reinterpret_cast<uint32_t*>(lds) + (size_t)wave * (WROWS / 2) * CR;
+    static_assert(CR == 64 && CR == CS, "raw staging of 64 columns per wave");
+    uint32_t* rst = stage;
     auto rword = [](int kp, int c) -> int {
       const int b1 = (kp >> 1) & 1;
       const int ch = (c >> 2) ^ (kp & 1) ^ (b1 << 3);
@@ -528,7 +529,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
       if (grow + 1 < rows)
         *reinterpret_cast<u32x4_t*>(rout + (size_t)(row0 + grow + 1) * a.Ncols + c0r) = hi;
     }
-    return;  // no hidden: the backward's activation pass derives it
+    if constexpr (Epi<EPI>::RAW_ONLY) return;  // the backward's activation pass derives H
+    // this wave's reads of the raw staging are complete
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
   }
   // kinds whose hidden is fp32 store it as two bf16 planes (hi, then lo =
   // bf16(h - hi)) through the same staging, one plane after the other
@@ -879,7 +883,9 @@ template <class F>
 void with_epi(const GemmArgs& a, F&& f) {
   auto up = [&](auto kind) {
     constexpr int K = decltype(kind)::value;
-    if (a.out2)
+    if (a.out2 && a.out)
+      f(std::integral_constant<int, EPI_KEEP_H + K>{});
+    else if (a.out2)
       f(std::integral_constant<int, EPI_KEEP + K>{});
     else if (a.scale0)
       f(std::integral_constant<int, EPI_SCALE + K>{});

@@ -174,8 +174,9 @@ struct GemmArgs {
   const float* scale0;    // int8 weights: per-output-channel scales
   const float* scale1;
   void* out;              // mode 0/1: H [N*K, F]; mode 2: Y [N*K, D]
-  void* out2;             // MFMA up projections: if set, the raw bf16 projections too,
-                          // [N*K, Ncols] in W1's column order (the backward's G|U);
+  void* out2;             // MFMA up projections: if set, the raw bf16 projections,
+                          // [N*K, Ncols] in W1's column order (the backward's G|U), and
+                          // the hidden only where out is set too;
                           // SIMT MLP up projection: the raw fp32 projections, rows
                           // ld2 apart (out may then be null: no hidden stored)
   int ld2;
@@ -291,8 +292,9 @@ enum { EPI_SWIGLU, EPI_GEGLU, EPI_MLP_SILU, EPI_MLP_GELU, EPI_MLP_RELU, EPI_MLP_
 
 // EPI_KEEP + an up-projection kind: the raw bf16 projections to
 // GemmArgs::out2 instead of the hidden (the MFMA backward derives H from
-// them in its activation pass).
+// them in its activation pass); EPI_KEEP_H + a kind: both.
 constexpr int EPI_KEEP = 16;
+constexpr int EPI_KEEP_H = 64;
 // EPI_SCALE + a kind: the accumulators are multiplied by a per-output-column
 // fp32 scale (GemmArgs::scale0, and scale1 for the up matrix of a GLU pair,
 // each [E][output columns]) before anything else; the int8 weights' flow on
@@ -302,7 +304,8 @@ constexpr int EPI_SCALE = 32;
 template <int EPI_>
 struct Epi {
   static constexpr int EPI = EPI_ & (EPI_KEEP - 1);
-  static constexpr bool KEEP_RAW = (EPI_ & EPI_KEEP) != 0;
+  static constexpr bool KEEP_RAW = (EPI_ & (EPI_KEEP | EPI_KEEP_H)) != 0;
+  static constexpr bool RAW_ONLY = (EPI_ & EPI_KEEP) != 0;
   static constexpr bool SCALED = (EPI_ & EPI_SCALE) != 0;
   static constexpr int MODE = EPI <= EPI_GEGLU ? MXM_GEMM_GLU
                               : (EPI == EPI_DOWN || EPI == EPI_DOWN_F32 || EPI == EPI_F32)
@@ -498,12 +501,7 @@ void mxm_launch_dwr_halves(const float* t, int D, int E, int Ep, float* dwr, hip
 // gp[p] = gates[s] and (if dyb is set) dyb[p] = bf16(gates[s] * dD[n]).
 void mxm_launch_dy_gate(const float* dd, const float* gates, const int32_t* slot_pos, int N, int D,
                         int K, uint16_t* ddb, uint16_t* dyb, float* gp, hipStream_t s);
-// The hidden H [rows][F] (hi, and lo = bf16(h - hi) after F columns when
-// hsplit) from raw bf16 up projections gu [rows][NC] with the up epilogue's
-// own activation code: bit for bit what the epilogue would store.
-void mxm_launch_hidden_from_raw_bf16(const uint16_t* gu, int rows, int F, int etype, int act,
-                                     float slope, bool hsplit, uint16_t* H, hipStream_t s);
-// ... then, per routed row p: the hidden h from the forward's raw bf16
+// Per routed row p: the hidden h from the forward's raw bf16
 // projections gu with the up epilogue's own activation code (bit for bit the
 // forward's); the gated hidden gp[p] * h written to Hg (hi, and lo =
 // bf16(v - hi) after F columns when hsplit) for dW_down = Hg^T dD over the
