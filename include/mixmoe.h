@@ -60,9 +60,10 @@ extern "C" {
 #define MXM_FLAG_MFMA_TILE_MASK 12
 #define MXM_FLAG_INT8_WEIGHTS 16 /* expert weights are int8 + per-output-channel scales
                                     (mxm_moe_set_input_q8); bf16 compute */
-/* Each mxm_moe_forward keeps the op's own copy of x and, under bf16 compute
- * on the MFMA family, its routing, router probabilities and raw up
- * projections, for mxm_moe_backward_kept: the backward of that forward,
+/* Each mxm_moe_forward keeps the op's own copy of x, its routing and router
+ * probabilities and, where the backward runs in bf16 (bf16 compute on the
+ * MFMA family, D a multiple of 128), its raw up projections, for
+ * mxm_moe_backward_kept: the backward of that forward,
  * which then does not run the forward again, as the reference's autodiff
  * keeps the forward's values for its backward.  No counterpart flag in the
  * reference (its graph keeps them implicitly). */

@@ -238,8 +238,7 @@ struct MoeOp {
   // the fp32 backward's products (run_backward_x3): bf16 planes of the
   // operands at the padded widths Dq x Fq, fp32 products
   bool bx_w_ready = false;
-  int bx_Dq = 0, bx_Fq = 0;
-  DevBuf bx_w1p, bx_w1t, bx_w2p, bx_w2t, bx_x3, bx_gu, bx_h3, bx_y, bx_dy3, bx_dh, bx_dgu3, bx_dxe;
+  DevBuf bx_w1p, bx_w1t, bx_w2p, bx_w2t, bx_x, bx_gu, bx_h, bx_y, bx_dy, bx_dh, bx_dgu, bx_dxe;
   int32_t bw_one_host[4] = {0, 0, 0, 0};
 
   // profiling: one set of MXM_NUM_STAGES+1 events per profiled forward
@@ -916,7 +915,7 @@ std::mutex g_scratch_mu;
 char* g_scratch[kMaxDevices] = {};
 
 // This device's scratch address.  The first call on a device looks it up and
-// clears the ticket (the first 256 bytes of every workspace layout; the
+// clears the tickets (the first 256 bytes of every workspace layout; the
 // kernels leave them zero after each call) with a fill kernel, then waits for
 // the device, so it must not run under stream capture: mxm_init does it
 // before any capture.
@@ -1266,22 +1265,21 @@ int mxm_moe_forward(int64_t h, const void* x, int x_dtype, int64_t rows, float* 
       op->kept = false;
       HIPCK(hipMemcpyAsync(op->kept_xbuf.p, x, xbytes, hipMemcpyDeviceToDevice, op->stream));
       const void* xk = op->kept_xbuf.p;
-      if (mfma_backward_fits(*op)) {
-        // keep what the backward's own forward would recompute
-        op->keep_probs = true;
-        try {
-          run_forward(*op, op->ws, xk, x_dtype, delta, aux, entropy, nullptr, bw_gu_buffer(*op));
-        } catch (...) {
-          op->keep_probs = false;
-          throw;
-        }
+      // keep what the backward's own forward would recompute: the routing, the
+      // probabilities and (MFMA backward) the raw projections
+      uint16_t* raw = mfma_backward_fits(*op) ? bw_gu_buffer(*op) : nullptr;
+      if (!op->bw_probs.p) op->bw_probs.alloc((size_t)op->N * op->E * 4);
+      op->keep_probs = true;
+      try {
+        run_forward(*op, op->ws, xk, x_dtype, delta, aux, entropy, nullptr, raw);
+      } catch (...) {
         op->keep_probs = false;
-        if (op->debug_probs)  // (mxm_moe_probs reads the workspace's copy)
-          HIPCK(hipMemcpyAsync(op->ws.probs, op->bw_probs.p, (size_t)op->N * op->E * 4,
-                               hipMemcpyDeviceToDevice, op->stream));
-      } else {
-        run_forward(*op, op->ws, xk, x_dtype, delta, aux, entropy);
+        throw;
       }
+      op->keep_probs = false;
+      if (op->debug_probs)  // (mxm_moe_probs reads the workspace's copy)
+        HIPCK(hipMemcpyAsync(op->ws.probs, op->bw_probs.p, (size_t)op->N * op->E * 4,
+                             hipMemcpyDeviceToDevice, op->stream));
       op->kept = true;
       op->kept_dtype = x_dtype;
     } else {
@@ -1616,6 +1614,7 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
   wa.lda = o.hsplit ? 2 * Fk : Fk;
   wa.aplane = Fk;
   wa.planes = o.hsplit ? 2 : 1;
+  wa.amap = 2;  // both planes of A against B's one
   wa.b = ddb;
   wa.b_rows = b.perm;
   wa.b_rows32 = !o.force64 && (size_t)o.N * D * 2 < ((size_t)1 << 32);
@@ -1631,15 +1630,26 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
   HIPCK(hipGetLastError());
 }
 
+// The padded widths of the fp32 backward's operands (multiples of 128).
+struct X3Widths {
+  int Dq, Fq, NCq;
+  explicit X3Widths(const MoeOp& o)
+      : Dq((o.D + 127) / 128 * 128), Fq((o.F + 127) / 128 * 128),
+        NCq(o.wpe == 3 ? 2 * Fq : Fq) {}
+};
+
 // The fp32 backward after the routing (fp32 compute, or the bf16 flow on
 // fp32 copies where the MFMA backward does not apply).  Every product of the
-// experts runs on the library's bf16 MFMA kernels as the product of the
-// operands' bf16 planes (hi = bf16(v), lo = bf16(v - hi), concatenated along
-// k so that one product sums hi.hi + hi.lo + lo.hi; mxm_launch_planes3):
-// about 2^-16 relative per term, accumulated in fp32.  Operands are padded
-// with zeros to Dq x Fq (multiples of 128); rows are in the forward's
-// permuted order and every grouped product takes its experts' row ranges
-// from the device-side offsets, so nothing waits for the host.
+// experts runs on the library's bf16 MFMA kernels as the sum over pairs of
+// the operands' bf16 planes (hi = bf16(v), lo = bf16(v - hi)): hi.hi + hi.lo
+// + lo.hi, about 2^-16 relative per term, accumulated in fp32.  Under bf16
+// compute x and the weights are bf16 values, their lo planes zero: those
+// operands are one plane, and the pairs that it would have made are left out
+// (one, two and two pairs for G|U, dH and dX, and dW1 instead of three each;
+// the same sums, without adding zeros).  Operands are padded with zeros to Dq
+// x Fq (multiples of 128); rows are in the forward's permuted order and every
+// grouped product takes its experts' row ranges from the device-side offsets,
+// so nothing waits for the host.
 //   G|U = Xp W1                 grouped product, A = x's planes through perm
 //   H = act(G, U)               planes of H
 //   Y = H W_down                (own_forward: fp32 compute; else the op's
@@ -1649,29 +1659,29 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
 //   dH = dY W_down^T            grouped product on dY's planes
 //   dG, dU                      the activation backward, as planes
 //   dXe = dGU W1^T, dx = dxr + sum_k dXe
-//   dW1 = Xp^T dGU, dW_down = H^T dY   the weight-gradient kernel, three
-//                                plane pairs each, the gradients stored in
-//                                the op's [D][F] / [F][D] layout
+//   dW1 = Xp^T dGU, dW_down = H^T dY   the weight-gradient kernel, the
+//                                gradients stored in the op's [D][F] / [F][D]
+//                                layout
 void run_backward_x3(MoeOp& o, BackwardArgs& b, bool own_forward) {
   hipStream_t st = o.stream;
   const bool glu = o.wpe == 3;
   const int D = o.D, F = o.F, E = o.E;
-  const int Dq = (D + 127) / 128 * 128, Fq = (F + 127) / 128 * 128, NCq = glu ? 2 * Fq : Fq;
+  const X3Widths w(o);
+  const int Dq = w.Dq, Fq = w.Fq, NCq = w.NCq;
+  const int np = o.bf16 ? 1 : 2;  // planes of x and the weights
   const size_t N = o.N, NK = (size_t)o.N * o.K, DF = (size_t)D * F;
-  if (o.bx_Dq != Dq || o.bx_Fq != Fq || !o.bx_x3.p) {
-    o.bx_Dq = Dq;
-    o.bx_Fq = Fq;
-    o.bx_w1p.alloc((size_t)E * NCq * 3 * Dq * 2);
-    o.bx_w1t.alloc((size_t)E * Dq * 3 * NCq * 2);
-    o.bx_w2p.alloc((size_t)E * Dq * 3 * Fq * 2);
-    o.bx_w2t.alloc((size_t)E * Fq * 3 * Dq * 2);
-    o.bx_x3.alloc(N * 3 * Dq * 2);
+  if (!o.bx_x.p) {
+    o.bx_w1p.alloc((size_t)E * NCq * np * Dq * 2);
+    o.bx_w1t.alloc((size_t)E * Dq * np * NCq * 2);
+    if (own_forward) o.bx_w2p.alloc((size_t)E * Dq * np * Fq * 2);
+    if (own_forward && Dq != D) o.bx_y.alloc(NK * Dq * 4);
+    o.bx_w2t.alloc((size_t)E * Fq * np * Dq * 2);
+    o.bx_x.alloc(N * np * Dq * 2);
     o.bx_gu.alloc(NK * NCq * 4);
-    o.bx_h3.alloc(NK * 3 * Fq * 2);
-    if (Dq != D) o.bx_y.alloc(NK * Dq * 4);
-    o.bx_dy3.alloc(NK * 3 * Dq * 2);
+    o.bx_h.alloc(NK * 2 * Fq * 2);
+    o.bx_dy.alloc(NK * 2 * Dq * 2);
     o.bx_dh.alloc(NK * Fq * 4);
-    o.bx_dgu3.alloc(NK * 3 * NCq * 2);
+    o.bx_dgu.alloc(NK * 2 * NCq * 2);
     o.bx_dxe.alloc(NK * Dq * 4);
     if (!o.bw_zero.p) {
       o.bw_zero.alloc(512);  // 256 zero bf16: the weight gradients' rows past an expert's end
@@ -1681,23 +1691,30 @@ void run_backward_x3(MoeOp& o, BackwardArgs& b, bool own_forward) {
     o.bx_w_ready = false;
   }
   if (!o.bx_w_ready) {
-    mxm_launch_planes3_weights(b.w1, glu ? b.w1b : nullptr, b.w2, E, D, F, Dq, Fq, glu,
-                               o.bx_w1p.as<uint16_t>(), o.bx_w1t.as<uint16_t>(),
-                               o.bx_w2p.as<uint16_t>(), o.bx_w2t.as<uint16_t>(), st);
+    mxm_launch_planes_weights(b.w1, glu ? b.w1b : nullptr, b.w2, E, D, F, Dq, Fq, glu, np,
+                              o.bx_w1p.as<uint16_t>(), o.bx_w1t.as<uint16_t>(),
+                              o.bx_w2p.as<uint16_t>(), o.bx_w2t.as<uint16_t>(), st);
     HIPCK(hipGetLastError());
     o.bx_w_ready = true;
   }
-  uint16_t *x3 = o.bx_x3.as<uint16_t>(), *h3 = o.bx_h3.as<uint16_t>(),
-           *dy3 = o.bx_dy3.as<uint16_t>(), *dgu3 = o.bx_dgu3.as<uint16_t>();
+  uint16_t *xp = o.bx_x.as<uint16_t>(), *hp = o.bx_h.as<uint16_t>(), *dyp = o.bx_dy.as<uint16_t>(),
+           *dgup = o.bx_dgu.as<uint16_t>();
   float *gu = o.bx_gu.as<float>(), *dh = o.bx_dh.as<float>(), *dxe = o.bx_dxe.as<float>();
-  // grouped product out [NK][Ncols] fp32 = A [NK][Kd] (rows through perm when
-  // gather) . B_e^T (B_e [Ncols][Kd] per expert)
-  auto product = [&](const uint16_t* A, const uint16_t* W, float* out, int Kd, int Ncols,
-                     bool gather) {
-    if (mxm_mfma_tile_rows(Ncols, Kd, MXM_TILE_AUTO) <= 0)
-      fail("OP_MOE_FEED_FORWARD backward: a %d x %d expert product exceeds the MFMA tiles' "
-           "addressing", Ncols, Kd);
+  // grouped product out [NK][Ncols] fp32 = A . B_e^T over the plane pairs: A
+  // rows (through perm when gather) of na planes, B_e [Ncols] rows of nb
+  auto product = [&](const uint16_t* A, int na, const uint16_t* W, int nb, float* out, int Kp,
+                     int Ncols, bool gather) {
     GemmArgs g{};
+    g.planes = na == 2 && nb == 2 ? 3 : na * nb;
+    // pairs (hi, hi), (hi, lo), (lo, hi) for X and H, (hi, hi), (lo, hi),
+    // (hi, lo) for the gradients, without those of a missing lo plane
+    g.amap = na == 2 ? (nb == 1 || A == dyp || A == dgup ? 2 : 4) : 0;
+    g.bmap = nb == 2 ? (na == 1 ? 2 : g.amap == 2 ? 4 : 2) : 0;
+    g.lda = na * Kp;
+    g.ldb = nb * Kp;
+    if (mxm_mfma_tile_rows(Ncols, g.planes * Kp, MXM_TILE_AUTO) <= 0)
+      fail("OP_MOE_FEED_FORWARD backward: a %d x %d expert product exceeds the MFMA tiles' "
+           "addressing", Ncols, g.planes * Kp);
     g.no_off32 = o.force64;
     g.mode = MXM_GEMM_DOWN;
     g.f32_out = true;
@@ -1706,7 +1723,7 @@ void run_backward_x3(MoeOp& o, BackwardArgs& b, bool own_forward) {
     g.out = out;
     g.offsets = b.offsets;
     g.E = E;
-    g.Kd = Kd;
+    g.Kd = g.planes * Kp;
     g.Ncols = Ncols;
     g.family = MXM_TILE_AUTO;
     g.gather_a = gather;
@@ -1717,7 +1734,7 @@ void run_backward_x3(MoeOp& o, BackwardArgs& b, bool own_forward) {
     HIPCK(hipGetLastError());
   };
   // x's planes (one row per token; the products gather them through perm)
-  mxm_launch_planes3(b.x, (int64_t)N, D, D, Dq, false, x3, st);
+  mxm_launch_planes(b.x, (int64_t)N, D, D, Dq, np, xp, st);
   // G|U = Xp W1 (fp32, W1's interleaved column order), H's planes.  An fp32
   // ReLU expert takes U from the exact-order SIMT projection instead -- the
   // forward's own fp32 sums: ReLU's derivative jumps at 0, and the plane
@@ -1750,43 +1767,46 @@ void run_backward_x3(MoeOp& o, BackwardArgs& b, bool own_forward) {
     mxm_launch_gemm_simt(g, false, st);
     HIPCK(hipGetLastError());
   } else {
-    product(x3, o.bx_w1p.as<uint16_t>(), gu, 3 * Dq, NCq, true);
+    product(xp, np, o.bx_w1p.as<uint16_t>(), np, gu, Dq, NCq, true);
   }
-  mxm_launch_hidden_planes3(gu, (int64_t)NK, Fq, o.etype, o.act, o.slope, h3, st);
+  mxm_launch_hidden_planes(gu, (int64_t)NK, Fq, o.etype, o.act, o.slope, hp, st);
   HIPCK(hipGetLastError());
   if (own_forward) {
     // the expert outputs Y = H W_down, which the gate gradients read
     float* y = static_cast<float*>(o.ws.Y);
-    product(h3, o.bx_w2p.as<uint16_t>(), Dq == D ? y : o.bx_y.as<float>(), 3 * Fq, Dq, false);
+    product(hp, 2, o.bx_w2p.as<uint16_t>(), np, Dq == D ? y : o.bx_y.as<float>(), Fq, Dq, false);
     if (Dq != D) mxm_launch_rows_to_f32(o.bx_y.p, MXM_DTYPE_F32, (int64_t)NK, D, Dq, y, st);
     HIPCK(hipGetLastError());
   }
   mxm_launch_backward_router(b, st);
   HIPCK(hipGetLastError());
   // dH = dY W_down^T, the activation backward, dXe = dGU W1^T, dx
-  mxm_launch_planes3(b.dy, (int64_t)NK, D, D, Dq, true, dy3, st);
-  product(dy3, o.bx_w2t.as<uint16_t>(), dh, 3 * Dq, Fq, false);
-  mxm_launch_act_bw_planes3(gu, dh, (int64_t)NK, Fq, o.etype, o.act, o.slope, dgu3, st);
+  mxm_launch_planes(b.dy, (int64_t)NK, D, D, Dq, 2, dyp, st);
+  product(dyp, 2, o.bx_w2t.as<uint16_t>(), np, dh, Dq, Fq, false);
+  mxm_launch_act_bw_planes(gu, dh, (int64_t)NK, Fq, o.etype, o.act, o.slope, dgup, st);
   HIPCK(hipGetLastError());
-  product(dgu3, o.bx_w1t.as<uint16_t>(), dxe, 3 * NCq, Dq, false);
+  product(dgup, 2, o.bx_w1t.as<uint16_t>(), np, dxe, NCq, Dq, false);
   mxm_launch_dx_sum(b.dxr, dxe, Dq, b.slot_pos, o.N, D, o.K, b.dx, st);
   HIPCK(hipGetLastError());
   // weight gradients: dW1 = Xp^T dGU over the plane pairs (x hi, dGU hi),
-  // (x hi, dGU lo), (x lo, dGU hi); dW_down = H^T dY likewise
+  // (x hi, dGU lo) and, with a lo plane of x, (x lo, dGU hi); dW_down = H^T dY
+  // over all three
   WgradArgs wa{};
   wa.offsets = b.offsets;
   wa.zero = o.bw_zero.as<uint16_t>();
   wa.scratch = o.bw_wscr.p;
   wa.E = E;
   wa.out_estride = (size_t)o.wpe * DF;
-  wa.planes = 3;
-  wa.a = x3;
+  wa.planes = np == 2 ? 3 : 2;
+  wa.amap = np == 2 ? 4 : 0;
+  wa.bmap = 2;
+  wa.a = xp;
   wa.a_rows = b.perm;
-  wa.a_rows32 = !o.force64 && N * 3 * Dq * 2 < ((size_t)1 << 32);
-  wa.lda = 3 * Dq;
+  wa.a_rows32 = !o.force64 && N * np * Dq * 2 < ((size_t)1 << 32);
+  wa.lda = np * Dq;
   wa.aplane = Dq;
-  wa.b = dgu3;
-  wa.ldb = 3 * NCq;
+  wa.b = dgup;
+  wa.ldb = 2 * NCq;
   wa.bplane = NCq;
   wa.M = Dq;
   wa.m_store = Dq != D ? D : 0;
@@ -1797,13 +1817,15 @@ void run_backward_x3(MoeOp& o, BackwardArgs& b, bool own_forward) {
   wa.glu_f = glu ? F : 0;
   mxm_launch_wgrad(wa, st);
   HIPCK(hipGetLastError());
-  wa.a = h3;
+  wa.planes = 3;
+  wa.amap = 4;
+  wa.a = hp;
   wa.a_rows = nullptr;
   wa.a_rows32 = false;
-  wa.lda = 3 * Fq;
+  wa.lda = 2 * Fq;
   wa.aplane = Fq;
-  wa.b = dy3;
-  wa.ldb = 3 * Dq;
+  wa.b = dyp;
+  wa.ldb = 2 * Dq;
   wa.bplane = Dq;
   wa.M = Fq;
   wa.m_store = Fq != F ? F : 0;
@@ -1890,7 +1912,8 @@ void run_backward(MoeOp& o, const void* x, int x_dtype, const float* d_delta, fl
   uint16_t* gu = mfma_bw ? bw_gu_buffer(o) : nullptr;
   // the kept forward (MXM_FLAG_KEEP_FOR_BACKWARD) left the routing, the
   // probabilities and the raw projections where this forward puts them
-  const bool reuse = mfma_bw && allow_kept && o.kept;
+  // (and, where the fp32 backward follows a bf16 forward, its expert outputs)
+  const bool reuse = allow_kept && o.kept;
   // fp32 compute: the forward's routing only; the experts' forward products
   // are computed by run_backward_x3
   const bool own_forward = !o.bf16;

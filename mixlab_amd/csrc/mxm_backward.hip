@@ -805,41 +805,68 @@ int wgrad_router_chunks_impl(int N, int D, int E) {
 // ---- the fp32 backward's products on the bf16 MFMA kernels ----
 // An fp32 value v is carried as two bf16 planes, hi = bf16(v) and lo =
 // bf16(v - hi) (|v - hi - lo| <= 2^-18 |v|), and an fp32 product A . B as
-// the bf16 product of the k-concatenated planes [a0 | a1 | a2] . [b0 | b1 |
-// b2] with (a, b) = (hi, hi), (hi, lo), (lo, hi): A . B to within about
-// 3 * 2^-18 relative per term (the lo . lo term, below 2^-18, is dropped),
-// accumulated in fp32 by the MFMA.  Operands that pair with A-side planes
-// are laid out HHL = [hi | hi | lo], those on the B side HLH = [hi | lo | hi].
+// the sum of the bf16 products of the plane pairs (hi, hi), (hi, lo), (lo,
+// hi): A . B to within about 3 * 2^-18 relative per term (the lo . lo term,
+// below 2^-18, is dropped), accumulated in fp32 by the MFMA.  An operand of
+// bf16 values has no lo plane.  These kernels are streams of their operands:
+// 8 consecutive elements per thread, 16 or 32-byte loads and 16-byte stores
+// of each plane (one element per thread with 2-byte stores reached 3.7-4.4
+// TB/s of an 8192-row hidden or its backward, of 6 for a copy).
 
-__device__ __forceinline__ void split_bf16(float v, uint16_t& hi, uint16_t& lo) {
-  hi = mxm_f2bf(v);
-  lo = mxm_f2bf(v - mxm_bf2f(hi));
+__device__ __forceinline__ void split8(const float (&v)[8], uint4& hi, uint4& lo) {
+  uint32_t h[4], l[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    h[q] = mxm_pack_bf2_fast(v[2 * q], v[2 * q + 1]);
+    l[q] = mxm_pack_bf2_fast(v[2 * q] - mxm_u2f(h[q] << 16),
+                             v[2 * q + 1] - mxm_u2f(h[q] & 0xffff0000u));
+  }
+  hi = make_uint4(h[0], h[1], h[2], h[3]);
+  lo = make_uint4(l[0], l[1], l[2], l[3]);
 }
 
-// dst[r][p * ldq + c] = plane p (order hlh: HLH, else HHL) of src[r][c] for
-// c < cols, 0 for cols <= c < ldq.
-__global__ void planes3_kernel(const float* __restrict__ src, int64_t rows, int cols, int lds,
-                               int ldq, int hlh, uint16_t* __restrict__ dst) {
-  const int64_t n = rows * ldq;
+__device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
+  const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
+  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+  v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+
+// VEC: src and its rows are 16-byte aligned and cols is a multiple of 8.
+template <bool VEC>
+__global__ __launch_bounds__(256) void planes_kernel(const float* __restrict__ src, int64_t rows,
+                                                     int cols, int lds, int ldq, int np,
+                                                     uint16_t* __restrict__ dst) {
+  const int nb = ldq / 8;
+  const int64_t n = rows * nb;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = i / ldq;
-    const int c = (int)(i - r * ldq);
-    uint16_t hi = 0, lo = 0;
-    if (c < cols) split_bf16(src[(size_t)r * lds + c], hi, lo);
-    uint16_t* d = dst + (size_t)r * 3 * ldq + c;
-    d[0] = hi;
-    d[ldq] = hlh ? lo : hi;
-    d[2 * ldq] = hlh ? hi : lo;
+    const int64_t r = i / nb;
+    const int c = (int)(i - r * nb) * 8;
+    float v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = 0.0f;
+    const float* p = src + (size_t)r * lds + c;
+    if (VEC) {
+      if (c < cols) load8(p, v);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        if (c + q < cols) v[q] = p[q];
+    }
+    uint4 hi, lo;
+    split8(v, hi, lo);
+    uint16_t* d = dst + (size_t)r * np * ldq + c;
+    *reinterpret_cast<uint4*>(d) = hi;
+    if (np > 1) *reinterpret_cast<uint4*>(d + ldq) = lo;
   }
 }
 
 // One fp32 expert matrix of the x.W layout in the planes of an MFMA B
-// operand [R][3 Kq] bf16 per expert: dst[e][r][p * Kq + k] = plane p of the
+// operand [R][np Kq] bf16 per expert: dst[e][r][p * Kq + k] = plane p of the
 // source value at (r, k), 0 past the real extent.  For the up projections
 // (gate, up: src0, src1 [D][F]) or the down one (src0 [F][D]); the row or the
 // k index may be a GLU-interleaved column (groups of 32 gate then 32 up).
-struct Planes3W {
+struct PlanesW {
   const float* src0;
   const float* src1;    // the up matrix of a GLU pair (interleaved index), else null
   int E, R, Kq;         // rows and padded k per expert
@@ -847,11 +874,11 @@ struct Planes3W {
   int glu_r, glu_k;     // the row / k index is GLU-interleaved
   int64_t sr, sk;       // source strides of the decoded row and k indices
   int64_t es;           // source stride between experts
-  int hlh;
+  int np;
   uint16_t* dst;
 };
 
-__global__ void planes3_w_kernel(Planes3W a) {
+__global__ void planes_w_kernel(PlanesW a) {
   const int64_t per = (int64_t)a.R * a.Kq;
   const int64_t n = (int64_t)a.E * per;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
@@ -871,72 +898,98 @@ __global__ void planes3_w_kernel(Planes3W a) {
     uint16_t hi = 0, lo = 0;
     if (rr < a.r_lim && kk < a.k_lim) {
       const float* src = slot ? a.src1 : a.src0;
-      split_bf16(src[(size_t)e * a.es + (size_t)rr * a.sr + (size_t)kk * a.sk], hi, lo);
+      const float v = src[(size_t)e * a.es + (size_t)rr * a.sr + (size_t)kk * a.sk];
+      hi = mxm_f2bf(v);
+      lo = mxm_f2bf(v - mxm_bf2f(hi));
     }
-    uint16_t* d = a.dst + ((size_t)e * a.R + r) * 3 * a.Kq + k;
+    uint16_t* d = a.dst + ((size_t)e * a.R + r) * a.np * a.Kq + k;
     d[0] = hi;
-    d[a.Kq] = a.hlh ? lo : hi;
-    d[2 * (size_t)a.Kq] = a.hlh ? hi : lo;
+    if (a.np > 1) d[a.Kq] = lo;
   }
 }
 
-// The hidden units of the raw projections gu [rows][NC] fp32 (GLU: gate and
-// up interleaved in groups of 32; NC = 2 Fq, else Fq), as the HHL planes of
-// H [rows][3 Fq].
-__global__ void hidden_planes3_kernel(const float* __restrict__ gu, int64_t rows, int Fq, int etype,
-                                      int act, float slope, uint16_t* __restrict__ h3) {
+// 8 hidden units f .. f + 7 of row r of the raw projections gu [rows][NC] fp32
+// (GLU: gate and up interleaved in groups of 32; NC = 2 Fq, else Fq).
+__device__ __forceinline__ void load_gu8(const float* gu, int64_t r, int NC, int f, bool glu,
+                                         float (&g)[8], float (&u)[8]) {
+  const float* row = gu + (size_t)r * NC;
+  if (glu) {
+    const float* p = row + (f >> 5) * 64 + (f & 31);
+    load8(p, g);
+    load8(p + 32, u);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) g[q] = 0.0f;
+    load8(row + f, u);
+  }
+}
+
+// The hidden units of gu as the planes of H [rows][2 Fq].
+__global__ __launch_bounds__(256) void hidden_planes_kernel(const float* __restrict__ gu,
+                                                            int64_t rows, int Fq, int etype,
+                                                            int act, float slope,
+                                                            uint16_t* __restrict__ h) {
   const bool glu = etype != MXM_EXPERT_MLP;
-  const int NC = glu ? 2 * Fq : Fq;
-  const int64_t n = rows * Fq;
+  const int NC = glu ? 2 * Fq : Fq, nb = Fq / 8;
+  const int64_t n = rows * nb;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = i / Fq;
-    const int f = (int)(i - r * Fq);
-    const float* row = gu + (size_t)r * NC;
-    const int qg = (f >> 5) * 64 + (f & 31);
-    const float g = glu ? row[qg] : 0.0f, u = glu ? row[qg + 32] : row[f];
-    float h, cg, cu;
-    act_eval(etype, act, slope, g, u, h, cg, cu);
-    uint16_t hi, lo;
-    split_bf16(h, hi, lo);
-    uint16_t* d = h3 + (size_t)r * 3 * Fq + f;
-    d[0] = hi;
-    d[Fq] = hi;
-    d[2 * (size_t)Fq] = lo;
+    const int64_t r = i / nb;
+    const int f = (int)(i - r * nb) * 8;
+    float g[8], u[8], v[8];
+    load_gu8(gu, r, NC, f, glu, g, u);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      float cg, cu;
+      act_eval(etype, act, slope, g[q], u[q], v[q], cg, cu);
+    }
+    uint4 hi, lo;
+    split8(v, hi, lo);
+    uint16_t* d = h + (size_t)r * 2 * Fq + f;
+    *reinterpret_cast<uint4*>(d) = hi;
+    *reinterpret_cast<uint4*>(d + Fq) = lo;
   }
 }
 
 // The activation backward: from gu (as above) and dh [rows][Fq] fp32, dG and
-// dU as the HLH planes of dGU [rows][3 NC] in gu's column order.
-__global__ void act_bw_planes3_kernel(const float* __restrict__ gu, const float* __restrict__ dh,
-                                      int64_t rows, int Fq, int etype, int act, float slope,
-                                      uint16_t* __restrict__ dgu3) {
+// dU as the planes of dGU [rows][2 NC] in gu's column order.
+__global__ __launch_bounds__(256) void act_bw_planes_kernel(const float* __restrict__ gu,
+                                                            const float* __restrict__ dh,
+                                                            int64_t rows, int Fq, int etype,
+                                                            int act, float slope,
+                                                            uint16_t* __restrict__ dgu) {
   const bool glu = etype != MXM_EXPERT_MLP;
-  const int NC = glu ? 2 * Fq : Fq;
-  const int64_t n = rows * Fq;
+  const int NC = glu ? 2 * Fq : Fq, nb = Fq / 8;
+  const int64_t n = rows * nb;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = i / Fq;
-    const int f = (int)(i - r * Fq);
-    const float* row = gu + (size_t)r * NC;
-    const int qg = (f >> 5) * 64 + (f & 31);
-    const float g = glu ? row[qg] : 0.0f, u = glu ? row[qg + 32] : row[f];
-    float h, cg, cu;
-    act_eval(etype, act, slope, g, u, h, cg, cu);
-    const float d = dh[(size_t)r * Fq + f];
-    uint16_t* base = dgu3 + (size_t)r * 3 * NC;
-    auto put = [&](int q, float v) {
-      uint16_t hi, lo;
-      split_bf16(v, hi, lo);
-      base[q] = hi;
-      base[NC + q] = lo;
-      base[2 * NC + q] = hi;
-    };
+    const int64_t r = i / nb;
+    const int f = (int)(i - r * nb) * 8;
+    float g[8], u[8], d[8];
+    load_gu8(gu, r, NC, f, glu, g, u);
+    load8(dh + (size_t)r * Fq + f, d);
+    float dg[8], du[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      float h, cg, cu;
+      act_eval(etype, act, slope, g[q], u[q], h, cg, cu);
+      dg[q] = d[q] * cg;
+      du[q] = d[q] * cu;
+    }
+    uint16_t* row = dgu + (size_t)r * 2 * NC;
+    uint4 hi, lo;
     if (glu) {
-      put(qg, d * cg);
-      put(qg + 32, d * cu);
+      uint16_t* o = row + (f >> 5) * 64 + (f & 31);
+      split8(dg, hi, lo);
+      *reinterpret_cast<uint4*>(o) = hi;
+      *reinterpret_cast<uint4*>(o + NC) = lo;
+      split8(du, hi, lo);
+      *reinterpret_cast<uint4*>(o + 32) = hi;
+      *reinterpret_cast<uint4*>(o + NC + 32) = lo;
     } else {
-      put(f, d * cu);
+      split8(du, hi, lo);
+      *reinterpret_cast<uint4*>(row + f) = hi;
+      *reinterpret_cast<uint4*>(row + NC + f) = lo;
     }
   }
 }
@@ -1085,47 +1138,52 @@ void mxm_launch_backward_router(const BackwardArgs& a, hipStream_t s) {
 // The fp32 backward's operand planes and elementwise parts; its products run
 // on the MFMA grouped GEMM and weight-gradient kernels over bf16 planes
 // (three plane pairs per fp32 product, fp32 accumulation).
-void mxm_launch_planes3(const float* src, int64_t rows, int cols, int lds, int ldq, bool hlh,
-                        uint16_t* dst, hipStream_t s) {
-  const int64_t n = rows * ldq;
-  if (n > 0)
-    hipLaunchKernelGGL(planes3_kernel, dim3(grid_of((size_t)n)), dim3(256), 0, s, src, rows, cols,
-                       lds, ldq, hlh ? 1 : 0, dst);
+void mxm_launch_planes(const float* src, int64_t rows, int cols, int lds, int ldq, int np,
+                       uint16_t* dst, hipStream_t s) {
+  const int64_t n = rows * (ldq / 8);
+  if (n <= 0) return;
+  const bool vec = cols % 8 == 0 && lds % 4 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0;
+  if (vec)
+    hipLaunchKernelGGL(planes_kernel<true>, dim3(grid_of((size_t)n)), dim3(256), 0, s, src, rows,
+                       cols, lds, ldq, np, dst);
+  else
+    hipLaunchKernelGGL(planes_kernel<false>, dim3(grid_of((size_t)n)), dim3(256), 0, s, src, rows,
+                       cols, lds, ldq, np, dst);
 }
 
-void mxm_launch_planes3_weights(const float* w1, const float* w1b, const float* w2, int E, int D,
-                                int F, int Dq, int Fq, bool glu, uint16_t* w1p, uint16_t* w1t,
-                                uint16_t* w2p, uint16_t* w2t, hipStream_t s) {
+void mxm_launch_planes_weights(const float* w1, const float* w1b, const float* w2, int E, int D,
+                               int F, int Dq, int Fq, bool glu, int np, uint16_t* w1p,
+                               uint16_t* w1t, uint16_t* w2p, uint16_t* w2t, hipStream_t s) {
   const int NCq = glu ? 2 * Fq : Fq;
   const int64_t DF = (int64_t)D * F;
-  auto go = [&](Planes3W a) {
+  auto go = [&](PlanesW a) {
     const int64_t n = (int64_t)a.E * a.R * a.Kq;
-    if (n > 0) hipLaunchKernelGGL(planes3_w_kernel, dim3(grid_of((size_t)n)), dim3(256), 0, s, a);
+    if (n > 0) hipLaunchKernelGGL(planes_w_kernel, dim3(grid_of((size_t)n)), dim3(256), 0, s, a);
   };
-  // up projections: B of G|U = X W1 is [NCq][3 Dq] HLH (row = column of W1)
-  go(Planes3W{w1, glu ? w1b : nullptr, E, NCq, Dq, F, D, glu ? 1 : 0, 0, 1, F, DF, 1, w1p});
-  // B of dX = dGU W1^T is [Dq][3 NCq] HHL (row = d, k = column of W1)
-  go(Planes3W{w1, glu ? w1b : nullptr, E, Dq, NCq, D, F, 0, glu ? 1 : 0, F, 1, DF, 0, w1t});
-  // down projection W2 [F][D]: B of Y = H W2 is [Dq][3 Fq] HLH (row = d, k = f)
-  go(Planes3W{w2, nullptr, E, Dq, Fq, D, F, 0, 0, 1, D, DF, 1, w2p});
-  // B of dH = dY W2^T is [Fq][3 Dq] HHL (row = f, k = d)
-  go(Planes3W{w2, nullptr, E, Fq, Dq, F, D, 0, 0, D, 1, DF, 0, w2t});
+  // up projections: B of G|U = X W1 is [NCq][Dq] (row = column of W1)
+  go(PlanesW{w1, glu ? w1b : nullptr, E, NCq, Dq, F, D, glu ? 1 : 0, 0, 1, F, DF, np, w1p});
+  // B of dX = dGU W1^T is [Dq][NCq] (row = d, k = column of W1)
+  go(PlanesW{w1, glu ? w1b : nullptr, E, Dq, NCq, D, F, 0, glu ? 1 : 0, F, 1, DF, np, w1t});
+  // down projection W2 [F][D]: B of Y = H W2 is [Dq][Fq] (row = d, k = f)
+  if (w2p) go(PlanesW{w2, nullptr, E, Dq, Fq, D, F, 0, 0, 1, D, DF, np, w2p});
+  // B of dH = dY W2^T is [Fq][Dq] (row = f, k = d)
+  go(PlanesW{w2, nullptr, E, Fq, Dq, F, D, 0, 0, D, 1, DF, np, w2t});
 }
 
-void mxm_launch_hidden_planes3(const float* gu, int64_t rows, int Fq, int etype, int act,
-                               float slope, uint16_t* h3, hipStream_t s) {
-  const int64_t n = rows * Fq;
+void mxm_launch_hidden_planes(const float* gu, int64_t rows, int Fq, int etype, int act,
+                              float slope, uint16_t* h, hipStream_t s) {
+  const int64_t n = rows * (Fq / 8);
   if (n > 0)
-    hipLaunchKernelGGL(hidden_planes3_kernel, dim3(grid_of((size_t)n)), dim3(256), 0, s, gu, rows,
-                       Fq, etype, act, slope, h3);
+    hipLaunchKernelGGL(hidden_planes_kernel, dim3(grid_of((size_t)n)), dim3(256), 0, s, gu, rows,
+                       Fq, etype, act, slope, h);
 }
 
-void mxm_launch_act_bw_planes3(const float* gu, const float* dh, int64_t rows, int Fq, int etype,
-                               int act, float slope, uint16_t* dgu3, hipStream_t s) {
-  const int64_t n = rows * Fq;
+void mxm_launch_act_bw_planes(const float* gu, const float* dh, int64_t rows, int Fq, int etype,
+                              int act, float slope, uint16_t* dgu, hipStream_t s) {
+  const int64_t n = rows * (Fq / 8);
   if (n > 0)
-    hipLaunchKernelGGL(act_bw_planes3_kernel, dim3(grid_of((size_t)n)), dim3(256), 0, s, gu, dh,
-                       rows, Fq, etype, act, slope, dgu3);
+    hipLaunchKernelGGL(act_bw_planes_kernel, dim3(grid_of((size_t)n)), dim3(256), 0, s, gu, dh,
+                       rows, Fq, etype, act, slope, dgu);
 }
 
 void mxm_launch_dx_sum(const float* dxr, const float* dxe, int ld, const int32_t* slot_pos, int N,

@@ -183,8 +183,24 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
   // B rows hold Kb k values; the split down projection reads W_down [D][F]
   // twice along its reduction over the hi and lo planes (k wraps at F)
   const int Kb = DOWN_SPLIT ? Kd / 2 : Kd;
+  // pairs of operand planes along k (GemmArgs::f32_out)
+  constexpr bool PAIRS = Epi<EPI>::PLANE_PAIRS;
+  const int Kp = PAIRS ? Kd / a.planes : Kd;
+  const int lda = PAIRS ? a.lda : Kd, ldb = PAIRS ? a.ldb : Kb;
+  // first element of stage k0 within A's and B's rows
+  auto ka = [&](int k0) {
+    if constexpr (!PAIRS) return k0;
+    const int p = (k0 >= Kp) + (k0 >= 2 * Kp);
+    return k0 - p * Kp + ((a.amap >> p) & 1) * Kp;
+  };
+  auto kb = [&](int k0) {
+    if constexpr (DOWN_SPLIT) return k0 >= Kb ? k0 - Kb : k0;
+    if constexpr (!PAIRS) return k0;
+    const int p = (k0 >= Kp) + (k0 >= 2 * Kp);
+    return k0 - p * Kp + ((a.bmap >> p) & 1) * Kp;
+  };
   const uint16_t* __restrict__ B =
-      static_cast<const uint16_t*>(a.b0) + (size_t)e * a.Ncols * Kb;
+      static_cast<const uint16_t*>(a.b0) + (size_t)e * a.Ncols * ldb;
 
   // Global->LDS: global_load_lds_dwordx4 writes lane l's 16 bytes to
   // LDS base + 16*l, so one wave-load fills 1 KB = 64/CH consecutive tile
@@ -213,14 +229,14 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
     const int r = (lwave + LW * i) * RPW + lrow;
     const int p = row0 + min(r, rows - 1);  // rows past the segment reload a valid row
     const int src = (MODE == MXM_GEMM_DOWN && !a.gather_a) ? p : a.perm[p];
-    aoff[i] = 2 * ((size_t)src * Kd + lkc * 8);  // bytes
+    aoff[i] = 2 * ((size_t)src * lda + lkc * 8);  // bytes
   }
-  const size_t bstep = (size_t)(LW * RPW) * Kb;
+  const size_t bstep = (size_t)(LW * RPW) * ldb;
   // the B loads as 32-bit byte offsets from the expert's matrix (one expert's
   // Ncols x Kb bf16 stays far below 4 GiB); the wave index in an SGPR keeps
   // every load's LDS destination scalar
   const int wv = __builtin_amdgcn_readfirstlane(lwave);
-  const unsigned boff = (unsigned)(2 * ((size_t)(n0 + wv * RPW + lrow) * Kb + lkc * 8));
+  const unsigned boff = (unsigned)(2 * ((size_t)(n0 + wv * RPW + lrow) * ldb + lkc * 8));
   const unsigned bstep_b = (unsigned)(2 * bstep);
 
 // Direct-to-LDS loads Q0 .. Q1-1 of one stage (load q < QA fills A rows,
@@ -230,7 +246,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
     if (q_ < QA) {                                                                            \
       ALOAD;                                                                                  \
     } else {                                                                                  \
-      dma16s(B + (DOWN_SPLIT && (K0) >= Kb ? (K0) - Kb : (K0)), boff + (q_ - QA) * bstep_b,   \
+      dma16s(B + kb(K0), boff + (q_ - QA) * bstep_b,                                          \
              STAGE + A_CH + (wv + LW * (q_ - QA)) * 64);                                      \
     }                                                                                         \
   }
@@ -238,10 +254,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
   do {                                                                                        \
     if (A_OFF32 && a.a_off32) {                                                               \
       MXM_DMA_LOOP(STAGE, K0, Q0, Q1,                                                         \
-                   dma16s(A + (K0), (unsigned)aoff[q_], STAGE + (wv + LW * q_) * 64))         \
+                   dma16s(A + ka(K0), (unsigned)aoff[q_], STAGE + (wv + LW * q_) * 64))       \
     } else {                                                                                  \
       MXM_DMA_LOOP(STAGE, K0, Q0, Q1,                                                         \
-                   dma16(reinterpret_cast<const char*>(A + (K0)) + aoff[q_],                  \
+                   dma16(reinterpret_cast<const char*>(A + ka(K0)) + aoff[q_],                \
                          STAGE + (wv + LW * q_) * 64))                                        \
     }                                                                                         \
   } while (0)

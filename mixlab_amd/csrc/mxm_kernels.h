@@ -209,9 +209,12 @@ struct GemmArgs {
   // ... unless the caller forbids it (64-bit addressing throughout)
   bool no_off32;
   // MFMA mode 2 (MXM_GEMM_DOWN): store the fp32 accumulators as they are,
-  // out [rows][Ncols] fp32 (the products of the fp32 backward, each an
-  // A . B^T over bf16 planes concatenated along k)
+  // out [rows][Ncols] fp32 -- the products of the fp32 backward, each an
+  // A . B^T over pairs of bf16 planes, the pairs one after the other along k:
+  // Kd = planes * Kp, pair p takes A's plane (amap >> p) & 1 and B's (bmap >>
+  // p) & 1, planes of Kp columns in rows of lda (A) and ldb (B) elements
   bool f32_out;
+  int planes, amap, bmap, lda, ldb;
   // decode kernels (mxm_launch_gemm_q8): the weights are bf16 in the 2 KB
   // block layout of mxm_launch_shuffle_bf16, without scales (bf16 ops at
   // decode sizes), instead of int8 with scale0 / scale1
@@ -246,17 +249,19 @@ enum { MXM_TILE_AUTO = 0, MXM_TILE_128x128 = 1, MXM_TILE_256x128 = 2, MXM_TILE_2
 int mxm_mfma_tile_rows(int Ncols, int Kd, int family);
 
 // Weight gradients on MFMA (mxm_wgrad.hip): per expert e,
-//   out[e][m][c] = sum_p sum_k A[k][p * aplane + m] * B[k][p * bplane + c]   (fp32)
-// over rows k = offsets[e] .. offsets[e+1]-1 and planes p < planes.  With
+//   out[e][m][c] = sum_p sum_k A[k][ap * aplane + m] * B[k][bp * bplane + c]   (fp32)
+// over rows k = offsets[e] .. offsets[e+1]-1 and plane pairs p < planes, (ap, bp)
+// by amap and bmap.  With
 // glu_f > 0 the C columns are GLU-interleaved in groups of 32 (gate, up) and
 // land de-interleaved: column c -> out[e] + ((c/32) % 2) * out_slot +
 // m * glu_f + (c/64)*32 + c%32; else out[e] + m * C + c.
 struct WgradArgs {
   const uint16_t* a;        // bf16 [rows][lda]
-  int lda, aplane, planes;
+  int lda, aplane, planes;  // pair p takes A's plane (amap >> p) & 1 (aplane columns apart)
   const uint16_t* b;        // bf16 [rows][ldb]
   int ldb;
-  int bplane;               // B's columns of plane p start at p * bplane (0: B is shared)
+  int bplane;               // ... and B's (bmap >> p) & 1
+  int amap, bmap;
   const int32_t* offsets;   // [E + 1]
   const uint16_t* zero;     // 256 zero bf16 (rows past an expert's end)
   int E, M, C;
@@ -318,6 +323,8 @@ struct Epi {
   // the accumulators stored in fp32 (the split down projection's y, or a
   // plain product: GemmArgs::f32_out)
   static constexpr bool Y_F32 = EPI == EPI_DOWN_F32 || EPI == EPI_F32;
+  // a product over pairs of operand planes (GemmArgs::planes)
+  static constexpr bool PLANE_PAIRS = EPI == EPI_F32;
   static constexpr int ETYPE = EPI == EPI_SWIGLU ? MXM_EXPERT_SWIGLU
                                : EPI == EPI_GEGLU ? MXM_EXPERT_GEGLU
                                                   : MXM_EXPERT_MLP;
@@ -513,28 +520,29 @@ void mxm_launch_act_bw_gated_bf16(const uint16_t* gu, const uint16_t* dhr, uint1
                                   bool hsplit, const float* gp, int rows, int F, int etype, int act,
                                   float slope, uint16_t* dgu, float* dgp, hipStream_t s);
 
-// fp32 products on the bf16 MFMA kernels (the fp32 backward): fp32 values
-// as bf16 planes hi = bf16(v), lo = bf16(v - hi), concatenated along k as
-// HHL = [hi | hi | lo] (A side) or HLH = [hi | lo | hi] (B side), so that one
-// bf16 product gives hi.hi + hi.lo + lo.hi.
-// dst [rows][3 ldq]: the planes of src [rows][cols] (row stride lds), zero
-// for cols <= c < ldq.
-void mxm_launch_planes3(const float* src, int64_t rows, int cols, int lds, int ldq, bool hlh,
-                        uint16_t* dst, hipStream_t s);
+// fp32 products on the bf16 MFMA kernels (the fp32 backward): fp32 values as
+// bf16 planes hi = bf16(v), lo = bf16(v - hi), one beside the other, and a
+// product as the sum of the plane pairs hi.hi + hi.lo + lo.hi.  Operands that
+// hold bf16 values (the bf16 flow's x and weights) are their hi plane alone
+// (np = 1), which leaves the pairs of the other operand's planes.
+// dst [rows][np ldq]: the planes of src [rows][cols] (row stride lds), zero
+// for cols <= c < ldq (a multiple of 8).
+void mxm_launch_planes(const float* src, int64_t rows, int cols, int lds, int ldq, int np,
+                       uint16_t* dst, hipStream_t s);
 // The four B operands of the experts' products from fp32 x.W weights (w1 /
 // w1b [E][D][F], w2 [E][F][D]), padded to Dq x Fq (NCq = 2 Fq for GLU, GLU
-// columns interleaved in groups of 32): w1p [E][NCq][3 Dq] (HLH) for
-// G|U = X W1, w1t [E][Dq][3 NCq] (HHL) for dX = dGU W1^T, w2p [E][Dq][3 Fq]
-// (HLH) for Y = H W2, w2t [E][Fq][3 Dq] (HHL) for dH = dY W2^T.
-void mxm_launch_planes3_weights(const float* w1, const float* w1b, const float* w2, int E, int D,
-                                int F, int Dq, int Fq, bool glu, uint16_t* w1p, uint16_t* w1t,
-                                uint16_t* w2p, uint16_t* w2t, hipStream_t s);
-// H [rows][3 Fq] (HHL) from the raw fp32 projections gu [rows][NC].
-void mxm_launch_hidden_planes3(const float* gu, int64_t rows, int Fq, int etype, int act,
-                               float slope, uint16_t* h3, hipStream_t s);
-// dGU [rows][3 NC] (HLH) from gu and dH [rows][Fq] fp32.
-void mxm_launch_act_bw_planes3(const float* gu, const float* dh, int64_t rows, int Fq, int etype,
-                               int act, float slope, uint16_t* dgu3, hipStream_t s);
+// columns interleaved in groups of 32), np planes per row: w1p [E][NCq][Dq]
+// for G|U = X W1, w1t [E][Dq][NCq] for dX = dGU W1^T, w2p [E][Dq][Fq] for
+// Y = H W2 (null: not made), w2t [E][Fq][Dq] for dH = dY W2^T.
+void mxm_launch_planes_weights(const float* w1, const float* w1b, const float* w2, int E, int D,
+                               int F, int Dq, int Fq, bool glu, int np, uint16_t* w1p,
+                               uint16_t* w1t, uint16_t* w2p, uint16_t* w2t, hipStream_t s);
+// H's planes [rows][2 Fq] from the raw fp32 projections gu [rows][NC].
+void mxm_launch_hidden_planes(const float* gu, int64_t rows, int Fq, int etype, int act,
+                              float slope, uint16_t* h, hipStream_t s);
+// dGU's planes [rows][2 NC] from gu and dH [rows][Fq] fp32.
+void mxm_launch_act_bw_planes(const float* gu, const float* dh, int64_t rows, int Fq, int etype,
+                              int act, float slope, uint16_t* dgu, hipStream_t s);
 // dx[n] = dxr[n] + sum_k dxe[slot_pos[n, k]] (dxe rows ld apart).
 void mxm_launch_dx_sum(const float* dxr, const float* dxe, int ld, const int32_t* slot_pos, int N,
                        int D, int K, float* dx, hipStream_t s);

@@ -1,10 +1,10 @@
 // Weight gradients of the grouped expert FFN on bf16 MFMA (gfx950).
 //
-//   Out[e][m][c] = sum_p sum_k A[k][p * aplane + m] * B[k][c]   (fp32)
+//   Out[e][m][c] = sum_p sum_k A[k][ap * aplane + m] * B[k][bp * bplane + c]   (fp32)
 //
 // over expert e's rows k = offsets[e] .. offsets[e+1]-1 (the forward's
-// permuted slot order) and the planes p of A (two for a hidden stored as
-// bf16 hi and lo planes, else one).  This is dW1 = Xp^T dG|dU (A = x, row k
+// permuted slot order) and the pairs p of planes of A and B (two for a hidden
+// stored as bf16 hi and lo planes, up to three for fp32 operands, else one).  This is dW1 = Xp^T dG|dU (A = x, row k
 // read at the token index a_rows[k] of the slot, B = the activation
 // backward's output) and dW_down = Hg^T dD (A = the gated hidden gate * h,
 // rows in slot order, B = the upstream gradient's bf16 row of the slot's
@@ -449,11 +449,11 @@ __global__ __launch_bounds__(TL::NT, 1) void wgrad_kernel(WgradArgs a) {
     // next stage to load, into ring slot kt % NS
     auto dma_part = [&](int kt, int l0, int l1) {
       unsigned char* st = lds + (kt % NS) * BUF;
-      const int p = dp, kk = dkk;
+      const int ap = (a.amap >> dp) & 1, bp = (a.bmap >> dp) & 1, kk = dkk;
       if (kk + BK <= cnt) {
         // a whole stage of rows
-        const uint16_t* as = A + (size_t)(row0 + kk) * a.lda + (size_t)p * a.aplane;
-        const uint16_t* bs = B + (size_t)(row0 + kk) * a.ldb + (size_t)p * a.bplane;
+        const uint16_t* as = A + (size_t)(row0 + kk) * a.lda + (size_t)ap * a.aplane;
+        const uint16_t* bs = B + (size_t)(row0 + kk) * a.ldb + (size_t)bp * a.bplane;
         auto whole = [&](auto off32) {
 #pragma unroll
           for (int q = 0; q < LDPS; ++q) {
@@ -462,10 +462,10 @@ __global__ __launch_bounds__(TL::NT, 1) void wgrad_kernel(WgradArgs a) {
               // gathered rows: each candidate row's byte offset (scalar) plus
               // the lane's column, the lane taking its own row's
               if constexpr (GA && decltype(off32)::value) {
-                wg_dma16s(A + (size_t)p * a.aplane, pick_off(srow[q], ra, rpwa, a_pitch, a_colb),
+                wg_dma16s(A + (size_t)ap * a.aplane, pick_off(srow[q], ra, rpwa, a_pitch, a_colb),
                           st + (wv + NW * q) * 1024);
               } else if constexpr (GA) {
-                wg_dma16(A + (size_t)pick(srow[q], ra, rpwa) * a.lda + (size_t)p * a.aplane + m0 +
+                wg_dma16(A + (size_t)pick(srow[q], ra, rpwa) * a.lda + (size_t)ap * a.aplane + m0 +
                              lca * 8,
                          st + (wv + NW * q) * 1024);
               } else {
@@ -474,10 +474,10 @@ __global__ __launch_bounds__(TL::NT, 1) void wgrad_kernel(WgradArgs a) {
             } else {
               const int qb = q - QA;
               if constexpr (GB && decltype(off32)::value) {
-                wg_dma16s(B + (size_t)p * a.bplane, pick_off(srowb[qb], rb, rpwb, b_pitch, b_colb),
+                wg_dma16s(B + (size_t)bp * a.bplane, pick_off(srowb[qb], rb, rpwb, b_pitch, b_colb),
                           st + A_BYTES + (wv + NW * qb) * 1024);
               } else if constexpr (GB) {
-                wg_dma16(B + (size_t)pick(srowb[qb], rb, rpwb) * a.ldb + (size_t)p * a.bplane + c0 +
+                wg_dma16(B + (size_t)pick(srowb[qb], rb, rpwb) * a.ldb + (size_t)bp * a.bplane + c0 +
                              lcb * 8,
                          st + A_BYTES + (wv + NW * qb) * 1024);
               } else {
@@ -497,7 +497,7 @@ __global__ __launch_bounds__(TL::NT, 1) void wgrad_kernel(WgradArgs a) {
             const int k = kk + (wv + NW * q) * RPWA + ra;
             int arw = row0 + k;
             if constexpr (GA) arw = pick(srow[q], ra, rpwa);
-            const uint16_t* src = k < cnt ? A + (size_t)arw * a.lda + (size_t)p * a.aplane + m0 + lca * 8
+            const uint16_t* src = k < cnt ? A + (size_t)arw * a.lda + (size_t)ap * a.aplane + m0 + lca * 8
                                           : a.zero + lca * 8;
             wg_dma16(src, st + (wv + NW * q) * 1024);
           } else {
@@ -505,7 +505,7 @@ __global__ __launch_bounds__(TL::NT, 1) void wgrad_kernel(WgradArgs a) {
             const int k = kk + (wv + NW * qb) * RPWB + rb;
             int brw = row0 + k;
             if constexpr (GB) brw = pick(srowb[qb], rb, rpwb);
-            const uint16_t* src = k < cnt ? B + (size_t)brw * a.ldb + (size_t)p * a.bplane + c0 +
+            const uint16_t* src = k < cnt ? B + (size_t)brw * a.ldb + (size_t)bp * a.bplane + c0 +
                                                 lcb * 8
                                           : a.zero + lcb * 8;
             wg_dma16(src, st + A_BYTES + (wv + NW * qb) * 1024);
