@@ -280,6 +280,9 @@ struct WgradArgs {
   // of C (0: all).  With the interleave, glu_f is the real width: hidden
   // units f >= glu_f are not stored.
   int m_store, c_store;
+  // set by the launcher: the operands' columns (M and C before it rounds them
+  // up to its tiles)
+  int a_cols, b_cols;
 };
 // M and C multiples of 128.
 bool mxm_wgrad_fits(int M, int C);

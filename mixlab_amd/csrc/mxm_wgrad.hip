@@ -383,17 +383,19 @@ __global__ __launch_bounds__(TL::NT, 1) void wgrad_kernel(WgradArgs a) {
     // element offsets of this lane's loads within a whole stage, fixed for
     // the item: the stage adds a uniform base (rows row0 + dkk, plane dp)
     const int wv = __builtin_amdgcn_readfirstlane(wave);
+    // this lane's columns; past the operand's last (a tile that reaches over
+    // it) its last 8 again, for outputs that are not stored
+    const int acol = min(m0 + lca * 8, a.a_cols - 8), bcol = min(c0 + lcb * 8, a.b_cols - 8);
     int a_lane[QA], b_lane[LDPS - QA];
 #pragma unroll
-    for (int q = 0; q < QA; ++q) a_lane[q] = ((wv + NW * q) * RPWA + ra) * a.lda + m0 + lca * 8;
+    for (int q = 0; q < QA; ++q) a_lane[q] = ((wv + NW * q) * RPWA + ra) * a.lda + acol;
 #pragma unroll
-    for (int q = 0; q < LDPS - QA; ++q)
-      b_lane[q] = ((wv + NW * q) * RPWB + rb) * a.ldb + c0 + lcb * 8;
+    for (int q = 0; q < LDPS - QA; ++q) b_lane[q] = ((wv + NW * q) * RPWB + rb) * a.ldb + bcol;
     // a gathered operand below 4 GiB: the lane's column part in bytes and the
     // row pitch in bytes (rows are added per stage from the scalar row indices)
-    const unsigned a_colb = 2u * (unsigned)(m0 + lca * 8);
+    const unsigned a_colb = 2u * (unsigned)acol;
     const unsigned a_pitch = 2u * (unsigned)a.lda;
-    const unsigned b_colb = 2u * (unsigned)(c0 + lcb * 8);
+    const unsigned b_colb = 2u * (unsigned)bcol;
     const unsigned b_pitch = 2u * (unsigned)a.ldb;
     const bool g32 = (GA && a.a_rows32) || (GB && a.b_rows32);
 
@@ -465,8 +467,7 @@ __global__ __launch_bounds__(TL::NT, 1) void wgrad_kernel(WgradArgs a) {
                 wg_dma16s(A + (size_t)ap * a.aplane, pick_off(srow[q], ra, rpwa, a_pitch, a_colb),
                           st + (wv + NW * q) * 1024);
               } else if constexpr (GA) {
-                wg_dma16(A + (size_t)pick(srow[q], ra, rpwa) * a.lda + (size_t)ap * a.aplane + m0 +
-                             lca * 8,
+                wg_dma16(A + (size_t)pick(srow[q], ra, rpwa) * a.lda + (size_t)ap * a.aplane + acol,
                          st + (wv + NW * q) * 1024);
               } else {
                 wg_dma16s(as, 2u * (unsigned)a_lane[q], st + (wv + NW * q) * 1024);
@@ -477,8 +478,8 @@ __global__ __launch_bounds__(TL::NT, 1) void wgrad_kernel(WgradArgs a) {
                 wg_dma16s(B + (size_t)bp * a.bplane, pick_off(srowb[qb], rb, rpwb, b_pitch, b_colb),
                           st + A_BYTES + (wv + NW * qb) * 1024);
               } else if constexpr (GB) {
-                wg_dma16(B + (size_t)pick(srowb[qb], rb, rpwb) * a.ldb + (size_t)bp * a.bplane + c0 +
-                             lcb * 8,
+                wg_dma16(B + (size_t)pick(srowb[qb], rb, rpwb) * a.ldb + (size_t)bp * a.bplane +
+                             bcol,
                          st + A_BYTES + (wv + NW * qb) * 1024);
               } else {
                 wg_dma16s(bs, 2u * (unsigned)b_lane[qb], st + A_BYTES + (wv + NW * qb) * 1024);
@@ -497,7 +498,7 @@ __global__ __launch_bounds__(TL::NT, 1) void wgrad_kernel(WgradArgs a) {
             const int k = kk + (wv + NW * q) * RPWA + ra;
             int arw = row0 + k;
             if constexpr (GA) arw = pick(srow[q], ra, rpwa);
-            const uint16_t* src = k < cnt ? A + (size_t)arw * a.lda + (size_t)ap * a.aplane + m0 + lca * 8
+            const uint16_t* src = k < cnt ? A + (size_t)arw * a.lda + (size_t)ap * a.aplane + acol
                                           : a.zero + lca * 8;
             wg_dma16(src, st + (wv + NW * q) * 1024);
           } else {
@@ -505,8 +506,7 @@ __global__ __launch_bounds__(TL::NT, 1) void wgrad_kernel(WgradArgs a) {
             const int k = kk + (wv + NW * qb) * RPWB + rb;
             int brw = row0 + k;
             if constexpr (GB) brw = pick(srowb[qb], rb, rpwb);
-            const uint16_t* src = k < cnt ? B + (size_t)brw * a.ldb + (size_t)bp * a.bplane + c0 +
-                                                lcb * 8
+            const uint16_t* src = k < cnt ? B + (size_t)brw * a.ldb + (size_t)bp * a.bplane + bcol
                                           : a.zero + lcb * 8;
             wg_dma16(src, st + A_BYTES + (wv + NW * qb) * 1024);
           }
@@ -686,8 +686,8 @@ __global__ __launch_bounds__(TL::NT, 1) void wgrad_kernel(WgradArgs a) {
 // Work units are 16-row slices of the (split expert, tile) pairs; a thread
 // takes 4 float4 of a slice (4 consecutive columns stay inside one GLU group
 // of 32) and keeps their loads in flight together.
-// VEC: whole float4 of the output (16-byte aligned rows, nothing past the
-// stored region); else element by element within the stored region.
+// VEC: whole float4 of the output (16-byte aligned rows of a multiple of 4);
+// else element by element.  Either way within the output's shape only.
 template <int BM, int BN, bool VEC>
 __global__ __launch_bounds__(256) void wgrad_reduce_kernel(WgradArgs a) {
   constexpr int SR = 16;                       // rows per unit
@@ -748,15 +748,16 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(WgradArgs a) {
     }
     float4* o[V];
     float4 v[V];
+    bool in[V];  // inside the output's shape (whole float4: 4 divides its width)
 #pragma unroll
     for (int q = 0; q < V; ++q) {
       const int i = tid + 256 * q;
       const int m = r0 + i / (BN / 4), c = c0 + (i % (BN / 4)) * 4;
-      const size_t cofs = a.glu_f > 0
-                              ? (size_t)((c >> 5) & 1) * a.out_slot + (size_t)((c >> 6) * 32 + (c & 31))
-                              : (size_t)c;
+      const int cu = a.glu_f > 0 ? (c >> 6) * 32 + (c & 31) : c;
+      const size_t cofs = a.glu_f > 0 ? (size_t)((c >> 5) & 1) * a.out_slot + (size_t)cu : (size_t)c;
       o[q] = reinterpret_cast<float4*>(out + (size_t)(m0 + m) * ld + cofs);
-      v[q] = *o[q];
+      in[q] = m0 + m < mst && cu < ld;
+      v[q] = in[q] ? *o[q] : float4{};
     }
     const int n = nch[e];
     for (int jc = 1; jc < n; ++jc) {
@@ -774,7 +775,8 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(WgradArgs a) {
       }
     }
 #pragma unroll
-    for (int q = 0; q < V; ++q) *o[q] = v[q];
+    for (int q = 0; q < V; ++q)
+      if (in[q]) *o[q] = v[q];
   }
 }
 
@@ -820,12 +822,9 @@ struct WFamily {
       launch_main<true>(a, s);
     else
       launch_main<false>(a, s);
-    // whole float4 when the output rows are 16-byte aligned and every column
-    // of the padded operands is stored
+    // whole float4 when the output rows are 16-byte aligned
     const int ld = a.glu_f > 0 ? a.glu_f : a.c_store > 0 ? a.c_store : a.C;
-    const bool vec = ld % 4 == 0 && (a.m_store <= 0 || a.m_store == a.M) &&
-                     (a.glu_f > 0 ? 2 * a.glu_f == a.C : (a.c_store <= 0 || a.c_store == a.C)) &&
-                     reinterpret_cast<uintptr_t>(a.out) % 16 == 0 && a.out_estride % 4 == 0 &&
+    const bool vec = ld % 4 == 0 && reinterpret_cast<uintptr_t>(a.out) % 16 == 0 && a.out_estride % 4 == 0 &&
                      a.out_slot % 4 == 0;
     if (vec)
       hipLaunchKernelGGL((wgrad_reduce_kernel<BM, BN, true>), dim3(std::max(8, n_cus() * 2)),
@@ -838,7 +837,17 @@ struct WFamily {
 using WBig = WFamily<256, 256, 2, 4, 64, 2>;
 using WSmall = WFamily<128, 128, 2, 2, 64, 2>;
 
-bool wgrad_big(int M, int C) { return M % 256 == 0 && C % 256 == 0; }
+// 256 x 256 tiles where they fit, or reach past the output by at most a third
+// of it: per multiply-add they are well over a third faster than 128 x 128
+// ones (4096 rows x 2 of D 544 padded to 640 against 3072 columns, two plane
+// pairs: 195 us on 128 x 128 tiles, 125 on 256 x 256 over 768 rows; whole bf16
+// training steps 302 -> 226 us at D 640 / ffn 1709, 2448 -> 2057 at D 776 /
+// ffn 3904).  Also where they are fewer than the CUs: keeping 128 x 128 there
+// took the first of those steps back to 299 us.
+bool wgrad_big(int M, int C) {
+  const int64_t Mp = (M + 255) / 256 * 256, Cp = (C + 255) / 256 * 256;
+  return 3 * Mp * Cp <= 4 * (int64_t)M * C;
+}
 
 }  // namespace
 
@@ -848,10 +857,22 @@ size_t mxm_wgrad_scratch_bytes(int M, int C) {
   return wgrad_big(M, C) ? WBig::scratch_bytes() : WSmall::scratch_bytes();
 }
 
-void mxm_launch_wgrad(const WgradArgs& a, hipStream_t s) {
-  if (a.E <= 0) return;
-  if (wgrad_big(a.M, a.C))
-    WBig::launch(a, s);
-  else
+void mxm_launch_wgrad(const WgradArgs& args, hipStream_t s) {
+  if (args.E <= 0) return;
+  WgradArgs a = args;
+  a.a_cols = a.M;
+  a.b_cols = a.C;
+  if (!wgrad_big(a.M, a.C)) {
     WSmall::launch(a, s);
+    return;
+  }
+  if (a.M % 256 != 0) {
+    if (a.m_store <= 0) a.m_store = a.M;
+    a.M = (a.M + 255) / 256 * 256;
+  }
+  if (a.C % 256 != 0) {  // (never with the GLU interleave: its C are pairs of 128)
+    if (a.c_store <= 0) a.c_store = a.C;
+    a.C = (a.C + 255) / 256 * 256;
+  }
+  WBig::launch(a, s);
 }
