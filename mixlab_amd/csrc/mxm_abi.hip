@@ -1195,9 +1195,9 @@ int64_t mxm_moe_create(const float* float_params, int n_float_params, const int3
         HIPCK(hipStreamSynchronize(o->stream));
       }
     } else {
-      o->w1.alloc(EE * DF * 4);
-      if (o->wpe == 3) o->w1b.alloc(EE * DF * 4);
-      o->w2.alloc(EE * DF * 4);
+      o->w1.alloc(EE * DF * 4 + MXM_SIMT_PAD);
+      if (o->wpe == 3) o->w1b.alloc(EE * DF * 4 + MXM_SIMT_PAD);
+      o->w2.alloc(EE * DF * 4 + MXM_SIMT_PAD);
     }
     std::lock_guard<std::mutex> lk(g_mu);
     handle = g_next_handle++;
@@ -1861,7 +1861,7 @@ void run_backward(MoeOp& o, const void* x, int x_dtype, const float* d_delta, fl
     if (!mfma_bw) o.bw_dy.alloc(NK * D * 4);  // (the MFMA backward keeps no dY)
     o.bw_dgates.alloc(NK * 4);
     o.bw_dlogits.alloc(N * E * 4);
-    o.bw_wrt.alloc(D * E * 4);
+    o.bw_wrt.alloc(D * E * 4 + MXM_SIMT_PAD);
     o.bw_wr_part.alloc((size_t)wgrad_router_chunks(o.N, D, E) * D * E * 4);
     o.bw_one.alloc(16);
     o.bw_one_host[1] = o.N;

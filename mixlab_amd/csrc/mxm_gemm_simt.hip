@@ -23,6 +23,8 @@
 // against fmaf chains bit for bit), so each output is the same fmaf chain
 // over the same k steps, zero padding included, as on the vector unit, at
 // twice the non-packed fp32 rate.
+#include <type_traits>
+
 #include "mxm_kernels.h"
 
 namespace {
@@ -232,6 +234,127 @@ __global__ __launch_bounds__(NT) void gemm_simt_kernel(GemmArgs a) {
   }
 }
 
+// The 64 x 64 matrix-core tile on fp32 rows, loads of 4 floats per lane: the
+// element loads of the kernel above are each under a bounds check, a branch
+// apiece in the loop (12 per thread and k tile with GLU), and its fragment reads
+// wait one by one; this one's loop has 2 or 3 unconditional 16-byte loads (4-byte
+// aligned: rows of any length), one barrier per k tile (two LDS buffers) and 8 k
+// steps of fragments read ahead of the 8 being multiplied.  Rows past the
+// segment reload its last one and columns past NC read what follows in the
+// matrix (its buffer ends in MXM_SIMT_PAD spare bytes): neither is stored, and
+// no stored output reads them.  The last k tile of a Kd that is no multiple of
+// 16 is loaded element by element with zeros past Kd.  The same fmaf chains as
+// above, bit for bit.  Bound by the matrix core (k = 1 products at about 140
+// TFLOP/s) and the LDS reads and barriers around it: 16384 tokens of D 512 / E 8
+// / K 2 / ffn 2048 gate+up 1562 -> 1435 us (96 TFLOP/s), down 875 -> 766 us; 4096
+// of ffn 1367 340 -> 306 and 204 -> 184 us.
+typedef float f4_u __attribute__((ext_vector_type(4), aligned(4)));
+
+template <bool BF16, int MODE>
+__global__ __launch_bounds__(NT) void gemm_simt_mf_kernel(GemmArgs a) {
+  constexpr int NB = (MODE == MXM_GEMM_GLU) ? 2 : 1;
+  constexpr int T = 64, BK = 16, LD = T + 4;
+  constexpr int KG = 8;  // k steps of fragments in flight
+  __shared__ __attribute__((aligned(16))) float As[2][BK][LD];
+  __shared__ __attribute__((aligned(16))) float Bs[2][NB][BK][LD];
+
+  const int mtile = blockIdx.y;
+  if (mtile >= a.mstart[a.E]) return;
+  const int e = find_expert(a.mstart, a.E, mtile);
+  const int row0 = a.offsets[e] + (mtile - a.mstart[e]) * T;
+  const int rows = min(T, a.offsets[e + 1] - row0);
+  const int n0 = blockIdx.x * T;
+  const int Kd = a.Kd, NC = a.Ncols;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+
+  // this thread's pieces: A row tid / 4, k 4 (tid % 4) .. + 3 of the k tile;
+  // B k tid / 16, columns 4 (tid % 16) .. + 3
+  const int ar = tid >> 2, ak = (tid & 3) * 4, bk = tid >> 4, bc = (tid & 15) * 4;
+  const int p = row0 + min(ar, rows - 1);
+  const float* __restrict__ A =
+      static_cast<const float*>(a.a) + (size_t)(MODE == MXM_GEMM_DOWN ? p : a.perm[p]) * Kd + ak;
+  const float* __restrict__ B[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+    B[b] = static_cast<const float*>(b == 0 ? a.b0 : a.b1) + (size_t)e * Kd * NC +
+           (size_t)bk * NC + n0 + bc;
+  f4_u ra, rb[NB];
+  auto fetch = [&](int k0) {
+    if (k0 + BK <= Kd) {
+      ra = *reinterpret_cast<const f4_u*>(A + k0);
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        rb[b] = *reinterpret_cast<const f4_u*>(B[b] + (size_t)k0 * NC);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) ra[q] = k0 + ak + q < Kd ? A[k0 + q] : 0.0f;
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          rb[b][q] = k0 + bk < Kd && n0 + bc + q < NC ? B[b][(size_t)k0 * NC + q] : 0.0f;
+    }
+  };
+
+  mf_v16 acc[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) acc[b] = mf_v16{};
+  const int wr0 = 32 * (wave >> 1), wc0 = 32 * (wave & 1);
+  const int arow_l = wr0 + 16 * ((lane >> 4) >> 1) + (lane & 15);
+  const int bcol_l = wc0 + 16 * ((lane >> 4) & 1) + (lane & 15);
+  fetch(0);
+  int buf = 0;
+  for (int k0 = 0; k0 < Kd; k0 += BK, buf ^= 1) {
+    // (this buffer's readers passed the barrier of the tile before)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) As[buf][ak + q][ar] = ra[q];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) *reinterpret_cast<f4_u*>(&Bs[buf][b][bk][bc]) = rb[b];
+    __syncthreads();
+    if (k0 + BK < Kd) fetch(k0 + BK);
+    float av[2][KG], bv[2][NB][KG];
+    auto frags = [&](int set, int kk0) {
+#pragma unroll
+      for (int k = 0; k < KG; ++k) {
+        av[set][k] = As[buf][kk0 + k][arow_l];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) bv[set][b][k] = Bs[buf][b][kk0 + k][bcol_l];
+      }
+    };
+    frags(0, 0);
+    static_assert(BK == 2 * KG, "two groups of k steps");
+    frags(1, KG);
+    __builtin_amdgcn_sched_barrier(0);  // (not one read and one wait per product)
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int k = 0; k < KG; ++k)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+          acc[b] = __builtin_amdgcn_mfma_f32_16x16x1f32(av[g][k], bv[g][b][k], acc[b], 0, 0, 0);
+  }
+
+  float* out = static_cast<float*>(a.out);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int row = wr0 + 16 * ((i >> 2) >> 1) + (lane >> 4) * 4 + (i & 3);
+    const int c = n0 + wc0 + 16 * ((i >> 2) & 1) + (lane & 15);
+    if (row >= rows || c >= NC) continue;
+    float v;
+    if (MODE == MXM_GEMM_GLU) {
+      v = mxm_hidden<BF16>(a.expert_type, a.activation, a.slope, acc[0][i], acc[NB - 1][i]);
+    } else if (MODE == MXM_GEMM_MLP) {
+      const float u = acc[0][i];
+      if (a.out2) static_cast<float*>(a.out2)[(size_t)(row0 + row) * a.ld2 + c] = u;
+      v = mxm_hidden<BF16>(MXM_EXPERT_MLP, a.activation, a.slope, 0.0f, u);
+    } else {
+      v = acc[0][i];
+      if (a.y_bf16) v = mxm_rbf(v);
+    }
+    if (out) out[(size_t)(row0 + row) * NC + c] = v;
+  }
+}
+
 // k tiles of 16 for the 64 x 64 tile (each thread's 16 outputs per k step
 // amortise the tile's barriers), 32 for the 32 x 32 tile (4 outputs per k
 // step: half as many barrier and LDS round trips per k)
@@ -239,19 +362,22 @@ template <typename TA, bool BF16, int T, bool MF>
 void launch_t(const GemmArgs& a, hipStream_t s) {
   constexpr int BK = T == 64 ? 16 : 32;
   const dim3 grid((a.Ncols + T - 1) / T, a.max_mtiles);
+  auto go = [&](auto mode) {
+    constexpr int MODE = decltype(mode)::value;
+    // (the down projection's rows, H, are fp32 in either flow)
+    using T2 = typename std::conditional<MODE == MXM_GEMM_DOWN, float, TA>::type;
+    if constexpr (MF && sizeof(T2) == 4)
+      hipLaunchKernelGGL((gemm_simt_mf_kernel<BF16, MODE>), grid, dim3(NT), 0, s, a);
+    else
+      hipLaunchKernelGGL((gemm_simt_kernel<T2, BF16, MODE, T, T, BK, MF>), grid, dim3(NT), 0, s, a);
+  };
   switch (a.mode) {
     case MXM_GEMM_GLU:
-      hipLaunchKernelGGL((gemm_simt_kernel<TA, BF16, MXM_GEMM_GLU, T, T, BK, MF>), grid, dim3(NT),
-                         0, s, a);
-      break;
+      return go(std::integral_constant<int, MXM_GEMM_GLU>{});
     case MXM_GEMM_MLP:
-      hipLaunchKernelGGL((gemm_simt_kernel<TA, BF16, MXM_GEMM_MLP, T, T, BK, MF>), grid, dim3(NT),
-                         0, s, a);
-      break;
+      return go(std::integral_constant<int, MXM_GEMM_MLP>{});
     default:
-      hipLaunchKernelGGL((gemm_simt_kernel<float, BF16, MXM_GEMM_DOWN, T, T, BK, MF>), grid,
-                         dim3(NT), 0, s, a);
-      break;
+      return go(std::integral_constant<int, MXM_GEMM_DOWN>{});
   }
 }
 

@@ -236,6 +236,8 @@ struct GemmArgs {
   // workgroup that computes aux and entropy
   DecodeAux daux;
 };
+// Spare bytes at the end of every B matrix buffer given to the SIMT family.
+#define MXM_SIMT_PAD 256
 // SIMT family: weights in the reference layout (x . W, [in, out]) per expert,
 // fp32 storage; H and Y are fp32.  Accumulation is fmaf in ascending k.
 void mxm_launch_gemm_simt(const GemmArgs& a, bool bf16, hipStream_t s);
