@@ -233,7 +233,7 @@ struct MoeOp {
   // bf16 ops of the MFMA family: bf16 intermediates of the MFMA backward and
   // the weights re-laid for its products (W_down [F][D], W1 [D][NC])
   bool bw_wbf_ready = false;
-  DevBuf bw_dhb, bw_gub, bw_dgub, bw_dxeb, bw_zero, bw_w2o, bw_w1u, bw_wscr,
+  DevBuf bw_gub, bw_dgub, bw_dxeb, bw_zero, bw_w2o, bw_w1u, bw_wscr,
       bw_ddb, bw_gp, bw_dgp, bw_dlb, bw_dwr2;
   // the fp32 backward's products (run_backward_x3): bf16 planes of the
   // operands at the padded widths Dq x Fq, fp32 products
@@ -435,7 +435,7 @@ void alloc_workspace(MoeOp& o) {
 // Refuse to launch a GEMM whose operands are not all allocated (a kernel
 // would otherwise read through a null pointer).
 void require_operands(const GemmArgs& g, bool second_matrix, bool scaled) {
-  if (!g.a || !g.b0 || (!g.out && !g.out2) || !g.offsets || (second_matrix && !g.b1) ||
+  if (!g.a || !g.b0 || (!g.out && !g.out2 && !g.abw.dgu) || !g.offsets || (second_matrix && !g.b1) ||
       (scaled && (!g.scale0 || (g.mode == MXM_GEMM_GLU && !g.scale1))) ||
       (g.mode != MXM_GEMM_DOWN && !g.perm))
     fail_rt("OP_MOE_FEED_FORWARD internal error: expert GEMM operand not allocated (mode %d)", g.mode);
@@ -1446,12 +1446,12 @@ bool mfma_backward_fits(const MoeOp& o) {
 //   G|U = Xp W1                kept by the forward (its gate+up GEMM stores
 //                              only the raw projections, GemmArgs::out2)
 //   dH' = dD[token] W_down^T   MFMA grouped GEMM on the bf16 dD rows gathered
-//                              through perm, W_down kept as [F][D] bf16; not
-//                              yet gated
-//   dgates = <dH', h>          (= <dD, Y>), dH = gate * dH', dG|dU and the
+//                              through perm, W_down kept as [F][D] bf16; never
+//                              stored: its epilogue (ActBwArgs) gives
+//   dgates = <dH', h>          (= <dD, Y>), with dH = gate * dH' dG|dU, and the
 //                              gated hidden Hg = gate * h, h from G|U as the
-//                              forward's epilogue computes it: one pass
-//                              (act_bw_gated_bf16), then the router part
+//                              forward's epilogue computes it; then the router
+//                              part
 //   dXe = dG|dU W1^T           MFMA grouped GEMM, W1 kept as [D][NC] bf16
 //   dx  = dlogits Wr^T + sum_k dXe   (dx_fused_bf16; with a dx that is not
 //                              16-byte aligned: dxr + sum_k dXe, dx_bf16)
@@ -1472,8 +1472,7 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
   const bool dwr_mfma =
       o.dwr_mode >= 0 ? o.dwr_mode == 1 : (double)o.N * D * E >= (double)(1 << 28);
   const int Ep = (E + 63) / 64 * 64;  // that product's hi and lo halves of Ep columns
-  if (!o.bw_dhb.p) {
-    o.bw_dhb.alloc(NK * Fk * 2);
+  if (!o.bw_dgub.p) {
     o.bw_dgub.alloc(NK * NC * 2);
     o.bw_dxeb.alloc(NK * D * 2);
     o.bw_zero.alloc(512);  // 256 zero bf16: the weight gradients' rows past an expert's end
@@ -1490,7 +1489,7 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
     o.bw_w1u.alloc((size_t)E * D * NC * 2);
     o.bw_ddb.alloc((size_t)o.N * D * 2);
     o.bw_gp.alloc(NK * 4);
-    o.bw_dgp.alloc(NK * 4);
+    o.bw_dgp.alloc((size_t)(Fk / 64) * NK * 4);
   }
   if (!o.bw_wbf_ready) {
     for (int e = 0; e < E; ++e) {
@@ -1503,15 +1502,14 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
     HIPCK(hipGetLastError());
     o.bw_wbf_ready = true;
   }
-  uint16_t *dhb = o.bw_dhb.as<uint16_t>(), *gub = o.bw_gub.as<uint16_t>(),
-           *dgub = o.bw_dgub.as<uint16_t>(), *dxeb = o.bw_dxeb.as<uint16_t>(),
+  uint16_t *gub = o.bw_gub.as<uint16_t>(), *dgub = o.bw_dgub.as<uint16_t>(), *dxeb = o.bw_dxeb.as<uint16_t>(),
            *ddb = o.bw_ddb.as<uint16_t>();
   // dD in bf16 per token and the gates by slot position (dW_down takes the
   // gate on its left operand, so no per-slot dY = gate * dD is written)
   mxm_launch_dy_gate(b.d_delta, b.gates, b.slot_pos, o.N, D, o.K, ddb, nullptr,
                      o.bw_gp.as<float>(), st);
   auto product = [&](const uint16_t* A, const void* W, uint16_t* out, int Kd, int Ncols,
-                     bool gather) {
+                     bool gather, const ActBwArgs* abw) {
     GemmArgs g{};
     g.no_off32 = o.force64;
     g.mode = MXM_GEMM_DOWN;
@@ -1526,21 +1524,31 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
     g.gather_a = gather;  // A rows = token rows through perm
     g.perm = b.perm;
     g.rows_total = (int)NK;
+    if (abw) {
+      g.abw = *abw;
+      g.expert_type = o.etype;
+      g.activation = o.act;
+      g.slope = o.slope;
+    }
     require_operands(g, false, false);
     mxm_launch_gemm_mfma(g, st);
     HIPCK(hipGetLastError());
   };
-  // dH' = dD W_down^T for each slot's token, ungated: with H it gives the
-  // gate gradients <dD, Y> = <dH', h>, and dH = gate * dH'
-  product(ddb, o.bw_w2o.p, dhb, D, Fk, true);
-  // gub holds G|U from the forward (run_forward's pre_out)
-  mxm_launch_act_bw_gated_bf16(gub, dhb, static_cast<uint16_t*>(o.ws.H), o.hsplit,
-                               o.bw_gp.as<float>(), (int)NK, Fk, o.etype, o.act, o.slope, dgub,
-                               o.bw_dgp.as<float>(), st);
-  HIPCK(hipGetLastError());
+  // dH' = dD W_down^T for each slot's token, ungated: with the hidden (from
+  // the forward's G|U in gub) it gives the gate gradients <dD, Y> = <dH', h>,
+  // and dH = gate * dH' the activation backward, all in the product's epilogue
+  ActBwArgs abw{};
+  abw.gu = gub;
+  abw.gp = o.bw_gp.as<float>();
+  abw.Hg = static_cast<uint16_t*>(o.ws.H);
+  abw.dgu = dgub;
+  abw.dgp = o.bw_dgp.as<float>();
+  abw.hsplit = o.hsplit;
+  product(ddb, o.bw_w2o.p, nullptr, D, Fk, true, &abw);
   // the router part from those gate gradients
   BackwardArgs br = b;
   br.dgp = o.bw_dgp.as<float>();
+  br.dgp_parts = Fk / 64;
   br.dwr_by_caller = dwr_mfma;
   mxm_launch_backward_router(br, st);
   HIPCK(hipGetLastError());
@@ -1569,7 +1577,7 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
     mxm_launch_dwr_halves(o.bw_dwr2.as<float>(), D, E, Ep, b.dwr, st);
     HIPCK(hipGetLastError());
   }
-  product(dgub, o.bw_w1u.p, dxeb, NC, D, false);
+  product(dgub, o.bw_w1u.p, dxeb, NC, D, false, nullptr);
   if (b.dxr)
     mxm_launch_dx_bf16(b.dxr, dxeb, b.slot_pos, o.N, D, o.K, dx, st);
   else

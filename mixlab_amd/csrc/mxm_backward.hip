@@ -25,6 +25,7 @@
 // deterministic.
 #include <algorithm>
 
+#include "mxm_act_bw.h"
 #include "mxm_kernels.h"
 
 namespace {
@@ -131,7 +132,9 @@ __global__ __launch_bounds__(256) void router_bw_kernel(BackwardArgs a) {
   const int32_t* sp = a.slot_pos + (size_t)n * K;
   // gate gradient of slot k (by slot position when the caller computed them there)
   for (int k = lane; k < K; k += 64) {
-    dgs[wave][k] = a.dgp ? a.dgp[sp[k]] : a.dgates[(size_t)n * K + k];
+    float dg = a.dgp ? a.dgp[sp[k]] : a.dgates[(size_t)n * K + k];
+    for (int c = 1; c < a.dgp_parts; ++c) dg = dg + a.dgp[(size_t)c * a.N * K + sp[k]];
+    dgs[wave][k] = dg;
     tps[wave][k] = p[sel[k]];
   }
   for (int e = lane; e < E; e += 64) add[wave][e] = 0.0f;
@@ -185,14 +188,6 @@ __global__ __launch_bounds__(256) void router_bw_kernel(BackwardArgs a) {
     const int e = lane + 64 * i;
     if (e < E) out[e] = pe[i] * (dp[i] - ps);
   }
-}
-
-__device__ __forceinline__ float gelu_t(float v, float& deriv) {
-  const float c = 0.7978845608f, k = 0.044715f;
-  const float in = c * (v + k * v * v * v);
-  const float t = tanhf(in);
-  deriv = 0.5f * (1.0f + t) + 0.5f * v * (1.0f - t * t) * c * (1.0f + 3.0f * k * v * v);
-  return 0.5f * v * (1.0f + t);
 }
 
 // The hidden unit of one routed row and its derivatives (fp32 flow): h, and
@@ -584,45 +579,6 @@ __global__ __launch_bounds__(256) void dx_fused_one_bf16_kernel(
   }
 }
 
-// dG and dU of one hidden unit from its gate and up projections g, u and dH
-// (fp32; GLU: dG and dU, MLP: dU only).
-__device__ __forceinline__ void act_bw_one(int etype, int act, float slope, float g, float u,
-                                           float dh, float& dg, float& du) {
-  if (etype == MXM_EXPERT_MLP) {
-    float d;
-    switch (act) {
-      case MXM_ACT_SILU: {
-        const float sg = 1.0f / (1.0f + expf(-u));
-        d = sg * (1.0f + u * (1.0f - sg));
-        break;
-      }
-      case MXM_ACT_GELU:
-        (void)gelu_t(u, d);
-        break;
-      case MXM_ACT_RELU:
-        d = u > 0.0f ? 1.0f : 0.0f;
-        break;
-      default: {
-        const float y = u > 0.0f ? u : u * slope;
-        d = 2.0f * y * (u > 0.0f ? 1.0f : slope);
-        break;
-      }
-    }
-    dg = 0.0f;
-    du = dh * d;
-  } else {
-    float a, d;
-    if (etype == MXM_EXPERT_SWIGLU) {
-      a = 1.0f / (1.0f + expf(-g));
-      d = a * (1.0f - a);
-    } else {
-      a = gelu_t(g, d);
-    }
-    dg = dh * u * d;
-    du = dh * a;
-  }
-}
-
 // One workgroup per token n: ddb[n] = bf16(dD[n]); for each slot s = n*K + k
 // at position p = slot_pos[s]: gp[p] = gates[s] and, if dyb is set, dyb[p] =
 // bf16(gates[s] * dD[n]).  V = 4: 4 consecutive d per thread (16-byte dD
@@ -660,112 +616,6 @@ __global__ __launch_bounds__(256) void dy_gate_kernel(const float* __restrict__ 
         *o = mxm_f2bf(g * v[0]);
     }
   }
-}
-
-// One wave per routed row p (4 rows per workgroup), 8 hidden units per lane
-// and step, from the forward's raw bf16 projections gu [N*K, NC] (GLU: NC =
-// 2F, gate and up columns interleaved in groups of 32 as the MFMA family's W1
-// rows; MLP: NC = F, up only): the hidden h = mxm_hidden_fast of them, as the
-// up GEMM's epilogue computes it; the gated hidden gp[p] * h stored to Hg in
-// bf16 (two planes hi and lo = bf16(v - hi) for a split hidden), dW_down's
-// left operand; dH = gp[p] * dhr (dhr = dD W_down^T for the row's token, not
-// yet gated); dG and dU from dH, written to dgu at the columns of g and u in
-// bf16; and the gate gradient dgp[p] = <dhr[p], h[p]> with h as the forward
-// stores it (bf16, or hi + lo when split), summed per lane in f order and
-// then over the wave by a fixed butterfly.
-__global__ __launch_bounds__(256) void act_bw_gated_bf16_kernel(
-    const uint16_t* __restrict__ gu, const uint16_t* __restrict__ dhr,
-    uint16_t* __restrict__ Hg, bool hsplit, const float* __restrict__ gp, int rows, int F,
-    int etype, int act, float slope, uint16_t* __restrict__ dgu, float* __restrict__ dgp) {
-  const int p = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (p >= rows) return;  // (the whole wave)
-  const bool glu = etype != MXM_EXPERT_MLP;
-  const int NC = glu ? 2 * F : F;
-  const float gate = gp[p];
-  float dot = 0.0f;
-  const size_t hstride = hsplit ? 2 * (size_t)F : (size_t)F;
-  // U steps of 8 hidden units per lane: their loads go out together
-  constexpr int U = 4;
-  for (int f0 = lane * 8; f0 < F; f0 += 512 * U) {
-    uint4 hv[U], uv[U], gv[U];
-#pragma unroll
-    for (int j = 0; j < U; ++j) {
-      const int f = min(f0 + 512 * j, F - 8);  // (steps past F reload the last group)
-      const size_t cu = (size_t)p * NC + (glu ? (size_t)(f >> 5) * 64 + 32 + (f & 31) : (size_t)f);
-      hv[j] = *reinterpret_cast<const uint4*>(dhr + (size_t)p * F + f);
-      uv[j] = *reinterpret_cast<const uint4*>(gu + cu);
-      gv[j] = glu ? *reinterpret_cast<const uint4*>(gu + cu - 32) : make_uint4(0u, 0u, 0u, 0u);
-    }
-#pragma unroll
-    for (int j = 0; j < U; ++j) {
-      const int f = f0 + 512 * j;
-      if (f >= F) break;
-      const size_t cu = (size_t)p * NC + (glu ? (size_t)(f >> 5) * 64 + 32 + (f & 31) : (size_t)f);
-      const uint32_t hw[4] = {hv[j].x, hv[j].y, hv[j].z, hv[j].w};
-      const uint32_t uw[4] = {uv[j].x, uv[j].y, uv[j].z, uv[j].w};
-      const uint32_t gw[4] = {gv[j].x, gv[j].y, gv[j].z, gv[j].w};
-      uint32_t og[4], ou[4], xw[4], lw[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float r0 = mxm_u2f(hw[q] << 16), r1 = mxm_u2f(hw[q] & 0xffff0000u);
-        // the hidden as the up epilogue computes it (mxm_hidden_fast on the
-        // bf16 projections), then as stored
-        // (sigmoid-GLU: the one fast sigmoid serves h and the derivative)
-        const bool sw = etype == MXM_EXPERT_SWIGLU;
-        float h[2], sg[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const float gg = glu ? mxm_u2f(t ? gw[q] & 0xffff0000u : gw[q] << 16) : 0.0f;
-          const float uu = mxm_u2f(t ? uw[q] & 0xffff0000u : uw[q] << 16);
-          if (sw) {
-            sg[t] = mxm_sigmoid_fast(gg);
-            h[t] = mxm_rbf_fast(mxm_rbf_fast(sg[t]) * uu);  // as mxm_hidden_fast
-          } else {
-            h[t] = mxm_hidden_fast<true>(glu ? etype : MXM_EXPERT_MLP, act, slope, gg, uu);
-          }
-        }
-        // h as the forward stores it, for the gate gradient
-        float h0 = mxm_rbf_fast(h[0]), h1 = mxm_rbf_fast(h[1]);
-        if (hsplit) {
-          h0 = h0 + mxm_rbf_fast(h[0] - h0);
-          h1 = h1 + mxm_rbf_fast(h[1] - h1);
-        }
-        dot = __builtin_fmaf(r0, h0, dot);
-        dot = __builtin_fmaf(r1, h1, dot);
-        // the gated hidden
-        const float v0 = gate * h[0], v1 = gate * h[1];
-        xw[q] = mxm_pack_bf2_fast(v0, v1);
-        if (hsplit)
-          lw[q] = mxm_pack_bf2_fast(v0 - mxm_u2f(xw[q] << 16), v1 - mxm_u2f(xw[q] & 0xffff0000u));
-        float dg0, du0, dg1, du1;
-        if (sw) {
-          const float u0 = mxm_u2f(uw[q] << 16), u1 = mxm_u2f(uw[q] & 0xffff0000u);
-          const float d0 = gate * r0, d1 = gate * r1;
-          dg0 = d0 * u0 * (sg[0] * (1.0f - sg[0]));
-          du0 = d0 * sg[0];
-          dg1 = d1 * u1 * (sg[1] * (1.0f - sg[1]));
-          du1 = d1 * sg[1];
-        } else {
-          act_bw_one(etype, act, slope, mxm_u2f(gw[q] << 16), mxm_u2f(uw[q] << 16), gate * r0,
-                     dg0, du0);
-          act_bw_one(etype, act, slope, mxm_u2f(gw[q] & 0xffff0000u),
-                     mxm_u2f(uw[q] & 0xffff0000u), gate * r1, dg1, du1);
-        }
-        og[q] = (uint32_t)mxm_f2bf(dg0) | ((uint32_t)mxm_f2bf(dg1) << 16);
-        ou[q] = (uint32_t)mxm_f2bf(du0) | ((uint32_t)mxm_f2bf(du1) << 16);
-      }
-      *reinterpret_cast<uint4*>(dgu + cu) = make_uint4(ou[0], ou[1], ou[2], ou[3]);
-      if (glu) *reinterpret_cast<uint4*>(dgu + cu - 32) = make_uint4(og[0], og[1], og[2], og[3]);
-      *reinterpret_cast<uint4*>(Hg + (size_t)p * hstride + f) = make_uint4(xw[0], xw[1], xw[2], xw[3]);
-      if (hsplit)
-        *reinterpret_cast<uint4*>(Hg + (size_t)p * hstride + F + f) =
-            make_uint4(lw[0], lw[1], lw[2], lw[3]);
-    }
-  }
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) dot = dot + mxm_xor_lane_f(dot, m);
-  if (lane == 0) dgp[p] = dot;
 }
 
 // dx[n] = dxr[n] + sum_k dxe[slot_pos(n, k)] (bf16 rows), k ascending
@@ -1070,15 +920,6 @@ void mxm_launch_dy_gate(const float* dd, const float* gates, const int32_t* slot
   else
     hipLaunchKernelGGL(dy_gate_kernel<1>, dim3(N), dim3(block_for(D, 1)), 0, s, dd, gates,
                        slot_pos, D, K, ddb, dyb, gp);
-}
-
-void mxm_launch_act_bw_gated_bf16(const uint16_t* gu, const uint16_t* dhr, uint16_t* Hg,
-                                  bool hsplit, const float* gp, int rows, int F, int etype, int act,
-                                  float slope, uint16_t* dgu, float* dgp, hipStream_t s) {
-  // F is a multiple of 32 (the MFMA family's GLU interleave)
-  if (rows > 0)
-    hipLaunchKernelGGL(act_bw_gated_bf16_kernel, dim3((rows + 3) / 4), dim3(256), 0, s, gu, dhr,
-                       Hg, hsplit, gp, rows, F, etype, act, slope, dgu, dgp);
 }
 
 void mxm_launch_dx_bf16(const float* dxr, const uint16_t* dxe, const int32_t* slot_pos, int N,

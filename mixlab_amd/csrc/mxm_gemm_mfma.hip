@@ -46,6 +46,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "mxm_act_bw.h"
 #include "mxm_kernels.h"
 
 namespace {
@@ -448,6 +449,88 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] *= scv[j];
   }
+  if constexpr (Epi<EPI>::ACT_BW) {
+    // The activation backward on dH in the accumulators, 32 rows at a time: each
+    // wave stages its 32 x 64 block in LDS and takes 8 hidden units of a row per
+    // lane, whose raw projections are loaded before.  (As a pass of its own over
+    // a stored bf16 dH it read and wrote 0.8 GB: the product and it took 229 us
+    // at 32768 rows of ffn 2048, the product with this epilogue 187.)
+    constexpr bool SW = Epi<EPI>::EPI == EPI_ACT_BW_SW;
+    constexpr int SR = 72;  // floats per staged row: the two half-waves' writes in other banks
+    static_assert(TN == 2 && TL::CW * 32 * SR * 4 <= (int)sizeof(u32x4_t) * NS * BUF, "staging");
+    float* st = reinterpret_cast<float*>(lds) + wave * (32 * SR);
+    const bool glu = SW || a.expert_type != MXM_EXPERT_MLP;
+    const int F = a.Ncols, NC = glu ? 2 * F : F;
+    const int wc = n0 + wn * 64, f = wc + (lane & 7) * 8;
+    const int cu = glu ? (f >> 5) * 64 + 32 + (f & 31) : f;
+    const size_t hstride = a.abw.hsplit ? 2 * (size_t)F : (size_t)F;
+    float* __restrict__ dgp = a.abw.dgp + (size_t)(wc >> 6) * a.rows_total;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int lr0 = wm * TM * 32 + i * 32 + (lane >> 3);
+      auto load = [&](int s, uint4& gv, uint4& uv, float& gate) {
+        const int p = row0 + min(lr0 + 8 * s, rows - 1);  // (rows past the segment: its last)
+        const uint16_t* g = a.abw.gu + (size_t)p * NC + cu;
+        uv = *reinterpret_cast<const uint4*>(g);
+        gv = glu ? *reinterpret_cast<const uint4*>(g - 32) : make_uint4(0u, 0u, 0u, 0u);
+        gate = a.abw.gp[p];
+      };
+      auto apply = [&](int s, uint4 gv, uint4 uv, float gate) {
+        const float4* q = reinterpret_cast<const float4*>(st + (8 * s + (lane >> 3)) * SR +
+                                                          (lane & 7) * 8);
+        const float4 r0 = q[0], r1 = q[1];
+        const float rr[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
+        uint4 og, ou, hw, hl;
+        float dot = 0.0f;
+        act_bw8<SW>(a.expert_type, a.activation, a.slope, a.abw.hsplit, rr, gv, uv, gate, og, ou,
+                    hw, hl, dot);
+        dot = dot + mxm_xor_lane_f(dot, 1);
+        dot = dot + mxm_xor_lane_f(dot, 2);
+        dot = dot + mxm_xor_lane_f(dot, 4);
+        const int lr = lr0 + 8 * s;
+        if (lr < rows) {
+          const size_t p = (size_t)(row0 + lr);
+          uint16_t* o = a.abw.dgu + p * NC + cu;
+          *reinterpret_cast<uint4*>(o) = ou;
+          if (glu) *reinterpret_cast<uint4*>(o - 32) = og;
+          uint16_t* h = a.abw.Hg + p * hstride + f;
+          *reinterpret_cast<uint4*>(h) = hw;
+          if (!SW && a.abw.hsplit) *reinterpret_cast<uint4*>(h + F) = hl;
+          if ((lane & 7) == 0) dgp[p] = dot;
+        }
+      };
+      uint4 gv[4], uv[4];
+      float gate[4];
+      if constexpr (SW) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) load(s, gv[s], uv[s], gate[s]);
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          st[((r >> 2) * 8 + (lane >> 5) * 4 + (r & 3)) * SR + j * 32 + (lane & 31)] = acc[i][j][r];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      if constexpr (SW) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) apply(s, gv[s], uv[s], gate[s]);
+      } else {
+        // (the kinds' code once per block: four copies keep the block loop,
+        // and so the accumulators' indexes, from being unrolled)
+#pragma unroll 1
+        for (int s = 0; s < 4; ++s) {
+          load(s, gv[0], uv[0], gate[0]);
+          apply(s, gv[0], uv[0], gate[0]);
+        }
+      }
+      // this wave's reads are complete before the next block is staged
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_wave_barrier();
+    }
+    return;
+  }
   if constexpr (Epi<EPI>::Y_F32) {
     // y in fp32, straight from the accumulators: register r of lane l holds
     // C[(r/4)*8 + (l/32)*4 + r%4][l%32], so each store instruction writes
@@ -502,7 +585,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
   if constexpr (Epi<EPI>::KEEP_RAW) {
     // the raw bf16 projections (all TN column tiles: gate and up interleaved
     // as W1's rows) to out2, through the same staging with 64 columns per
-    // wave, before the activation overwrites the accumulators
+    // wave, before the activation overwrites the accumulators.  The kept
+    // forwards go on to the hidden from the same accumulators: 188 us at
+    // 32768 rows of ffn 2048, where the projections alone took 172 and a
+    // hidden pass that read them back another 76.
     constexpr int CR = TN * 32;
     static_assert(CR == 64 && CR == CS, "raw staging of 64 columns per wave");
     uint32_t* rst = stage;
@@ -545,7 +631,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
       if (grow + 1 < rows)
         *reinterpret_cast<u32x4_t*>(rout + (size_t)(row0 + grow + 1) * a.Ncols + c0r) = hi;
     }
-    if constexpr (Epi<EPI>::RAW_ONLY) return;  // the backward's activation pass derives H
+    if constexpr (Epi<EPI>::RAW_ONLY) return;  // the backward's hidden-gradient product derives H
     // this wave's reads of the raw staging are complete
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_wave_barrier();
@@ -917,6 +1003,10 @@ void with_epi(const GemmArgs& a, F&& f) {
       f(std::integral_constant<int, EPI_DOWN_F32>{});
     else if (a.f32_out)
       f(std::integral_constant<int, EPI_F32>{});
+    else if (a.abw.dgu && a.expert_type == MXM_EXPERT_SWIGLU)
+      f(std::integral_constant<int, EPI_ACT_BW_SW>{});
+    else if (a.abw.dgu)
+      f(std::integral_constant<int, EPI_ACT_BW>{});
     else
       f(std::integral_constant<int, EPI_DOWN>{});
     return;

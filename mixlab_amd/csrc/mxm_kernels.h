@@ -165,6 +165,21 @@ struct DecodeAux {
 // activation, 2 = down projection.
 enum { MXM_GEMM_GLU = 0, MXM_GEMM_MLP = 1, MXM_GEMM_DOWN = 2 };
 
+// The activation backward fused into the product dH = dD W_down^T of the bf16
+// backward (MXM_GEMM_DOWN over the hidden units, dgu set): dH itself is not
+// stored.  Per routed row p: dG and dU to dgu [rows][NC] in W1's column order,
+// the gated hidden gp[p] * h to Hg (hi, and lo after Ncols columns when hsplit),
+// and the gate gradient <dH, h> over each 64 hidden units to dgp [Ncols / 64]
+// [rows_total].
+struct ActBwArgs {
+  const uint16_t* gu;   // raw bf16 projections [rows][NC]
+  const float* gp;      // [rows] gates by slot position
+  uint16_t* Hg;
+  uint16_t* dgu;
+  float* dgp;
+  bool hsplit;
+};
+
 struct GemmArgs {
   int mode;
   const void* a;          // mode 0/1: x [N, Kd]; mode 2: H [N*K, Kd]
@@ -235,6 +250,7 @@ struct GemmArgs {
   // ... and with daux.aux set, the up projection's launch has one more
   // workgroup that computes aux and entropy
   DecodeAux daux;
+  ActBwArgs abw;
 };
 // Spare bytes at the end of every B matrix buffer given to the SIMT family.
 #define MXM_SIMT_PAD 256
@@ -298,11 +314,11 @@ int mxm_simt_bm(int64_t rows, int E, int ncols, int n_cu);
 // Epilogue kinds: the hidden activation (expert type x activation) of the up
 // projections, or the plain bf16 store of the down projection.
 enum { EPI_SWIGLU, EPI_GEGLU, EPI_MLP_SILU, EPI_MLP_GELU, EPI_MLP_RELU, EPI_MLP_LEAKY, EPI_DOWN,
-       EPI_DOWN_F32, EPI_F32 };
+       EPI_DOWN_F32, EPI_F32, EPI_ACT_BW, EPI_ACT_BW_SW };
 
 // EPI_KEEP + an up-projection kind: the raw bf16 projections to
 // GemmArgs::out2 instead of the hidden (the MFMA backward derives H from
-// them in its activation pass); EPI_KEEP_H + a kind: both.
+// them in its hidden-gradient product); EPI_KEEP_H + a kind: both.
 constexpr int EPI_KEEP = 16;
 constexpr int EPI_KEEP_H = 64;
 // EPI_SCALE + a kind: the accumulators are multiplied by a per-output-column
@@ -318,8 +334,7 @@ struct Epi {
   static constexpr bool RAW_ONLY = (EPI_ & EPI_KEEP) != 0;
   static constexpr bool SCALED = (EPI_ & EPI_SCALE) != 0;
   static constexpr int MODE = EPI <= EPI_GEGLU ? MXM_GEMM_GLU
-                              : (EPI == EPI_DOWN || EPI == EPI_DOWN_F32 || EPI == EPI_F32)
-                                  ? MXM_GEMM_DOWN
+                              : EPI >= EPI_DOWN ? MXM_GEMM_DOWN
                                   : MXM_GEMM_MLP;
   // up projections whose hidden is fp32 in the bf16 flow: H in two planes
   static constexpr bool H_SPLIT = EPI == EPI_GEGLU || EPI == EPI_MLP_GELU || EPI == EPI_MLP_LEAKY;
@@ -328,6 +343,9 @@ struct Epi {
   // the accumulators stored in fp32 (the split down projection's y, or a
   // plain product: GemmArgs::f32_out)
   static constexpr bool Y_F32 = EPI == EPI_DOWN_F32 || EPI == EPI_F32;
+  // dH of the bf16 backward with the activation backward (GemmArgs::abw), for
+  // any kind and for sigmoid-GLU
+  static constexpr bool ACT_BW = EPI == EPI_ACT_BW || EPI == EPI_ACT_BW_SW;
   // a product over pairs of operand planes (GemmArgs::planes)
   static constexpr bool PLANE_PAIRS = EPI == EPI_F32;
   static constexpr int ETYPE = EPI == EPI_SWIGLU ? MXM_EXPERT_SWIGLU
@@ -473,8 +491,9 @@ struct BackwardArgs {
   float d_aux, d_ent;
   // scratch
   float* dy;                 // [N*K, D]: dY = gate * dD by slot position
-  const float* dgp;          // [N*K] gate gradients by slot position (set: the caller computed
-                             // them; dgates is then not used)
+  const float* dgp;          // [dgp_parts][N*K] gate gradients by slot position, in parts to
+                             // be added (set: the caller computed them; dgates is not used)
+  int dgp_parts;
   float *dgates, *dlogits, *dxr;                          // [N*K], [N, E], [N, D] (dxr unset:
                                                           // the caller fuses dx's router term)
   uint16_t* dyb16;           // [N*K, D]: when set, dY is written here in bf16 instead of dy
@@ -513,17 +532,6 @@ void mxm_launch_dwr_halves(const float* t, int D, int E, int Ep, float* dwr, hip
 // gp[p] = gates[s] and (if dyb is set) dyb[p] = bf16(gates[s] * dD[n]).
 void mxm_launch_dy_gate(const float* dd, const float* gates, const int32_t* slot_pos, int N, int D,
                         int K, uint16_t* ddb, uint16_t* dyb, float* gp, hipStream_t s);
-// Per routed row p: the hidden h from the forward's raw bf16
-// projections gu with the up epilogue's own activation code (bit for bit the
-// forward's); the gated hidden gp[p] * h written to Hg (hi, and lo =
-// bf16(v - hi) after F columns when hsplit) for dW_down = Hg^T dD over the
-// slots' tokens; dH = gp[p] * dhr[p] (dhr = dD W_down^T of the row's token,
-// ungated), dG and dU (the activation backward); and the gate gradient
-// dgp[p] = <dhr[p], h[p]> with h as the forward stores it (hi + lo when
-// hsplit).
-void mxm_launch_act_bw_gated_bf16(const uint16_t* gu, const uint16_t* dhr, uint16_t* Hg,
-                                  bool hsplit, const float* gp, int rows, int F, int etype, int act,
-                                  float slope, uint16_t* dgu, float* dgp, hipStream_t s);
 
 // fp32 products on the bf16 MFMA kernels (the fp32 backward): fp32 values as
 // bf16 planes hi = bf16(v), lo = bf16(v - hi), one beside the other, and a
