@@ -68,6 +68,7 @@ __device__ __forceinline__ void lds_vec(const float* p, float (&v)[T]) {
 }
 
 typedef float mf_v16 __attribute__((ext_vector_type(16)));
+typedef float mf_v32 __attribute__((ext_vector_type(32)));
 
 // BM x BN tile, TM x TN outputs per thread (a 16 x 16 thread grid), k tiles
 // of BK.  MF (BM = BN = 64): wave w owns rows 32 (w >> 1) .. + 31 and columns
@@ -234,41 +235,49 @@ __global__ __launch_bounds__(NT) void gemm_simt_kernel(GemmArgs a) {
   }
 }
 
-// The 64 x 64 matrix-core tile on fp32 rows, loads of 4 floats per lane: the
-// element loads of the kernel above are each under a bounds check, a branch
-// apiece in the loop (12 per thread and k tile with GLU), and its fragment reads
-// wait one by one; this one's loop has 2 or 3 unconditional 16-byte loads (4-byte
-// aligned: rows of any length), one barrier per k tile (two LDS buffers) and 8 k
-// steps of fragments read ahead of the 8 being multiplied.  Rows past the
-// segment reload its last one and columns past NC read what follows in the
-// matrix (its buffer ends in MXM_SIMT_PAD spare bytes): neither is stored, and
-// no stored output reads them.  The last k tile of a Kd that is no multiple of
-// 16 is loaded element by element with zeros past Kd.  The same fmaf chains as
-// above, bit for bit.  Bound by the matrix core (k = 1 products at about 140
-// TFLOP/s) and the LDS reads and barriers around it: 16384 tokens of D 512 / E 8
-// / K 2 / ffn 2048 gate+up 1562 -> 1435 us (96 TFLOP/s), down 875 -> 766 us; 4096
-// of ffn 1367 340 -> 306 and 204 -> 184 us.
+// The matrix-core tile of 64 rows x C columns on fp32 rows, loads of 4 floats
+// per lane: the element loads of the kernel above are each under a bounds check,
+// a branch apiece in the loop (12 per thread and k tile with GLU), and its
+// fragment reads wait one by one; this one's loop has 2 to 5 unconditional
+// 16-byte loads (4-byte aligned: rows of any length), one barrier per k tile (two
+// LDS buffers) and 8 k steps of fragments read ahead of the 8 being multiplied.
+// Rows past the segment reload its last one and columns past NC read what follows
+// in the matrix (its buffer ends in MXM_SIMT_PAD spare bytes): neither is stored,
+// and no stored output reads them.  The last k tile of a Kd that is no multiple
+// of 16 is loaded element by element with zeros past Kd.  The same fmaf chains as
+// above, bit for bit.
+// C = 64: a wave's 32 x 32 quarter as four blocks of v_mfma_f32_16x16x1_4b.  C =
+// 128: its 32 x 64 quarter as the two blocks of v_mfma_f32_32x32x1_2b (block b
+// columns 32 b .., both from the same rows), which does twice the products per
+// pair of fragment registers: every register that is read from LDS between
+// products takes issue slots from them.
+// Bound by the matrix core (k = 1 products at about 140 TFLOP/s) and the LDS
+// reads and barriers around it: 16384 tokens of D 512 / E 8 / K 2 / ffn 2048
+// gate+up 1562 us with element loads, 1367 at C = 64, 1263 at C = 128 (109
+// TFLOP/s); down 875, 750 and 691 us.
 typedef float f4_u __attribute__((ext_vector_type(4), aligned(4)));
 
-template <bool BF16, int MODE>
+template <bool BF16, int MODE, int C>
 __global__ __launch_bounds__(NT) void gemm_simt_mf_kernel(GemmArgs a) {
   constexpr int NB = (MODE == MXM_GEMM_GLU) ? 2 : 1;
-  constexpr int T = 64, BK = 16, LD = T + 4;
+  constexpr int T = 64, BK = 16, LD = T + 4, LDC = C + 4;
+  constexpr bool WIDE = C == 128;
+  constexpr int Q = C / 64;  // pieces of B per thread
   constexpr int KG = 8;  // k steps of fragments in flight
   __shared__ __attribute__((aligned(16))) float As[2][BK][LD];
-  __shared__ __attribute__((aligned(16))) float Bs[2][NB][BK][LD];
+  __shared__ __attribute__((aligned(16))) float Bs[2][NB][BK][LDC];
 
   const int mtile = blockIdx.y;
   if (mtile >= a.mstart[a.E]) return;
   const int e = find_expert(a.mstart, a.E, mtile);
   const int row0 = a.offsets[e] + (mtile - a.mstart[e]) * T;
   const int rows = min(T, a.offsets[e + 1] - row0);
-  const int n0 = blockIdx.x * T;
+  const int n0 = blockIdx.x * C;
   const int Kd = a.Kd, NC = a.Ncols;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
 
   // this thread's pieces: A row tid / 4, k 4 (tid % 4) .. + 3 of the k tile;
-  // B k tid / 16, columns 4 (tid % 16) .. + 3
+  // B k tid / 16, columns 4 (tid % 16) .. + 3 of each 64
   const int ar = tid >> 2, ak = (tid & 3) * 4, bk = tid >> 4, bc = (tid & 15) * 4;
   const int p = row0 + min(ar, rows - 1);
   const float* __restrict__ A =
@@ -278,30 +287,37 @@ __global__ __launch_bounds__(NT) void gemm_simt_mf_kernel(GemmArgs a) {
   for (int b = 0; b < NB; ++b)
     B[b] = static_cast<const float*>(b == 0 ? a.b0 : a.b1) + (size_t)e * Kd * NC +
            (size_t)bk * NC + n0 + bc;
-  f4_u ra, rb[NB];
+  f4_u ra, rb[NB][Q];
   auto fetch = [&](int k0) {
     if (k0 + BK <= Kd) {
       ra = *reinterpret_cast<const f4_u*>(A + k0);
 #pragma unroll
       for (int b = 0; b < NB; ++b)
-        rb[b] = *reinterpret_cast<const f4_u*>(B[b] + (size_t)k0 * NC);
+#pragma unroll
+        for (int j = 0; j < Q; ++j)
+          rb[b][j] = *reinterpret_cast<const f4_u*>(B[b] + (size_t)k0 * NC + 64 * j);
     } else {
 #pragma unroll
       for (int q = 0; q < 4; ++q) ra[q] = k0 + ak + q < Kd ? A[k0 + q] : 0.0f;
 #pragma unroll
       for (int b = 0; b < NB; ++b)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          rb[b][q] = k0 + bk < Kd && n0 + bc + q < NC ? B[b][(size_t)k0 * NC + q] : 0.0f;
+        for (int j = 0; j < Q; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            rb[b][j][q] = k0 + bk < Kd && n0 + bc + 64 * j + q < NC
+                              ? B[b][(size_t)k0 * NC + 64 * j + q]
+                              : 0.0f;
     }
   };
 
-  mf_v16 acc[NB];
+  using acc_t = typename std::conditional<WIDE, mf_v32, mf_v16>::type;
+  acc_t acc[NB];
 #pragma unroll
-  for (int b = 0; b < NB; ++b) acc[b] = mf_v16{};
-  const int wr0 = 32 * (wave >> 1), wc0 = 32 * (wave & 1);
-  const int arow_l = wr0 + 16 * ((lane >> 4) >> 1) + (lane & 15);
-  const int bcol_l = wc0 + 16 * ((lane >> 4) & 1) + (lane & 15);
+  for (int b = 0; b < NB; ++b) acc[b] = acc_t{};
+  const int wr0 = 32 * (wave >> 1), wc0 = C / 2 * (wave & 1);
+  const int arow_l = wr0 + (WIDE ? lane & 31 : 16 * ((lane >> 4) >> 1) + (lane & 15));
+  const int bcol_l = wc0 + (WIDE ? lane : 16 * ((lane >> 4) & 1) + (lane & 15));
   fetch(0);
   int buf = 0;
   for (int k0 = 0; k0 < Kd; k0 += BK, buf ^= 1) {
@@ -309,7 +325,9 @@ __global__ __launch_bounds__(NT) void gemm_simt_mf_kernel(GemmArgs a) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) As[buf][ak + q][ar] = ra[q];
 #pragma unroll
-    for (int b = 0; b < NB; ++b) *reinterpret_cast<f4_u*>(&Bs[buf][b][bk][bc]) = rb[b];
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int j = 0; j < Q; ++j) *reinterpret_cast<f4_u*>(&Bs[buf][b][bk][bc + 64 * j]) = rb[b][j];
     __syncthreads();
     if (k0 + BK < Kd) fetch(k0 + BK);
     float av[2][KG], bv[2][NB][KG];
@@ -330,15 +348,20 @@ __global__ __launch_bounds__(NT) void gemm_simt_mf_kernel(GemmArgs a) {
 #pragma unroll
       for (int k = 0; k < KG; ++k)
 #pragma unroll
-        for (int b = 0; b < NB; ++b)
-          acc[b] = __builtin_amdgcn_mfma_f32_16x16x1f32(av[g][k], bv[g][b][k], acc[b], 0, 0, 0);
+        for (int b = 0; b < NB; ++b) {
+          if constexpr (WIDE)
+            acc[b] = __builtin_amdgcn_mfma_f32_32x32x1f32(av[g][k], bv[g][b][k], acc[b], 0, 0, 0);
+          else
+            acc[b] = __builtin_amdgcn_mfma_f32_16x16x1f32(av[g][k], bv[g][b][k], acc[b], 0, 0, 0);
+        }
   }
 
   float* out = static_cast<float*>(a.out);
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int row = wr0 + 16 * ((i >> 2) >> 1) + (lane >> 4) * 4 + (i & 3);
-    const int c = n0 + wc0 + 16 * ((i >> 2) & 1) + (lane & 15);
+  for (int i = 0; i < 16 * Q; ++i) {
+    const int row = wr0 + (WIDE ? 8 * ((i & 15) >> 2) + (lane >> 5) * 4 + (i & 3)
+                                : 16 * ((i >> 2) >> 1) + (lane >> 4) * 4 + (i & 3));
+    const int c = n0 + wc0 + (WIDE ? 32 * (i >> 4) + (lane & 31) : 16 * ((i >> 2) & 1) + (lane & 15));
     if (row >= rows || c >= NC) continue;
     float v;
     if (MODE == MXM_GEMM_GLU) {
@@ -355,6 +378,18 @@ __global__ __launch_bounds__(NT) void gemm_simt_mf_kernel(GemmArgs a) {
   }
 }
 
+// Tiles of 128 columns instead of 64 on the matrix cores: where their grid has
+// 1280 workgroups or more (a CU holds three of them at once with GLU, five
+// without), the reduction is long enough for the loop to be the time, and the
+// columns are no more than a sixteenth above those of 64.  On both sides of
+// the line, 64 / 128 columns: grids of 8320 and 2080 above; 1496 workgroups (k
+// 512) 274 / 254 us, 1152 200 / 202, 544 163 / 170, 528 (k 128) 35.8 / 39.5;
+// 1848 with 7.7 % more columns 113 / 115.
+bool mf_wide(const GemmArgs& a) {
+  const int64_t c64 = (a.Ncols + 63) / 64, c128 = (a.Ncols + 127) / 128;
+  return a.Kd >= 256 && 32 * c128 <= 17 * c64 && c128 * a.max_mtiles >= 1280;
+}
+
 // k tiles of 16 for the 64 x 64 tile (each thread's 16 outputs per k step
 // amortise the tile's barriers), 32 for the 32 x 32 tile (4 outputs per k
 // step: half as many barrier and LDS round trips per k)
@@ -366,10 +401,15 @@ void launch_t(const GemmArgs& a, hipStream_t s) {
     constexpr int MODE = decltype(mode)::value;
     // (the down projection's rows, H, are fp32 in either flow)
     using T2 = typename std::conditional<MODE == MXM_GEMM_DOWN, float, TA>::type;
-    if constexpr (MF && sizeof(T2) == 4)
-      hipLaunchKernelGGL((gemm_simt_mf_kernel<BF16, MODE>), grid, dim3(NT), 0, s, a);
-    else
+    if constexpr (MF && sizeof(T2) == 4) {
+      const dim3 wide((a.Ncols + 127) / 128, a.max_mtiles);
+      if (mf_wide(a))
+        hipLaunchKernelGGL((gemm_simt_mf_kernel<BF16, MODE, 128>), wide, dim3(NT), 0, s, a);
+      else
+        hipLaunchKernelGGL((gemm_simt_mf_kernel<BF16, MODE, 64>), grid, dim3(NT), 0, s, a);
+    } else {
       hipLaunchKernelGGL((gemm_simt_kernel<T2, BF16, MODE, T, T, BK, MF>), grid, dim3(NT), 0, s, a);
+    }
   };
   switch (a.mode) {
     case MXM_GEMM_GLU:

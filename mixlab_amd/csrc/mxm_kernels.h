@@ -253,7 +253,7 @@ struct GemmArgs {
   ActBwArgs abw;
 };
 // Spare bytes at the end of every B matrix buffer given to the SIMT family.
-#define MXM_SIMT_PAD 256
+#define MXM_SIMT_PAD 512
 // SIMT family: weights in the reference layout (x . W, [in, out]) per expert,
 // fp32 storage; H and Y are fp32.  Accumulation is fmaf in ascending k.
 void mxm_launch_gemm_simt(const GemmArgs& a, bool bf16, hipStream_t s);

@@ -28,3 +28,19 @@ def test_simt_tile_edges(gpu_lib, monkeypatch, N, D, E, K, F, etype):
     want = run_oracle(x, wr, experts, K=K, expert_type=etype, activation=act)
     assert same_bits(delta, want["delta"])
     assert same_bits(delta[:-1], got[0][:-1])
+
+
+@pytest.mark.parametrize("N,D,E,K,F,etype", [
+    (9100, 380, 4, 3, 382, 0), (9100, 383, 3, 3, 321, 2), (7000, 257, 5, 4, 640, 1)])
+def test_simt_wide_tile(gpu_lib, monkeypatch, N, D, E, K, F, etype):
+    """The 128-column tile (large grids): column and reduction remainders, rows
+    past a segment, against the vector-unit tile bit for bit."""
+    x, wr, experts = random_case(N + D + F, N, D, E, F, expert_type=etype, wscale=0.1)
+    x[-1] = np.nan
+    got = []
+    for mf in ("1", "0"):
+        monkeypatch.setenv("MXM_SIMT_MFMA", mf)
+        got.append(run_gpu(x, wr, experts, B=1, T=N, K=K, expert_type=etype,
+                           activation=1 if etype else 0)[0])
+    assert np.isfinite(got[0][:-1]).all() and np.isnan(got[0][-1]).all()
+    assert same_bits(got[0][:-1], got[1][:-1])
