@@ -21,6 +21,7 @@
 // router, scan and scatter; see below).  Both kernels run the per-token
 // softmax / top-k / gate code of route_token, so their routing is the same
 // bit for bit.
+#include <algorithm>
 #include <type_traits>
 
 #include "mxm_kernels.h"
@@ -705,16 +706,17 @@ __global__ __launch_bounds__(NT) void router_kernel(RouterArgs a) {
                                   blockIdx.x * (TM / TT) + sub, a);
 }
 
-// Decode-sized batches: routing in one launch.  Workgroup n owns token n.
-// Its x row is staged in LDS as fp32, zero-padded to whole 64-d chunks.  The
+// Decode-sized batches: routing in one launch.  Workgroup n owns token n, or
+// tokens 4 n .. 4 n + 3 in larger batches (launch_route_small_t): each weight
+// then serves four fmaf chains.  The x rows are staged in LDS as fp32, zero-padded to whole 64-d chunks.  The
 // logits follow the chunked summation order of mxm_numerics.h, so the bits
 // are those of the tiled kernel: the waves of an expert group (one expert per
 // lane) compute chunk partials in rounds, each an fmaf chain from +0 with x
-// broadcast from LDS, and the group's first wave adds them in chunk order.
-// The router weights are a copy in the flow's dtype, lane-interleaved (each
+// broadcast from LDS, and the group's first T waves add them in chunk order,
+// a token each.  The router weights are a copy in the flow's dtype, lane-interleaved (each
 // wave load is 1 KB contiguous: 16 bytes = the lane's expert's next 4 or 8 d),
-// and the next pieces are in flight while a chunk is summed.  Wave 0 then
-// runs route_token and writes the token's picks, gates, probabilities and
+// and the next pieces are in flight while a chunk is summed.  A wave per
+// token then runs route_token and writes the token's picks, gates, probabilities and
 // entropy term.  Every workgroup then takes a ticket (wave 0: agent-scope
 // fence, atomic add); the one that takes the last ticket reads all tokens'
 // results back and computes what the scan and scatter kernels compute for
@@ -887,36 +889,43 @@ __device__ __forceinline__ void route_dispatch_body(const RouteSmallArgs& a, int
   }
 }
 
-template <typename TX, bool BF16, int NJ, bool VEC>
+template <typename TX, bool BF16, int NJ, bool VEC, int T>
 __global__ __launch_bounds__(RS_NT, 1) void route_small_kernel(RouteSmallArgs a) {
   extern __shared__ __attribute__((aligned(16))) float rs_dyn[];  // x row, then the slots
-  __shared__ float lg[NJ * 64];
-  __shared__ float rs_part[RS_PART_FLOATS];  // a round's chunk partials [RPC][NJ * 64]
-  __shared__ __attribute__((aligned(16))) RankScratch rank_scr;
+  __shared__ float lg[T][NJ * 64];
+  __shared__ float rs_part[RS_PART_FLOATS];  // a round's chunk partials [T][RPC][NJ * 64]
+  __shared__ __attribute__((aligned(16))) RankScratch rank_scr[T];
   __shared__ int cnt[MXM_MAX_EXPERTS];
   __shared__ int offs[MXM_MAX_EXPERTS];
   __shared__ int runc[MXM_MAX_EXPERTS];
   __shared__ uint32_t msk[MXM_MAX_EXPERTS][2];
   __shared__ int s_last;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int n = blockIdx.x;
+  const int n0 = blockIdx.x * T;
   const int N = a.N, D = a.D, E = a.E, K = a.K;
 
-  // ---- the token's x row -> LDS (fp32) ----------------------------------
-  const TX* xrow = static_cast<const TX*>(a.x) + (size_t)n * D;
-  float* xl = rs_dyn;
-  if (VEC) {
-    constexpr int PER = 16 / sizeof(TX);
-    for (int i = tid; i < D / PER; i += RS_NT) {
-      const uint4 raw = *reinterpret_cast<const uint4*>(xrow + i * PER);
-      float f[PER];
-      unpack16<TX>(raw, f);
+  // ---- the tokens' x rows -> LDS (fp32); past N the last one again ---------
+  const int Dp = (D + MXM_LOGIT_CHUNK - 1) / MXM_LOGIT_CHUNK * MXM_LOGIT_CHUNK;
+  float* xl = rs_dyn;  // [T][Dp]
 #pragma unroll
-      for (int q = 0; q < PER; q += 4)
-        *reinterpret_cast<float4*>(xl + i * PER + q) = make_float4(f[q], f[q + 1], f[q + 2], f[q + 3]);
+  for (int t = 0; t < T; ++t) {
+    const TX* xrow = static_cast<const TX*>(a.x) + (size_t)min(n0 + t, N - 1) * D;
+    float* xt = xl + t * Dp;
+    if (VEC) {
+      constexpr int PER = 16 / sizeof(TX);
+      for (int i = tid; i < D / PER; i += RS_NT) {
+        const uint4 raw = *reinterpret_cast<const uint4*>(xrow + i * PER);
+        float f[PER];
+        unpack16<TX>(raw, f);
+#pragma unroll
+        for (int q = 0; q < PER; q += 4)
+          *reinterpret_cast<float4*>(xt + i * PER + q) = make_float4(f[q], f[q + 1], f[q + 2], f[q + 3]);
+      }
+    } else {
+      for (int d = tid; d < D; d += RS_NT) xt[d] = ld_as_f32<TX>(xrow + d);
     }
-  } else {
-    for (int d = tid; d < D; d += RS_NT) xl[d] = ld_as_f32<TX>(xrow + d);
+    // zeros up to whole 64-d chunks (the padded weights are zero too)
+    for (int d = D + tid; d < Dp; d += RS_NT) xt[d] = 0.0f;
   }
   // the dispatch's counters (used by the last workgroup only)
   for (int e = tid; e < E; e += RS_NT) {
@@ -925,10 +934,6 @@ __global__ __launch_bounds__(RS_NT, 1) void route_small_kernel(RouteSmallArgs a)
     msk[e][0] = 0u;
     msk[e][1] = 0u;
   }
-  // zeros up to whole 64-d chunks (the padded weights are zero too)
-  for (int d = D + tid; d < (D + MXM_LOGIT_CHUNK - 1) / MXM_LOGIT_CHUNK * MXM_LOGIT_CHUNK;
-       d += RS_NT)
-    xl[d] = 0.0f;
   __syncthreads();
 
   // ---- logits ---------------------------------------------------------------
@@ -939,7 +944,7 @@ __global__ __launch_bounds__(RS_NT, 1) void route_small_kernel(RouteSmallArgs a)
   // weight pieces through a register ring of RS_RING items (an item is 32
   // registers of pieces: one bf16 chunk or half an fp32 chunk; the next item
   // is in flight while one is summed), and parks each chunk's partial in LDS.
-  // After the round's barrier the group's first wave adds the partials in
+  // After the round's barrier the group's first T waves add a token's partials in
   // chunk order.
   {
     constexpr int WPG = RS_WAVES / NJ;                  // waves per expert group
@@ -947,8 +952,8 @@ __global__ __launch_bounds__(RS_NT, 1) void route_small_kernel(RouteSmallArgs a)
     constexpr int PPC = MXM_LOGIT_CHUNK / PER;          // pieces per chunk (8 or 16)
     constexpr int IP = 8;                               // pieces per item
     constexpr int IPC = PPC / IP;                       // items per chunk (1 or 2)
-    constexpr int RPC = RS_PART_FLOATS / (NJ * 64);     // chunks per round
-    static_assert(PPC % IP == 0 && RPC >= WPG, "items and rounds");
+    constexpr int RPC = RS_PART_FLOATS / (NJ * 64 * T); // chunks per round
+    static_assert(PPC % IP == 0 && RPC >= WPG && WPG >= T, "items and rounds");
     // wave-uniform values in scalar registers, so every condition below is a
     // scalar branch and the loads sit outside divergent control flow
     const int swave = __builtin_amdgcn_readfirstlane(wave);
@@ -958,7 +963,8 @@ __global__ __launch_bounds__(RS_NT, 1) void route_small_kernel(RouteSmallArgs a)
     // this lane's piece p of chunk c: wlane + (c * PPC + p) * 64 * PER
     const TX* wlane = static_cast<const TX*>(a.wr_t) +
                       ((size_t)(active ? g : 0) * (a.ldw / PER) * 64 + lane) * PER;
-    float* part_lds = rs_part + g * 64 + lane;  // chunk i of the round at i * NJ * 64
+    // token t's chunk i of the round at (t * RPC + i) * NJ * 64
+    float* part_lds = rs_part + g * 64 + lane;
     float acc = 0.0f;
     for (int r0 = 0; r0 < nchunks; r0 += RPC) {
       const int rc = min(RPC, nchunks - r0);               // chunks in this round
@@ -985,7 +991,7 @@ __global__ __launch_bounds__(RS_NT, 1) void route_small_kernel(RouteSmallArgs a)
         for (int q = 0; q < IP; ++q)
           ring[S()][q] = *reinterpret_cast<const uint4*>(p + (size_t)q * 64 * PER);
       };
-      float part = 0.0f;
+      float part[T] = {};
       auto step = [&](auto S, int it) {
         load(std::integral_constant<int, (S() + RS_RING - 1) % RS_RING>{}, it + RS_RING - 1);
         if (it < nit) {
@@ -996,11 +1002,17 @@ __global__ __launch_bounds__(RS_NT, 1) void route_small_kernel(RouteSmallArgs a)
             float w[PER];
             unpack16<TX>(ring[S()][q], w);
 #pragma unroll
-            for (int t = 0; t < PER; ++t) part = __builtin_fmaf(xc[q * PER + t], w[t], part);
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+              for (int v = 0; v < PER; ++v)
+                part[t] = __builtin_fmaf(xc[t * Dp + q * PER + v], w[v], part[t]);
           }
           if (h == IPC - 1) {
-            part_lds[i * NJ * 64] = part;
-            part = 0.0f;
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+              part_lds[(t * RPC + i) * NJ * 64] = part[t];
+              part[t] = 0.0f;
+            }
           }
         }
       };
@@ -1013,23 +1025,24 @@ __global__ __launch_bounds__(RS_NT, 1) void route_small_kernel(RouteSmallArgs a)
         }
       }
       __syncthreads();
-      if (active && sub == 0) {
-        for (int i = 0; i < rc; ++i) acc = acc + part_lds[i * NJ * 64];
+      if (active && sub < T) {
+        for (int i = 0; i < rc; ++i) acc = acc + part_lds[(sub * RPC + i) * NJ * 64];
       }
       if (r0 + RPC < nchunks) __syncthreads();  // the next round reuses the partials
     }
-    if (active && sub == 0) lg[g * 64 + lane] = BF16 ? mxm_rbf(acc) : acc;
+    if (active && sub < T) lg[sub][g * 64 + lane] = BF16 ? mxm_rbf(acc) : acc;
   }
   __syncthreads();
 
   // ---- softmax, top-k, gates ---------------------------------------------
-  if (wave == 0) {
+  const int n = n0 + wave;  // wave t < T: token n0 + t
+  if (wave < T && n < N) {
     float v[NJ];
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) v[j] = lg[lane + 64 * j];
+    for (int j = 0; j < NJ; ++j) v[j] = lg[wave][lane + 64 * j];
     float p[NJ], pick_g[NJ];
     int pick_e[NJ];
-    const float ent = route_token<BF16, NJ>(v, lane, E, K, p, pick_e, pick_g, &rank_scr);
+    const float ent = route_token<BF16, NJ>(v, lane, E, K, p, pick_e, pick_g, &rank_scr[wave]);
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       const int e = lane + 64 * j;
@@ -1047,10 +1060,13 @@ __global__ __launch_bounds__(RS_NT, 1) void route_small_kernel(RouteSmallArgs a)
   if (!a.dispatch) return;
 
   // ---- ticket: the last workgroup continues --------------------------------
-  // Wave 0 wrote all of this token's results, so it alone releases them; in
+  // Wave 0 wrote all of a single token's results, so it alone releases them
+  // (several tokens': after a barrier that orders the other waves' stores
+  // before its release); in
   // the last workgroup wave 0 alone acquires the others' (the caches it
   // invalidates are the CU's and the XCD's, shared by the workgroup's waves,
   // and the barrier orders the other waves' reads after it).
+  if (T > 1) __syncthreads();
   if (wave == 0) {
     __threadfence();
     if (lane == 0) s_last = atomicAdd(a.ticket, 1) == (int)gridDim.x - 1;
@@ -1068,14 +1084,28 @@ template <typename TX, bool BF16, int NJ>
 void launch_route_small_t(const RouteSmallArgs& a, hipStream_t s) {
   constexpr int PER = 16 / (int)sizeof(TX);
   const bool vec = a.D % PER == 0 && (reinterpret_cast<uintptr_t>(a.x) % 16) == 0;
-  size_t lds = (size_t)(a.D + MXM_LOGIT_CHUNK - 1) / MXM_LOGIT_CHUNK * MXM_LOGIT_CHUNK * 4;
+  const size_t row = (size_t)(a.D + MXM_LOGIT_CHUNK - 1) / MXM_LOGIT_CHUNK * MXM_LOGIT_CHUNK * 4;
   const size_t slots = (size_t)a.N * a.K * 4;
-  if (slots > lds) lds = slots;
-  lds = (lds + 15) / 16 * 16;
-  if (vec)
-    hipLaunchKernelGGL((route_small_kernel<TX, BF16, NJ, true>), dim3(a.N), dim3(RS_NT), lds, s, a);
+  auto go = [&](auto tok) {
+    constexpr int T = decltype(tok)::value;
+    const size_t lds = (std::max(T * row, slots) + 15) / 16 * 16;
+    const dim3 grid((a.N + T - 1) / T);
+    if (vec)
+      hipLaunchKernelGGL((route_small_kernel<TX, BF16, NJ, true, T>), grid, dim3(RS_NT), lds, s, a);
+    else
+      hipLaunchKernelGGL((route_small_kernel<TX, BF16, NJ, false, T>), grid, dim3(RS_NT), lds, s, a);
+  };
+  // Four tokens per workgroup past one workgroup per CU (the registers allow one
+  // at a time), where single tokens run in several rounds, each workgroup with
+  // its ticket, and each reads all of the router's weights: whole forwards of
+  // small experts, 1 / 4 tokens: E 8 / D 512 at 256 37.7 / 36.3 us, 257 40.4 /
+  // 36.4, 512 52.8 / 44.4, 1024 83.7 / 63.2; E 64 / D 2048 at 256 53.0 / 53.7, 257
+  // 58.6 / 54.2, 1024 111 / 85; E 256 / D 1024 at 256 83 / 89, 320 102 / 98, 1024
+  // 194 / 165.  Their rows (fp32) and partials take up to 75 KB of LDS.
+  if (a.N > 256 && 4 * row <= 49152)
+    go(std::integral_constant<int, 4>{});
   else
-    hipLaunchKernelGGL((route_small_kernel<TX, BF16, NJ, false>), dim3(a.N), dim3(RS_NT), lds, s, a);
+    go(std::integral_constant<int, 1>{});
 }
 
 template <typename TX, bool BF16>
