@@ -708,13 +708,13 @@ __global__ __launch_bounds__(NT) void router_kernel(RouterArgs a) {
 
 // Decode-sized batches: routing in one launch.  Workgroup n owns token n, or
 // tokens 4 n .. 4 n + 3 in larger batches (launch_route_small_t): each weight
-// then serves four fmaf chains.  The x rows are staged in LDS as fp32, zero-padded to whole 64-d chunks.  The
-// logits follow the chunked summation order of mxm_numerics.h, so the bits
+// then serves four fmaf chains.  The x rows are staged in LDS as fp32,
+// zero-padded to whole 64-d chunks.  The logits follow the chunked summation order of mxm_numerics.h, so the bits
 // are those of the tiled kernel: the waves of an expert group (one expert per
 // lane) compute chunk partials in rounds, each an fmaf chain from +0 with x
 // broadcast from LDS, and the group's first T waves add them in chunk order,
-// a token each.  The router weights are a copy in the flow's dtype, lane-interleaved (each
-// wave load is 1 KB contiguous: 16 bytes = the lane's expert's next 4 or 8 d),
+// a token each.  The router weights are a copy in the flow's dtype,
+// lane-interleaved (each wave load is 1 KB contiguous: 16 bytes = the lane's expert's next 4 or 8 d),
 // and the next pieces are in flight while a chunk is summed.  A wave per
 // token then runs route_token and writes the token's picks, gates, probabilities and
 // entropy term.  Every workgroup then takes a ticket (wave 0: agent-scope
