@@ -1060,13 +1060,17 @@ __global__ __launch_bounds__(RS_NT, 1) void route_small_kernel(RouteSmallArgs a)
   if (!a.dispatch) return;
 
   // ---- ticket: the last workgroup continues --------------------------------
-  // Wave 0 wrote all of a single token's results, so it alone releases them
-  // (several tokens': after a barrier that orders the other waves' stores
-  // before its release); in
-  // the last workgroup wave 0 alone acquires the others' (the caches it
-  // invalidates are the CU's and the XCD's, shared by the workgroup's waves,
-  // and the barrier orders the other waves' reads after it).
-  if (T > 1) __syncthreads();
+  // Every wave that wrote a token's results releases them itself before the
+  // ticket (a barrier orders LDS, it does not wait for other waves' stores to
+  // global memory: without their own fence they may still be on their way when
+  // wave 0's ticket is seen).  In the last workgroup wave 0 alone acquires the
+  // others' (the caches it invalidates are the CU's and the XCD's, shared by
+  // the workgroup's waves, and the barrier orders the other waves' reads after
+  // it).
+  if (T > 1) {
+    if (wave < T) __threadfence();
+    __syncthreads();
+  }
   if (wave == 0) {
     __threadfence();
     if (lane == 0) s_last = atomicAdd(a.ticket, 1) == (int)gridDim.x - 1;
@@ -1101,7 +1105,9 @@ void launch_route_small_t(const RouteSmallArgs& a, hipStream_t s) {
   // small experts, 1 / 4 tokens: E 8 / D 512 at 256 37.7 / 36.3 us, 257 40.4 /
   // 36.4, 512 52.8 / 44.4, 1024 83.7 / 63.2; E 64 / D 2048 at 256 53.0 / 53.7, 257
   // 58.6 / 54.2, 1024 111 / 85; E 256 / D 1024 at 256 83 / 89, 320 102 / 98, 1024
-  // 194 / 165.  Their rows (fp32) and partials take up to 75 KB of LDS.
+  // 194 / 165.  Rows (fp32, up to 48 KB here) and the dispatch's slots (up to 64
+  // KB, MXM_SMALL_SLOTS) share the dynamic LDS; with the 30 KB of arrays beside
+  // it a workgroup takes up to 94 of the CU's 160 KB.
   if (a.N > 256 && 4 * row <= 49152)
     go(std::integral_constant<int, 4>{});
   else
