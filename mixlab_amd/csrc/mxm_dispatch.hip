@@ -276,72 +276,76 @@ __global__ __launch_bounds__(256) void combine_wave_kernel(CombineArgs a, int re
   const float sg = __builtin_bit_cast(float, __builtin_amdgcn_ds_permute(r << 2, __builtin_bit_cast(int, g)));
   const TY* __restrict__ y = static_cast<const TY*>(a.y);
   const size_t ldy = a.ldy > 0 ? (size_t)a.ldy : (size_t)D;
-  for (int d = ((wave % WPT) * 64 + lane) * VEC; d < D; d += WPT * 64 * VEC) {
-    float acc[VEC];
+  // D <= WPT * 64 * VEC: each lane has one piece of the row.  Lanes past D take
+  // its last piece again and only leave out the store: the picks are read from
+  // other lanes' registers, which is defined while every lane is active.
+  const int dw = ((wave % WPT) * 64 + lane) * VEC;
+  const int d = min(dw, D - VEC);
+  float acc[VEC];
 #pragma unroll
-    for (int q = 0; q < VEC; ++q) acc[q] = 0.0f;
-    for (int k0 = 0; k0 < K; k0 += KC) {
-      const int kn = min(KC, K - k0);
-      raw_t row[KC];
+  for (int q = 0; q < VEC; ++q) acc[q] = 0.0f;
+  for (int k0 = 0; k0 < K; k0 += KC) {
+    const int kn = min(KC, K - k0);
+    raw_t row[KC];
 #pragma unroll
-      for (int u = 0; u < KC; ++u)
-        if (u < kn)
-          row[u] = __builtin_nontemporal_load(reinterpret_cast<const raw_t*>(
-              y + (size_t)__builtin_amdgcn_readlane(sp, k0 + u) * ldy + d));
+    for (int u = 0; u < KC; ++u)
+      if (u < kn)
+        row[u] = __builtin_nontemporal_load(reinterpret_cast<const raw_t*>(
+            y + (size_t)__builtin_amdgcn_readlane(sp, k0 + u) * ldy + d));
 #pragma unroll
-      for (int u = 0; u < KC; ++u) {
-        if (u < kn) {
-          float f[VEC];
-          if constexpr (sizeof(TY) == 2) {
+    for (int u = 0; u < KC; ++u) {
+      if (u < kn) {
+        float f[VEC];
+        if constexpr (sizeof(TY) == 2) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              f[2 * q] = mxm_u2f(row[u][q] << 16);
-              f[2 * q + 1] = mxm_u2f(row[u][q] & 0xffff0000u);
-            }
-          } else {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) f[q] = row[u][q];
+          for (int q = 0; q < 4; ++q) {
+            f[2 * q] = mxm_u2f(row[u][q] << 16);
+            f[2 * q + 1] = mxm_u2f(row[u][q] & 0xffff0000u);
           }
-          const float gk = mxm_u2f(__builtin_amdgcn_readlane(mxm_f2u(sg), k0 + u));
+        } else {
 #pragma unroll
-          for (int q = 0; q < VEC; ++q) acc[q] = __fadd_rn(acc[q], __fmul_rn(f[q], gk));
+          for (int q = 0; q < 4; ++q) f[q] = row[u][q];
         }
+        const float gk = mxm_u2f(__builtin_amdgcn_readlane(mxm_f2u(sg), k0 + u));
+#pragma unroll
+        for (int q = 0; q < VEC; ++q) acc[q] = __fadd_rn(acc[q], __fmul_rn(f[q], gk));
       }
     }
-    if (a.resid) {
-      // block level: x + delta (* moe_scale), fp32
-      const size_t i0 = (size_t)n * D + d;
-      float xr[VEC];
-      if (resid_vec && !a.resid_bf16) {
-#pragma unroll
-        for (int q = 0; q < VEC; q += 4) {
-          const vf4 t = *reinterpret_cast<const vf4*>(static_cast<const float*>(a.resid) + i0 + q);
-#pragma unroll
-          for (int w = 0; w < 4; ++w) xr[q + w] = t[w];
-        }
-      } else {
-#pragma unroll
-        for (int q = 0; q < VEC; ++q)
-          xr[q] = a.resid_bf16 ? mxm_bf2f(static_cast<const uint16_t*>(a.resid)[i0 + q])
-                               : static_cast<const float*>(a.resid)[i0 + q];
-      }
-#pragma unroll
-      for (int q = 0; q < VEC; ++q) {
-        float v = acc[q];
-        if (a.rscale) {
-          const float sc = a.rscale_bf16 ? mxm_bf2f(static_cast<const uint16_t*>(a.rscale)[d + q])
-                                         : static_cast<const float*>(a.rscale)[d + q];
-          v = __fmul_rn(v, sc);
-        }
-        acc[q] = __fadd_rn(xr[q], v);
-      }
-    }
-    float* dst = a.delta + (size_t)n * D + d;
-#pragma unroll
-    for (int q = 0; q < VEC; q += 4)
-      __builtin_nontemporal_store(vf4{acc[q], acc[q + 1], acc[q + 2], acc[q + 3]},
-                                  reinterpret_cast<vf4*>(dst + q));
   }
+  if (a.resid) {
+    // block level: x + delta (* moe_scale), fp32
+    const size_t i0 = (size_t)n * D + d;
+    float xr[VEC];
+    if (resid_vec && !a.resid_bf16) {
+#pragma unroll
+      for (int q = 0; q < VEC; q += 4) {
+        const vf4 t = *reinterpret_cast<const vf4*>(static_cast<const float*>(a.resid) + i0 + q);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) xr[q + w] = t[w];
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < VEC; ++q)
+        xr[q] = a.resid_bf16 ? mxm_bf2f(static_cast<const uint16_t*>(a.resid)[i0 + q])
+                             : static_cast<const float*>(a.resid)[i0 + q];
+    }
+#pragma unroll
+    for (int q = 0; q < VEC; ++q) {
+      float v = acc[q];
+      if (a.rscale) {
+        const float sc = a.rscale_bf16 ? mxm_bf2f(static_cast<const uint16_t*>(a.rscale)[d + q])
+                                       : static_cast<const float*>(a.rscale)[d + q];
+        v = __fmul_rn(v, sc);
+      }
+      acc[q] = __fadd_rn(xr[q], v);
+    }
+  }
+  if (dw >= D) return;
+  float* dst = a.delta + (size_t)n * D + d;
+#pragma unroll
+  for (int q = 0; q < VEC; q += 4)
+    __builtin_nontemporal_store(vf4{acc[q], acc[q + 1], acc[q + 2], acc[q + 3]},
+                                reinterpret_cast<vf4*>(dst + q));
 }
 
 template <typename TY, int VEC>
