@@ -788,6 +788,18 @@ struct SchedLds {
   int wsum[2][MXM_MAX_EXPERTS / 64];
 };
 
+// Inclusive prefix sum over the wave (lanes past a row's or the wave's start
+// add 0): row shifts, then the rows' last lanes broadcast on.
+__device__ __forceinline__ int wave_prefix(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return v;
+}
+
 // Prefixes of the experts' row tiles of BM rows: (count + rnd) / BM big ones,
 // and a small one for rows left over (rnd = BM - 1 leaves none).
 template <int BM>
@@ -797,15 +809,7 @@ __device__ __forceinline__ void sched_build(SchedLds& S, const int32_t* offsets,
   const int o0 = tid < E ? offsets[tid] : 0;
   const int o1 = tid < E ? offsets[tid + 1] : 0;
   const int nb = (o1 - o0 + rnd) / BM, ns = o1 - o0 > nb * BM ? 1 : 0;
-  int ib = nb, is = ns;
-#pragma unroll
-  for (int sh = 1; sh < 64; sh <<= 1) {
-    const int vb = __shfl_up(ib, sh, 64), vs = __shfl_up(is, sh, 64);
-    if (lane >= sh) {
-      ib += vb;
-      is += vs;
-    }
-  }
+  int ib = wave_prefix(nb), is = wave_prefix(ns);
   if (lane == 63 && wave < MXM_MAX_EXPERTS / 64) {
     S.wsum[0][wave] = ib;
     S.wsum[1][wave] = is;
@@ -943,10 +947,27 @@ template <class TL, int BM, int BN, int WM, int WN, int EPI>
 __global__ __launch_bounds__(TL::NT, TL::WPS * 256 / TL::NT) void gemm_kernel(GemmArgs a) {
   __shared__ u32x4_t lds[TL::NS * TL::BUF];
   __shared__ SchedLds S;
-  const int E = a.E;
-  sched_build<BM>(S, a.offsets, E, BM - 1);
+  const int E = a.E, lane = threadIdx.x & 63;
   auto uni = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
-  const int BR = uni(S.big[E]), ncol = a.Ncols / BN;
+  // up to 64 experts: their row tiles in each wave's lanes (lane e: expert e),
+  // so that a tile's rows are known without LDS or a barrier.  These launches
+  // are often short, and what stands before the first load is part of each:
+  // 200 tokens of D 192 / E 4 / K 2 / ffn 256, 6.4 and 7.1 us for the two
+  // products from LDS prefixes with the whole device's workgroups launched,
+  // 5.7 and 5.7 like this with tile_grid's.
+  const bool lanes = E <= 64;
+  int o0 = 0, o1 = 0, pre = 0;
+  if (lanes) {
+    if (lane < E) {
+      o0 = a.offsets[lane];
+      o1 = a.offsets[lane + 1];
+    }
+    pre = wave_prefix((o1 - o0 + BM - 1) / BM);
+  } else {
+    sched_build<BM>(S, a.offsets, E, BM - 1);
+  }
+  const int BR = lanes ? __builtin_amdgcn_readlane(pre, 63) : uni(S.big[E]);
+  const int ncol = a.Ncols / BN;
   const int64_t T = (int64_t)BR * ncol;
   const int xcd = blockIdx.x & 7, s = blockIdx.x >> 3, W = gridDim.x >> 3;
   const int lo = (int)(T * xcd / 8), hi = (int)(T * (xcd + 1) / 8);
@@ -954,10 +975,18 @@ __global__ __launch_bounds__(TL::NT, TL::WPS * 256 / TL::NT) void gemm_kernel(Ge
     if (p != lo + s) asm volatile("s_barrier" ::: "memory");  // as above
     int mt, nt;
     sched_place(p, BR, ncol, mt, nt);
-    const int e = uni(sched_find(S.big, E, mt));
-    const int row0 = uni(S.off[e] + (mt - S.big[e]) * BM);
-    gemm_tile<TL, BM, BN, WM, WN, EPI>(a, lds, e, row0, min(BM, uni(S.off[e + 1]) - row0),
-                                       nt * BN);
+    int e, row0, rend;
+    if (lanes) {
+      e = __popcll(__ballot(pre <= mt));  // (lanes past E hold BR > mt)
+      row0 = __builtin_amdgcn_readlane(o0, e) +
+             (mt - (e > 0 ? __builtin_amdgcn_readlane(pre, e - 1) : 0)) * BM;
+      rend = __builtin_amdgcn_readlane(o1, e);
+    } else {
+      e = uni(sched_find(S.big, E, mt));
+      row0 = uni(S.off[e] + (mt - S.big[e]) * BM);
+      rend = uni(S.off[e + 1]);
+    }
+    gemm_tile<TL, BM, BN, WM, WN, EPI>(a, lds, e, row0, min(BM, rend - row0), nt * BN);
   }
 }
 
@@ -976,6 +1005,14 @@ static int persistent_grid(int per_cu) {
     ncu[dev] = n;
   }
   return std::max(8, ncu[dev] * per_cu / 8 * 8);
+}
+
+// ... but no more workgroups than the launch can have tiles (an expert's last
+// tile may be partial), in eights for the XCDs.
+static int tile_grid(const GemmArgs& a, int per_cu, int bm, int bn) {
+  const int64_t row_tiles = a.rows_total / bm + std::min(a.E, a.rows_total);
+  const int64_t tiles = row_tiles * ((a.Ncols + bn - 1) / bn);
+  return (int)std::min<int64_t>(persistent_grid(per_cu), (tiles + 7) / 8 * 8);
 }
 
 // Calls f with the epilogue kind of these arguments as a constant: an up
@@ -1036,15 +1073,16 @@ void launch_family(const GemmArgs& a, hipStream_t s) {
   static_assert(per_cu == 2, "two workgroups per CU");
   with_epi(a, [&](auto epi) {
     hipLaunchKernelGGL((gemm_kernel<TL, BM, BN, WM, WN, decltype(epi)::value>),
-                       dim3(persistent_grid(per_cu)), dim3(TL::NT), 0, s, a);
+                       dim3(tile_grid(a, per_cu, BM, BN)), dim3(TL::NT), 0, s, a);
   });
 }
 
-// The scheduled kernel: one workgroup per CU.  whole: 256 x 256 tiles only.
+// The scheduled kernel: one workgroup per CU, or per 128 x 128 tile (its list
+// is no longer than theirs).  whole: 256 x 256 tiles only.
 void launch_sched(const GemmArgs& a, hipStream_t s, int whole) {
   with_epi(a, [&](auto epi) {
-    hipLaunchKernelGGL((gemm_sched_kernel<decltype(epi)::value>), dim3(persistent_grid(1)),
-                       dim3(512), 0, s, a, whole);
+    hipLaunchKernelGGL((gemm_sched_kernel<decltype(epi)::value>),
+                       dim3(tile_grid(a, 1, 128, 128)), dim3(512), 0, s, a, whole);
   });
 }
 
