@@ -1543,7 +1543,6 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
   abw.Hg = static_cast<uint16_t*>(o.ws.H);
   abw.dgu = dgub;
   abw.dgp = o.bw_dgp.as<float>();
-  abw.hsplit = o.hsplit;
   product(ddb, o.bw_w2o.p, nullptr, D, Fk, true, &abw);
   // the router part from those gate gradients
   BackwardArgs br = b;

@@ -54,14 +54,16 @@ __device__ __forceinline__ void act_bw_one(int etype, int act, float slope, floa
 // 8 hidden units of one routed row of the bf16 flow: r = (dD W_down^T) ungated,
 // gv / uv the raw bf16 gate and up projections (gv unused for a plain mlp).
 //   h    as the up epilogue computes it (mxm_hidden_fast of the projections);
-//        dot += <r, h as the forward stores it> (hi + lo when hsplit)
+//        dot += <r, h as the forward stores it> (hi + lo for a split hidden)
 //   hw   gate * h in bf16, hl = bf16(gate * h - that) for a split hidden
 //   og, ou  dG and dU in bf16, from dH = gate * r
-// SW: sigmoid-GLU (the one fast sigmoid serves h and the derivative).
-template <bool SW>
-__device__ __forceinline__ void act_bw8(int etype, int act, float slope, bool hsplit,
-                                        const float (&r)[8], uint4 gv, uint4 uv, float gate,
-                                        uint4& og, uint4& ou, uint4& hw, uint4& hl, float& dot) {
+// KIND: the up projection's epilogue kind (sigmoid-GLU: the one fast sigmoid
+// serves h and the derivative).
+template <int KIND>
+__device__ __forceinline__ void act_bw8(float slope, const float (&r)[8], uint4 gv, uint4 uv,
+                                        float gate, uint4& og, uint4& ou, uint4& hw, uint4& hl,
+                                        float& dot) {
+  using EK = Epi<KIND>;
   const uint32_t uw[4] = {uv.x, uv.y, uv.z, uv.w}, gw[4] = {gv.x, gv.y, gv.z, gv.w};
   uint32_t o1[4], o2[4], xw[4], lw[4];
 #pragma unroll
@@ -73,17 +75,17 @@ __device__ __forceinline__ void act_bw8(int etype, int act, float slope, bool hs
       const float uu = mxm_u2f(t ? uw[q] & 0xffff0000u : uw[q] << 16);
       const float rr = r[2 * q + t], d = gate * rr;
       float h;
-      if constexpr (SW) {
+      if constexpr (KIND == EPI_SWIGLU) {
         const float sg = mxm_sigmoid_fast(gg);
         h = mxm_rbf_fast(mxm_rbf_fast(sg) * uu);  // as mxm_hidden_fast
         dg[t] = d * uu * (sg * (1.0f - sg));
         du[t] = d * sg;
       } else {
-        h = mxm_hidden_fast<true>(etype, act, slope, gg, uu);
-        act_bw_one(etype, act, slope, gg, uu, d, dg[t], du[t]);
+        h = mxm_hidden_fast<true>(EK::ETYPE, EK::ACT, slope, gg, uu);
+        act_bw_one(EK::ETYPE, EK::ACT, slope, gg, uu, d, dg[t], du[t]);
       }
       float hs = mxm_rbf_fast(h);
-      if (!SW && hsplit) hs = hs + mxm_rbf_fast(h - hs);
+      if constexpr (EK::H_SPLIT) hs = hs + mxm_rbf_fast(h - hs);
       dot = __builtin_fmaf(rr, hs, dot);
       v[t] = gate * h;
     }

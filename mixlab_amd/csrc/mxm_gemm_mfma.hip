@@ -454,16 +454,23 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
     // wave stages its 32 x 64 block in LDS and takes 8 hidden units of a row per
     // lane, whose raw projections are loaded before.  (As a pass of its own over
     // a stored bf16 dH it read and wrote 0.8 GB: the product and it took 229 us
-    // at 32768 rows of ffn 2048, the product with this epilogue 187.)
-    constexpr bool SW = Epi<EPI>::EPI == EPI_ACT_BW_SW;
+    // at 32768 rows of ffn 2048, the product with this epilogue 187.)  Each
+    // kind has its code, and a block's projections are requested together: with
+    // the kind looked up at run time and one request after the other, 18000
+    // rows of ffn 512 took 66.5 us for a plain silu, 59.2 for geglu; 29.0 and
+    // 42.2 like this.
+    constexpr int KIND = Epi<EPI>::BW_KIND;
+    constexpr bool glu = Epi<KIND>::MODE == MXM_GEMM_GLU, split = Epi<KIND>::H_SPLIT;
+    // kinds with a tanh: the code of 8 rows once per block (four copies keep
+    // the block loop, and so the accumulators' indexes, from being unrolled)
+    constexpr bool ONCE = Epi<KIND>::ACT == MXM_ACT_GELU;
     constexpr int SR = 72;  // floats per staged row: the two half-waves' writes in other banks
     static_assert(TN == 2 && TL::CW * 32 * SR * 4 <= (int)sizeof(u32x4_t) * NS * BUF, "staging");
     float* st = reinterpret_cast<float*>(lds) + wave * (32 * SR);
-    const bool glu = SW || a.expert_type != MXM_EXPERT_MLP;
     const int F = a.Ncols, NC = glu ? 2 * F : F;
     const int wc = n0 + wn * 64, f = wc + (lane & 7) * 8;
     const int cu = glu ? (f >> 5) * 64 + 32 + (f & 31) : f;
-    const size_t hstride = a.abw.hsplit ? 2 * (size_t)F : (size_t)F;
+    const size_t hstride = split ? 2 * (size_t)F : (size_t)F;
     float* __restrict__ dgp = a.abw.dgp + (size_t)(wc >> 6) * a.rows_total;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
@@ -482,8 +489,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
         const float rr[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
         uint4 og, ou, hw, hl;
         float dot = 0.0f;
-        act_bw8<SW>(a.expert_type, a.activation, a.slope, a.abw.hsplit, rr, gv, uv, gate, og, ou,
-                    hw, hl, dot);
+        act_bw8<KIND>(a.slope, rr, gv, uv, gate, og, ou, hw, hl, dot);
         dot = dot + mxm_xor_lane_f(dot, 1);
         dot = dot + mxm_xor_lane_f(dot, 2);
         dot = dot + mxm_xor_lane_f(dot, 4);
@@ -495,16 +501,14 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
           if (glu) *reinterpret_cast<uint4*>(o - 32) = og;
           uint16_t* h = a.abw.Hg + p * hstride + f;
           *reinterpret_cast<uint4*>(h) = hw;
-          if (!SW && a.abw.hsplit) *reinterpret_cast<uint4*>(h + F) = hl;
+          if (split) *reinterpret_cast<uint4*>(h + F) = hl;
           if ((lane & 7) == 0) dgp[p] = dot;
         }
       };
       uint4 gv[4], uv[4];
       float gate[4];
-      if constexpr (SW) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) load(s, gv[s], uv[s], gate[s]);
-      }
+      for (int s = 0; s < 4; ++s) load(s, gv[s], uv[s], gate[s]);
 #pragma unroll
       for (int r = 0; r < 16; ++r)
 #pragma unroll
@@ -513,16 +517,19 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if constexpr (SW) {
+      if constexpr (!ONCE) {
 #pragma unroll
         for (int s = 0; s < 4; ++s) apply(s, gv[s], uv[s], gate[s]);
       } else {
-        // (the kinds' code once per block: four copies keep the block loop,
-        // and so the accumulators' indexes, from being unrolled)
 #pragma unroll 1
         for (int s = 0; s < 4; ++s) {
-          load(s, gv[0], uv[0], gate[0]);
           apply(s, gv[0], uv[0], gate[0]);
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            gv[q] = gv[q + 1];
+            uv[q] = uv[q + 1];
+            gate[q] = gate[q + 1];
+          }
         }
       }
       // this wave's reads are complete before the next block is staged
@@ -1015,6 +1022,25 @@ static int tile_grid(const GemmArgs& a, int per_cu, int bm, int bn) {
   return (int)std::min<int64_t>(persistent_grid(per_cu), (tiles + 7) / 8 * 8);
 }
 
+// Calls f with the hidden activation's kind of these arguments as a constant.
+template <class F>
+void with_kind(const GemmArgs& a, F&& f) {
+  switch (mxm_epi_kind(a.expert_type, a.activation)) {
+    case EPI_GEGLU:
+      return f(std::integral_constant<int, EPI_GEGLU>{});
+    case EPI_MLP_SILU:
+      return f(std::integral_constant<int, EPI_MLP_SILU>{});
+    case EPI_MLP_GELU:
+      return f(std::integral_constant<int, EPI_MLP_GELU>{});
+    case EPI_MLP_RELU:
+      return f(std::integral_constant<int, EPI_MLP_RELU>{});
+    case EPI_MLP_LEAKY:
+      return f(std::integral_constant<int, EPI_MLP_LEAKY>{});
+    default:
+      return f(std::integral_constant<int, EPI_SWIGLU>{});
+  }
+}
+
 // Calls f with the epilogue kind of these arguments as a constant: an up
 // projection may keep its raw projections (GemmArgs::out2), and weights may
 // be int8 integers with per-column scales (scale0).
@@ -1040,28 +1066,15 @@ void with_epi(const GemmArgs& a, F&& f) {
       f(std::integral_constant<int, EPI_DOWN_F32>{});
     else if (a.f32_out)
       f(std::integral_constant<int, EPI_F32>{});
-    else if (a.abw.dgu && a.expert_type == MXM_EXPERT_SWIGLU)
-      f(std::integral_constant<int, EPI_ACT_BW_SW>{});
     else if (a.abw.dgu)
-      f(std::integral_constant<int, EPI_ACT_BW>{});
+      with_kind(a, [&](auto kind) {
+        f(std::integral_constant<int, EPI_ACT_BW + decltype(kind)::value>{});
+      });
     else
       f(std::integral_constant<int, EPI_DOWN>{});
     return;
   }
-  switch (mxm_epi_kind(a.expert_type, a.activation)) {
-    case EPI_GEGLU:
-      return up(std::integral_constant<int, EPI_GEGLU>{});
-    case EPI_MLP_SILU:
-      return up(std::integral_constant<int, EPI_MLP_SILU>{});
-    case EPI_MLP_GELU:
-      return up(std::integral_constant<int, EPI_MLP_GELU>{});
-    case EPI_MLP_RELU:
-      return up(std::integral_constant<int, EPI_MLP_RELU>{});
-    case EPI_MLP_LEAKY:
-      return up(std::integral_constant<int, EPI_MLP_LEAKY>{});
-    default:
-      return up(std::integral_constant<int, EPI_SWIGLU>{});
-  }
+  with_kind(a, up);
 }
 
 template <int BM, int BN, int WM, int WN, int WPS, int NSTG, int BKK>

@@ -168,7 +168,8 @@ enum { MXM_GEMM_GLU = 0, MXM_GEMM_MLP = 1, MXM_GEMM_DOWN = 2 };
 // The activation backward fused into the product dH = dD W_down^T of the bf16
 // backward (MXM_GEMM_DOWN over the hidden units, dgu set): dH itself is not
 // stored.  Per routed row p: dG and dU to dgu [rows][NC] in W1's column order,
-// the gated hidden gp[p] * h to Hg (hi, and lo after Ncols columns when hsplit),
+// the gated hidden gp[p] * h to Hg (hi, and lo after Ncols columns for kinds
+// with a split hidden),
 // and the gate gradient <dH, h> over each 64 hidden units to dgp [Ncols / 64]
 // [rows_total].
 struct ActBwArgs {
@@ -177,7 +178,6 @@ struct ActBwArgs {
   uint16_t* Hg;
   uint16_t* dgu;
   float* dgp;
-  bool hsplit;
 };
 
 struct GemmArgs {
@@ -314,7 +314,7 @@ int mxm_simt_bm(int64_t rows, int E, int ncols, int n_cu);
 // Epilogue kinds: the hidden activation (expert type x activation) of the up
 // projections, or the plain bf16 store of the down projection.
 enum { EPI_SWIGLU, EPI_GEGLU, EPI_MLP_SILU, EPI_MLP_GELU, EPI_MLP_RELU, EPI_MLP_LEAKY, EPI_DOWN,
-       EPI_DOWN_F32, EPI_F32, EPI_ACT_BW, EPI_ACT_BW_SW };
+       EPI_DOWN_F32, EPI_F32, EPI_ACT_BW /* + an up projection's kind */ };
 
 // EPI_KEEP + an up-projection kind: the raw bf16 projections to
 // GemmArgs::out2 instead of the hidden (the MFMA backward derives H from
@@ -343,9 +343,10 @@ struct Epi {
   // the accumulators stored in fp32 (the split down projection's y, or a
   // plain product: GemmArgs::f32_out)
   static constexpr bool Y_F32 = EPI == EPI_DOWN_F32 || EPI == EPI_F32;
-  // dH of the bf16 backward with the activation backward (GemmArgs::abw), for
-  // any kind and for sigmoid-GLU
-  static constexpr bool ACT_BW = EPI == EPI_ACT_BW || EPI == EPI_ACT_BW_SW;
+  // dH of the bf16 backward with the activation backward (GemmArgs::abw) of an
+  // up projection's kind
+  static constexpr bool ACT_BW = EPI >= EPI_ACT_BW;
+  static constexpr int BW_KIND = ACT_BW ? EPI - EPI_ACT_BW : 0;
   // a product over pairs of operand planes (GemmArgs::planes)
   static constexpr bool PLANE_PAIRS = EPI == EPI_F32;
   static constexpr int ETYPE = EPI == EPI_SWIGLU ? MXM_EXPERT_SWIGLU
