@@ -1489,7 +1489,7 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
     o.bw_w1u.alloc((size_t)E * D * NC * 2);
     o.bw_ddb.alloc((size_t)o.N * D * 2);
     o.bw_gp.alloc(NK * 4);
-    o.bw_dgp.alloc((size_t)(Fk / 64) * NK * 4);
+    o.bw_dgp.alloc((size_t)mxm_dgp_stride(Fk) * NK * 4);
   }
   if (!o.bw_wbf_ready) {
     for (int e = 0; e < E; ++e) {
@@ -1548,6 +1548,7 @@ void run_backward_mfma(MoeOp& o, const void* xb, const BackwardArgs& b, float* d
   BackwardArgs br = b;
   br.dgp = o.bw_dgp.as<float>();
   br.dgp_parts = Fk / 64;
+  br.dgp_stride = mxm_dgp_stride(Fk);
   br.dwr_by_caller = dwr_mfma;
   mxm_launch_backward_router(br, st);
   HIPCK(hipGetLastError());

@@ -471,7 +471,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
     const int wc = n0 + wn * 64, f = wc + (lane & 7) * 8;
     const int cu = glu ? (f >> 5) * 64 + 32 + (f & 31) : f;
     const size_t hstride = split ? 2 * (size_t)F : (size_t)F;
-    float* __restrict__ dgp = a.abw.dgp + (size_t)(wc >> 6) * a.rows_total;
+    const int dgs = mxm_dgp_stride(F);
+    float* __restrict__ dgp = a.abw.dgp + (wc >> 6);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int lr0 = wm * TM * 32 + i * 32 + (lane >> 3);
@@ -502,7 +503,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
           uint16_t* h = a.abw.Hg + p * hstride + f;
           *reinterpret_cast<uint4*>(h) = hw;
           if (split) *reinterpret_cast<uint4*>(h + F) = hl;
-          if ((lane & 7) == 0) dgp[p] = dot;
+          if ((lane & 7) == 0) dgp[p * dgs] = dot;
         }
       };
       uint4 gv[4], uv[4];

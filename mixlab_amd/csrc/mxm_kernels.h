@@ -170,8 +170,10 @@ enum { MXM_GEMM_GLU = 0, MXM_GEMM_MLP = 1, MXM_GEMM_DOWN = 2 };
 // stored.  Per routed row p: dG and dU to dgu [rows][NC] in W1's column order,
 // the gated hidden gp[p] * h to Hg (hi, and lo after Ncols columns for kinds
 // with a split hidden),
-// and the gate gradient <dH, h> over each 64 hidden units to dgp [Ncols / 64]
-// [rows_total].
+// and the gate gradient <dH, h> over each 64 hidden units to dgp [rows]
+// [mxm_dgp_stride(Ncols)], a row's parts side by side for the one lane that adds
+// them up.
+inline __host__ __device__ int mxm_dgp_stride(int Ncols) { return (Ncols / 64 + 3) / 4 * 4; }
 struct ActBwArgs {
   const uint16_t* gu;   // raw bf16 projections [rows][NC]
   const float* gp;      // [rows] gates by slot position
@@ -492,9 +494,10 @@ struct BackwardArgs {
   float d_aux, d_ent;
   // scratch
   float* dy;                 // [N*K, D]: dY = gate * dD by slot position
-  const float* dgp;          // [dgp_parts][N*K] gate gradients by slot position, in parts to
-                             // be added (set: the caller computed them; dgates is not used)
-  int dgp_parts;
+  const float* dgp;          // [N*K][dgp_stride] gate gradients by slot position, dgp_parts of
+                             // each to be added (set: the caller computed them; dgates is not
+                             // used; the stride a multiple of 4)
+  int dgp_parts, dgp_stride;
   float *dgates, *dlogits, *dxr;                          // [N*K], [N, E], [N, D] (dxr unset:
                                                           // the caller fuses dx's router term)
   uint16_t* dyb16;           // [N*K, D]: when set, dY is written here in bf16 instead of dy
