@@ -1136,10 +1136,16 @@ int64_t mxm_moe_create(const float* float_params, int n_float_params, const int3
     if (const char* v = std::getenv("MXM_SMALL_ROUTE"))
       o->small_route = std::atoi(v) != 0 && mxm_route_small_fits(o->N, o->D, o->E, o->K);
     // Tiles of 16 tokens, their reduction split over the workgroup's waves,
-    // up to MXM_ROUTER_SPLIT_N tokens (mxm_router.hip).  Their four times as
-    // many histograms must not take an op past the scratch of the
-    // no-allocation forward that fits it with tiles of 64.
-    if (o->N <= MXM_ROUTER_SPLIT_N) {
+    // up to MXM_ROUTER_SPLIT_N tokens (mxm_router.hip), for the rows that the
+    // matrix cores take: whole 16-byte pieces, in x or in its padded copy (the
+    // vector unit's workgroups own 64 tokens, and four tiles one after the
+    // other only add barriers and histograms: 1100 rows of D 127 / E 4 17.0 us,
+    // 12.8 as one tile).  Their four times as many histograms must not take an
+    // op past the scratch of the no-allocation forward that fits it with tiles
+    // of 64.
+    const bool pieces =
+        o->D % (o->bf16 ? 8 : 4) == 0 || ((o->mfma || o->q8) && o->Kx != o->D);
+    if (o->N <= MXM_ROUTER_SPLIT_N && pieces) {
       o->tile_tokens = 16;
       set_schedule(*o);
       if (layout_workspace(*o, nullptr).bytes > (size_t)MXM_NOALLOC_MAX_BYTES)

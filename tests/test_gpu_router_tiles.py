@@ -57,3 +57,24 @@ def test_dispatch_of_many_tiles(gpu_lib):
     assert_routing_equal(routing, want)
     assert abs(aux - want["aux"]) <= 1e-5 * abs(want["aux"])
     assert abs(ent - want["entropy"]) <= 1e-4 * abs(want["entropy"])
+
+
+@pytest.mark.parametrize("N,D,dtype,tile", [
+    (1100, 127, "fp32", 64), (1100, 128, "fp32", 16), (1500, 130, "bf16", 16),
+    (1500, 65, "bf16", 64), (16385, 128, "fp32", 64)])
+def test_tile_tokens(gpu_lib, N, D, dtype, tile):
+    """Tiles of 16 tokens only for rows that the matrix cores take (whole 16-byte
+    pieces of x, or of its padded copy for the matrix-core experts)."""
+    bf16 = dtype == "bf16"
+    E, K, F = 6, 2, 16 if D == 65 else 128
+    x, wr, experts = random_case(N + D, N, D, E, F)
+    if bf16:
+        x, wr = round_bf16(x), round_bf16(wr)
+        experts = [[round_bf16(w) for w in ws] for ws in experts]
+    _, aux, ent, routing, info = run_gpu(x, wr, experts, B=1, T=N, K=K, bf16=bf16)
+    assert info["route_flow"] == 0 and info["router_tiles"] == -(-N // tile)
+    want = run_oracle(x, wr, experts, K=K, bf16=bf16, rows=np.arange(4, dtype=np.int32))
+    assert_routing_equal(routing, want)
+    # fp32 sums of N probabilities (bf16: the means rounded to bf16, 2^-9)
+    assert abs(aux - want["aux"]) <= (1e-2 if bf16 else 1e-5) * abs(want["aux"])
+    assert abs(ent - want["entropy"]) <= 1e-4 * abs(want["entropy"])
