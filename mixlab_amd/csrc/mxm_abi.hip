@@ -186,6 +186,7 @@ struct MoeOp {
 
   // tile schedule of the forward (set at create from the op's parameters)
   int tile_tokens = MXM_ROUTER_TM;  // of the tiled router
+  bool dispatch_groups = true;      // its dispatch may keep sums over groups of tiles
   int ntiles = 0, bm1 = 0, bm2 = 0, max_mtiles1 = 0, max_mtiles2 = 0;
   int simt_tile = 0;  // MXM_SIMT_TILE at creation: the SIMT family's tile (0 picks)
   int simt_vec = 0;   // MXM_SIMT_MFMA=0 at creation: 64 x 64 SIMT tiles on the vector unit
@@ -400,7 +401,7 @@ Workspace layout_workspace(const MoeOp& o, char* base) {
   w.tile_counts = reinterpret_cast<int32_t*>(take(E * T * 4));
   w.tile_psum = reinterpret_cast<float*>(take(E * T * 4));
   w.tile_ent = reinterpret_cast<float*>(take(T * 4));
-  if (const size_t G = (size_t)mxm_dispatch_groups(o.ntiles, o.E)) {
+  if (const size_t G = o.dispatch_groups ? (size_t)mxm_dispatch_groups(o.ntiles, o.E) : 0) {
     w.group_counts = reinterpret_cast<int32_t*>(take(E * G * 4));
     w.group_psum = reinterpret_cast<float*>(take(E * G * 4));
     w.group_ent = reinterpret_cast<float*>(take(G * 4));
@@ -1145,14 +1146,21 @@ int64_t mxm_moe_create(const float* float_params, int n_float_params, const int3
     // of 64.
     const bool pieces =
         o->D % (o->bf16 ? 8 : 4) == 0 || ((o->mfma || o->q8) && o->Kx != o->D);
-    if (o->N <= MXM_ROUTER_SPLIT_N && pieces) {
-      o->tile_tokens = 16;
+    auto fits = [&] {
       set_schedule(*o);
-      if (layout_workspace(*o, nullptr).bytes > (size_t)MXM_NOALLOC_MAX_BYTES)
-        o->tile_tokens = MXM_ROUTER_TM;
-      set_schedule(*o);
-      if (layout_workspace(*o, nullptr).bytes > (size_t)MXM_NOALLOC_MAX_BYTES)
-        o->tile_tokens = 16;  // past it either way
+      return layout_workspace(*o, nullptr).bytes <= (size_t)MXM_NOALLOC_MAX_BYTES;
+    };
+    const int tiles = o->N <= MXM_ROUTER_SPLIT_N && pieces ? 16 : MXM_ROUTER_TM;
+    o->tile_tokens = tiles;
+    if (!fits()) {
+      o->tile_tokens = MXM_ROUTER_TM;
+      if (!fits()) {
+        o->dispatch_groups = false;  // (nor may the groups' sums)
+        if (!fits()) {               // past it either way
+          o->tile_tokens = tiles;
+          o->dispatch_groups = true;
+        }
+      }
     }
     set_schedule(*o);
     if (o->small_route || o->mf_router) {

@@ -590,7 +590,7 @@ int mxm_dispatch_groups(int ntiles, int E) {
 }
 
 void mxm_launch_dispatch(const DispatchArgs& a, bool bf16, hipStream_t s) {
-  const int groups = mxm_dispatch_groups(a.ntiles, a.E);
+  const int groups = a.group_counts ? mxm_dispatch_groups(a.ntiles, a.E) : 0;
   if (groups > 0) hipLaunchKernelGGL(dispatch_group_kernel, dim3(groups), dim3(256), 0, s, a);
   // up to 256 workgroups of whole tiles (more past DP_TPW tiles each); tiles
   // per workgroup a power of two, so that one lies within a group

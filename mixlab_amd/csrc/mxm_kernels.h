@@ -126,7 +126,7 @@ struct DispatchArgs {
   int N, E, K, ntiles, tile_tokens;
   int bm1, bm2;         // row-tile heights of the two grouped GEMMs
   // sums over groups of MXM_DISPATCH_GROUP tiles, where the batch has more
-  // than MXM_DISPATCH_TABLE histogram entries (mxm_dispatch_groups)
+  // than MXM_DISPATCH_TABLE histogram entries (mxm_dispatch_groups); null: none
   int32_t* group_counts;  // [groups, E]
   float* group_psum;      // [groups, E]
   float* group_ent;       // [groups]
@@ -142,7 +142,13 @@ struct DispatchArgs {
   float* aux_scaled;    // [1] or null
 };
 #define MXM_DISPATCH_GROUP 32
-#define MXM_DISPATCH_TABLE (1 << 18)
+// Every workgroup of the dispatch reads the whole table, so past this many
+// entries a launch that adds up groups of tiles first costs less.  Forwards of
+// small experts without / with it, by entries: 65536 94 / 101 us (16384 tokens of
+// E 64), 75 / 78 (4096 of E 256), 245 / 252 (65536 of E 64); 131072 100.5 / 93
+// (8192 of E 256), 137 / 129 (16384 of E 128), 234 / 226 (32768 of E 256);
+// 262144 181 / 149 (16384 of E 256).
+#define MXM_DISPATCH_TABLE 98304
 // Groups of tiles whose sums the dispatch keeps (0: it reads the tiles').
 int mxm_dispatch_groups(int ntiles, int E);
 void mxm_launch_dispatch(const DispatchArgs& a, bool bf16, hipStream_t s);

@@ -78,3 +78,18 @@ def test_tile_tokens(gpu_lib, N, D, dtype, tile):
     # fp32 sums of N probabilities (bf16: the means rounded to bf16, 2^-9)
     assert abs(aux - want["aux"]) <= (1e-2 if bf16 else 1e-5) * abs(want["aux"])
     assert abs(ent - want["entropy"]) <= 1e-4 * abs(want["entropy"])
+
+
+@pytest.mark.parametrize("N,E", [(6144, 256), (6145, 256), (16384, 100), (16383, 97)])
+def test_dispatch_groups_of_small_tiles(gpu_lib, N, E):
+    """Both sides of the line from which the dispatch reads sums over groups of
+    tiles, with tiles of 16 tokens and a last group of one or of all its tiles."""
+    D, K, F = 8, 3, 8
+    x, wr, experts = random_case(N + E, N, D, E, F)
+    wr = wr * np.float32(20.0)
+    _, aux, ent, routing, info = run_gpu(x, wr, experts, B=1, T=N, K=K)
+    assert info["router_tiles"] == -(-N // 16)
+    want = run_oracle(x, wr, experts, K=K, rows=np.arange(4, dtype=np.int32))
+    assert_routing_equal(routing, want)
+    assert abs(aux - want["aux"]) <= 1e-5 * abs(want["aux"])  # fp32 sums of N terms
+    assert abs(ent - want["entropy"]) <= 1e-4 * abs(want["entropy"])
