@@ -317,15 +317,21 @@ __device__ __forceinline__ void route_tile_seg(const float* lg, int wave, int la
 // A wave computes 16 tokens x 16 G experts (G = 1, 2, 4).  The blocks take
 // the G groups of 16 experts and 4 / G chunks at once, each block its own
 // chunk's chain: lane l works on token l % 16, expert group b % G (b = l / 16)
-// and chunk c + b / G, and holds those operands itself.  Register 4 b + q of
-// lane l of the result is token (l / 16) * 4 + q, expert l % 16 of its group,
-// so a token's partials of the round's chunks are in one lane, in registers.
+// and chunk c + b / G, and holds those operands itself -- except that at G = 4
+// all blocks take the same tokens at the same d, so lane group b holds only
+// the b-th 8 of each 32 d and the instruction broadcasts a group's operand to
+// all blocks (each lane its own copy of x: the router of 16384 tokens of D 1024
+// / E 256 in fp32 171 us, of 65536 of D 2048 / E 64 in bf16 258; 125 and 237
+// like this).  Register 4 b + q of lane l of the result is
+// token (l / 16) * 4 + q, expert l % 16 of its group, so a token's partials of
+// the round's chunks are in one lane, in registers.
 typedef float mxm_lg16 __attribute__((ext_vector_type(16)));
 
-template <typename TX>
+template <typename TX, int G>
 struct LgHalf {  // 32 d of a chunk
   static constexpr int P = 16 / (int)sizeof(TX);  // values per 16-byte piece
-  uint4 xu[32 / P];
+  static constexpr int XD = G == 4 ? 8 : 32;      // of x's in this lane
+  uint4 xu[XD / P];
   uint4 wu[32 / P];
 };
 
@@ -351,40 +357,54 @@ struct LgSrc {
   __amdgpu_buffer_rsrc_t xs, ws;
   int xoff;   // this lane's token row
   int woff;   // this lane's expert
+  int xd;     // its first x of each 32 d
   int D;
 };
 
-// d0 .. d0 + 31 of the lane's token and expert.  x pieces at or past D (its columns, D % P
-// == 0, so a piece is wholly in or out) take an offset past the records and
-// tokens past N lie past them, so both load as zeros; the router copy is
-// zero from D to its end, past which its pieces load as zeros too.
-template <typename TX>
-__device__ __forceinline__ void lg_load(LgHalf<TX>& R, const LgSrc<TX>& S, int d0) {
-  constexpr int P = LgHalf<TX>::P;
+// d0 .. d0 + 31 of the lane's expert, and of its token (or the lane group's 8 of
+// them).  x pieces at or past D (its columns, D % P == 0, so a piece is wholly
+// in or out) take an offset past the records and tokens past N lie past them,
+// so both load as zeros; the router copy is zero from D to its end, past which
+// its pieces load as zeros too.
+template <typename TX, int G>
+__device__ __forceinline__ void lg_load(LgHalf<TX, G>& R, const LgSrc<TX>& S, int d0) {
+  using H = LgHalf<TX, G>;
+  constexpr int P = H::P;
 #pragma unroll
   for (int h = 0; h < 32 / P; ++h) {
-    const int d = d0 + P * h;
-    const int off = d < S.D ? S.xoff + d * (int)sizeof(TX) : LG_OUT_OF_RANGE;
-    const lg_u4 v = __builtin_amdgcn_raw_buffer_load_b128(S.xs, off, 0, 0);
-    R.xu[h] = make_uint4(v.x, v.y, v.z, v.w);
-    const lg_u4 w = __builtin_amdgcn_raw_buffer_load_b128(S.ws, S.woff + (d / P) * 1024, 0, 0);
+    if (h < H::XD / P) {
+      const int d = d0 + S.xd + P * h;
+      const int off = d < S.D ? S.xoff + d * (int)sizeof(TX) : LG_OUT_OF_RANGE;
+      const lg_u4 v = __builtin_amdgcn_raw_buffer_load_b128(S.xs, off, 0, 0);
+      R.xu[h] = make_uint4(v.x, v.y, v.z, v.w);
+    }
+    const lg_u4 w = __builtin_amdgcn_raw_buffer_load_b128(S.ws, S.woff + (d0 / P + h) * 1024, 0, 0);
     R.wu[h] = make_uint4(w.x, w.y, w.z, w.w);
   }
 }
 
 // The 32 d in ascending order; FIRST starts the chunk partials at +0.
-template <typename TX, bool FIRST>
-__device__ __forceinline__ void lg_half(const LgHalf<TX>& R, mxm_lg16& c) {
-  constexpr int P = LgHalf<TX>::P;
+template <typename TX, int G, bool FIRST>
+__device__ __forceinline__ void lg_half(const LgHalf<TX, G>& R, mxm_lg16& c) {
+  using H = LgHalf<TX, G>;
+  constexpr int P = H::P;
+  if constexpr (FIRST) c = mxm_lg16{};
+  auto step = [&](auto group) {
+    constexpr int B = decltype(group)::value;  // d 8 B .. 8 B + 7
 #pragma unroll
-  for (int t = 0; t < 32; ++t) {
-    const float a = lg_val<TX>(R.xu[t / P], t % P);
-    const float b = lg_val<TX>(R.wu[t / P], t % P);
-    if (FIRST && t == 0)
-      c = __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, mxm_lg16{}, 0, 0, 0);
-    else
-      c = __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, c, 0, 0, 0);
-  }
+    for (int t = 8 * B; t < 8 * B + 8; ++t) {
+      const float b = lg_val<TX>(R.wu[t / P], t % P);
+      const float a = lg_val<TX>(R.xu[t % H::XD / P], t % P);
+      if constexpr (G == 4)
+        c = __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, c, 2, B, 0);
+      else
+        c = __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, c, 0, 0, 0);
+    }
+  };
+  step(std::integral_constant<int, 0>{});
+  step(std::integral_constant<int, 1>{});
+  step(std::integral_constant<int, 2>{});
+  step(std::integral_constant<int, 3>{});
 }
 
 // Sources of a wave for tokens n0w .. n0w + 15 and the experts 64 g .. a
@@ -404,6 +424,7 @@ __device__ __forceinline__ LgSrc<TX> lg_source(const TX* x, int ldx, const TX* w
                                            ldw * 64 * (int)sizeof(TX), LG_RSRC_W3);
   S.xoff = (lane & 15) * ldx * (int)sizeof(TX);
   S.woff = (((lane >> 4) % G) * 16 + (lane & 15)) * 16;
+  S.xd = G == 4 ? 8 * (lane >> 4) : 0;
   S.D = Dx;
   return S;
 }
@@ -531,10 +552,10 @@ __device__ __forceinline__ void route_tile(const float* lg, TileScratch<EP>& sc,
 // EP = 16 G experts, or 64 NP for E > 64 (passes of 64, G = 4).
 // Bound by the chain of rounds (a round of 64 k = 1 products is 2048 clocks of
 // the matrix core) and, in large batches, by the products themselves.
-// Measured, against 64-token tiles on the vector unit (E <= 32) or with 64
-// experts a round from broadcast x: 1999 tokens of D 1024 / E 16 37.5 -> 6.9
-// us, 4096 of D 2048 / E 64 89 -> 34 us, 16384 of D 512 / E 8 24 -> 11 us, 65536
-// of D 1024 / E 16 (tiles of 64) 79 -> 47 us, of D 2048 / E 64 unchanged at 225.
+// Measured, against 64-token tiles on the vector unit (E <= 32) or on 64-token
+// tiles of the matrix cores only: 1999 tokens of D 1024 / E 16 37.5 -> 6.9 us,
+// 4096 of D 2048 / E 64 89 -> 27 us, 16384 of D 512 / E 8 24 -> 11 us, 65536 of
+// D 1024 / E 16 (tiles of 64) 79 -> 47 us, of D 2048 / E 64 the same (222-237).
 template <typename TX, bool BF16, int G, int NP, int TT>
 __global__ __launch_bounds__(NT) void router_mf_kernel(RouterArgs a) {
   constexpr int EP = 16 * G * NP, LGS = EP + 1;
@@ -554,24 +575,24 @@ __global__ __launch_bounds__(NT) void router_mf_kernel(RouterArgs a) {
         static_cast<const TX*>(a.wr_t) + (size_t)pass * a.ldw * 64, a.ldw, a.N, a.Dx,
         n0 + (SPLIT ? 0 : 16 * wave), lane);
     auto d_of = [&](int r, int half) { return ((r * CPR + lc) * 2 + half) * 32; };
-    LgHalf<TX> ra, rb;
+    LgHalf<TX, G> ra, rb;
     mxm_lg16 acc;
     if constexpr (SPLIT) {
       float lgt[G];
 #pragma unroll
       for (int g = 0; g < G; ++g) lgt[g] = 0.0f;
-      lg_load<TX>(ra, S, d_of(wave, 0));
+      lg_load<TX, G>(ra, S, d_of(wave, 0));
       for (int r0 = 0, buf = 0; r0 < nr; r0 += 4, buf ^= 1) {
         const int r = r0 + wave;
         float* pb = part + buf * (4 * 16 * 64);
         if (r < nr) {
-          lg_load<TX>(rb, S, d_of(r, 1));
+          lg_load<TX, G>(rb, S, d_of(r, 1));
           __builtin_amdgcn_sched_barrier(0);
-          lg_half<TX, true>(ra, acc);
+          lg_half<TX, G, true>(ra, acc);
           __builtin_amdgcn_sched_barrier(0);
-          lg_load<TX>(ra, S, d_of(r + 4, 0));  // (past the end: zeros, unused)
+          lg_load<TX, G>(ra, S, d_of(r + 4, 0));  // (past the end: zeros, unused)
           __builtin_amdgcn_sched_barrier(0);
-          lg_half<TX, false>(rb, acc);
+          lg_half<TX, G, false>(rb, acc);
 #pragma unroll
           for (int i = 0; i < 16; ++i) pb[(wave * 16 + i) * 64 + lane] = acc[i];
         }
@@ -593,17 +614,17 @@ __global__ __launch_bounds__(NT) void router_mf_kernel(RouterArgs a) {
       float lgt[4 * G];
 #pragma unroll
       for (int i = 0; i < 4 * G; ++i) lgt[i] = 0.0f;
-      lg_load<TX>(ra, S, d_of(0, 0));
+      lg_load<TX, G>(ra, S, d_of(0, 0));
       // (the scheduling barriers keep each half's loads issued before the
       // other half's products instead of next to their own uses)
       for (int r = 0; r < nr; ++r) {
-        lg_load<TX>(rb, S, d_of(r, 1));
+        lg_load<TX, G>(rb, S, d_of(r, 1));
         __builtin_amdgcn_sched_barrier(0);
-        lg_half<TX, true>(ra, acc);
+        lg_half<TX, G, true>(ra, acc);
         __builtin_amdgcn_sched_barrier(0);
-        lg_load<TX>(ra, S, d_of(r + 1, 0));  // (past the end: zeros, unused)
+        lg_load<TX, G>(ra, S, d_of(r + 1, 0));  // (past the end: zeros, unused)
         __builtin_amdgcn_sched_barrier(0);
-        lg_half<TX, false>(rb, acc);
+        lg_half<TX, G, false>(rb, acc);
         // chunks past the last are +0 partials, which change no logit (a sum
         // from +0, never -0)
 #pragma unroll
