@@ -357,14 +357,15 @@ void set_schedule(MoeOp& o) {
   if (o.int8_kernels()) {
     o.bm1 = o.bm2 = 256;  // tile schedules are not used by the int8 kernels
   } else if (o.mfma) {
-    // Unless a family was requested, the scheduled kernel: it plans 256 x 256
-    // and 128 x 128 tiles from the experts' row counts.  bm is then the height
-    // that most rows run at: 256 where the columns allow and the launch has
-    // at least two such tiles per CU.
+    // What mxm_moe_info reports (these kernels find their own tiles): the
+    // height of the family's tiles, for the scheduled kernel the one that most
+    // rows run at -- 256 where the columns allow and the launch has at least
+    // two such tiles per CU.
     auto rows = [&](int ncols, int kd) {
+      const int family = mxm_mfma_family((int)NK, o.E, ncols, kd, o.family);
       const int64_t tiles = ((int64_t)NK + 255) / 256 * (ncols / 256);
-      if (o.family == MXM_TILE_AUTO && (ncols % 256 != 0 || tiles < 2 * (int64_t)o.n_cu)) return 128;
-      return mxm_mfma_tile_rows(ncols, kd, o.family);
+      if (family == MXM_TILE_AUTO && (ncols % 256 != 0 || tiles < 2 * (int64_t)o.n_cu)) return 128;
+      return mxm_mfma_tile_rows(ncols, kd, family);
     };
     o.bm1 = rows(glu ? 2 * o.Fk : o.Fk, o.Kx);
     o.bm2 = rows(o.Dk, o.hsplit ? 2 * o.Fk : o.Fk);

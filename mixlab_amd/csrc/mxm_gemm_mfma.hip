@@ -1119,30 +1119,30 @@ int mxm_mfma_tile_rows(int Ncols, int Kd, int family) {
   }
 }
 
+int mxm_mfma_family(int rows, int E, int Ncols, int Kd, int family) {
+  if (family != MXM_TILE_AUTO) return family;
+  // 128 x 128 tiles of a launch with evenly loaded experts, the last tile
+  // of each half full.  Between one and two of them per CU the pairs run
+  // them in one round (2000 tokens of D 1024 / E 16 / K 2 / ffn 2734, down:
+  // 312 tiles 43 us, 48 on the scheduled kernel; 6000 of D 512 / E 16 / ffn
+  // 1024: 407 tiles 17.2 / 20.2 us); below, the scheduled kernel's deeper
+  // ring is faster (219 tiles of 64 stages: 48 / 34 us), above, its big
+  // tiles (527: 29.7 / 26.8, 1040: 85 / 71).  A pair also overlaps one
+  // tile's epilogue with the other's products, which counts where tiles
+  // have few stages (6 and fewer: 20000 tokens of D 256, up 36.0 / 38.3 us,
+  // 12000 of D 384 52.4 / 54.9; at 8 stages 161 / 147), and 128 columns
+  // hold no big tile (23433 tokens, D 128: 15.7 / 18.5 us).
+  const int64_t tiles = ((int64_t)rows + 64 * (int64_t)E) / 128 * (Ncols / 128);
+  const int n_cu = persistent_grid(1);
+  return Ncols < 256 || Kd <= 384 || (tiles > n_cu && tiles <= 2 * n_cu) ? MXM_TILE_128x128
+                                                                        : MXM_TILE_AUTO;
+}
+
 void mxm_launch_gemm_mfma(const GemmArgs& args, hipStream_t s) {
   if (args.rows_total <= 0) return;
   GemmArgs a = args;
   a.a_off32 = !a.no_off32 && (size_t)a.rows_total * a.Kd * 2 < ((size_t)1 << 32);
-  int family = a.family;
-  if (family == MXM_TILE_AUTO) {
-    // 128 x 128 tiles of a launch with evenly loaded experts, the last tile
-    // of each half full.  Between one and two of them per CU the pairs run
-    // them in one round (2000 tokens of D 1024 / E 16 / K 2 / ffn 2734, down:
-    // 312 tiles 43 us, 48 on the scheduled kernel; 6000 of D 512 / E 16 / ffn
-    // 1024: 407 tiles 17.2 / 20.2 us); below, the scheduled kernel's deeper
-    // ring is faster (219 tiles of 64 stages: 48 / 34 us), above, its big
-    // tiles (527: 29.7 / 26.8, 1040: 85 / 71).  A pair also overlaps one
-    // tile's epilogue with the other's products, which counts where tiles
-    // have few stages (6 and fewer: 20000 tokens of D 256, up 36.0 / 38.3 us,
-    // 12000 of D 384 52.4 / 54.9; at 8 stages 161 / 147), and 128 columns
-    // hold no big tile (23433 tokens, D 128: 15.7 / 18.5 us).
-    const int64_t tiles =
-        ((int64_t)a.rows_total + 64 * (int64_t)a.E) / 128 * (a.Ncols / 128);
-    const int n_cu = persistent_grid(1);
-    if (a.Ncols < 256 || a.Kd <= 384 || (tiles > n_cu && tiles <= 2 * n_cu))
-      family = MXM_TILE_128x128;
-  }
-  switch (family) {
+  switch (mxm_mfma_family(a.rows_total, a.E, a.Ncols, a.Kd, a.family)) {
     case MXM_TILE_256x128:
       launch_family<256, 128, 2, 2, 2, 3, 32>(a, s);
       break;

@@ -273,6 +273,10 @@ enum { MXM_TILE_AUTO = 0, MXM_TILE_128x128 = 1, MXM_TILE_256x128 = 2, MXM_TILE_2
 // Row-tile height the MFMA launcher uses for a GEMM with these dimensions
 // (0: the family does not tile them).
 int mxm_mfma_tile_rows(int Ncols, int Kd, int family);
+// The family that a launch of these sizes takes (rows: routed rows in all);
+// MXM_TILE_AUTO: the scheduled kernel, which plans 256 x 256 and 128 x 128 tiles
+// from the experts' row counts.
+int mxm_mfma_family(int rows, int E, int Ncols, int Kd, int family);
 
 // Weight gradients on MFMA (mxm_wgrad.hip): per expert e,
 //   out[e][m][c] = sum_p sum_k A[k][ap * aplane + m] * B[k][bp * bplane + c]   (fp32)

@@ -220,14 +220,15 @@ def test_mfma_families_many_tiles(gpu_lib, flow):
     assert err <= BF16_TOL, err
 
 
-@pytest.mark.parametrize("N,F,bm", [(2048, 256, 128), (16384, 1024, 256)])
-def test_mfma_family_auto(gpu_lib, N, F, bm):
+@pytest.mark.parametrize("N,D,F,bm", [(2048, 512, 256, 128), (16384, 512, 1024, 256),
+                                      (16384, 256, 1024, 128)])
+def test_mfma_family_auto(gpu_lib, N, D, F, bm):
     """Without a family flag a GEMM takes 256 x 256 tiles only when that
     gives at least two tiles per CU (2048 tokens x 2 slots, 2F = 512:
     16 x 2 = 32 tiles -> 128 x 128; 16384 x 2, 2F = 2048: 128 x 8 = 1024
-    tiles -> 256 x 256); either way routing is bit-exact and the delta
-    within the bf16 bar."""
-    D, E, K = 256, 8, 2
+    tiles -> 256 x 256) over a reduction of more than 384 (D 256: 128 x 128);
+    either way routing is bit-exact and the delta within the bf16 bar."""
+    E, K = 8, 2
     x, wr, experts = random_case(4343 + N, N, D, E, F)
     x, wr = round_bf16(x), round_bf16(wr)
     experts = [[round_bf16(m) for m in ws] for ws in experts]
