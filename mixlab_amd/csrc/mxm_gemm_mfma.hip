@@ -38,9 +38,9 @@
 //
 // Tile order: row tiles are grouped GM at a time with the column tiles of a
 // group adjacent, and each XCD (the hardware hands workgroup L to XCD L % 8)
-// takes a contiguous eighth of that list, so its L2 sees a GM x (N/BN) block
-// of tiles sharing A rows and B columns and every CU gets the same number of
-// tiles to within one.  The epilogue applies the activation (hardware exp2 /
+// takes an eighth of that list in whole groups (XcdPart), so its L2 sees a GM x
+// (N/BN) block of tiles sharing A rows and B columns and every CU gets the same
+// number of tiles to within one.  The epilogue applies the activation (hardware exp2 /
 // rcp and bf16 conversion), stages each wave's bf16 tile through LDS
 // (chunk-swizzled) and writes 16-byte row segments.
 #include <algorithm>
@@ -776,7 +776,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, u32x4_t* lds, int e
 // The plan is a function of the counts only, computed by every workgroup in
 // LDS (prefixes over the experts of the big and the small row tiles), so it
 // needs neither a launch before it nor a lookup in memory per tile.  Each XCD
-// (workgroup L runs on XCD L % 8) takes a contiguous eighth of the big tiles,
+// (workgroup L runs on XCD L % 8) takes an eighth of the big tiles (XcdPart),
 // in groups of GM row tiles by all column tiles, then of the small ones; the
 // workgroups that have one big tile fewer start the small ones.
 //
@@ -859,6 +859,32 @@ __device__ __forceinline__ void sched_place(int q, int nrow, int ncol, int& mt, 
   nt = rr / rig;
 }
 
+// An XCD's part of a list of n tiles in groups of `chunk` (GM row tiles by all
+// column tiles): every eighth group, so that at any time all XCDs work on the
+// same few experts, whose weights then come from the last-level cache the second
+// time; what is left past whole eights of groups in contiguous eighths, so that
+// all CUs get the same number of tiles to within one.  (Contiguous eighths of
+// the whole list keep eight experts' weights in use at once: forwards of 65536
+// tokens of D 2048 / E 64 / K 8 / ffn 5468, 360 MB of them, 33.0 ms, 31.6 like
+// this; 32768 of D 2048 / E 8 / K 2 / ffn 8192 6.14 -> 5.95.)
+struct XcdPart {
+  int xcd, chunk, whole, base, size;  // whole: tiles of this XCD in whole groups
+  __device__ __forceinline__ XcdPart(int64_t n, int chunk_, int xcd_) : xcd(xcd_), chunk(chunk_) {
+    const int eights = (int)(n / (8 * (int64_t)chunk));
+    const int64_t rest = n - (int64_t)eights * 8 * chunk;
+    const int lo = (int)(rest * xcd / 8);
+    whole = eights * chunk;
+    base = (int)(n - rest) + lo;
+    size = whole + (int)(rest * (xcd + 1) / 8) - lo;
+  }
+  // place in the list of this XCD's tile p (< size)
+  __device__ __forceinline__ int operator()(int p) const {
+    if (p >= whole) return base + p - whole;
+    const int g = p / chunk;
+    return (g * 8 + xcd) * chunk + p - g * chunk;
+  }
+};
+
 template <int EPI>
 __global__ __launch_bounds__(512, 1) void gemm_sched_kernel(GemmArgs a, int whole) {
   static_assert(BigTile::NS * BigTile::BUF == SmallTile::NS * SmallTile::BUF &&
@@ -889,23 +915,23 @@ __global__ __launch_bounds__(512, 1) void gemm_sched_kernel(GemmArgs a, int whol
   const int Ns = S0 + 4 * (B - Bm);
   // this XCD's part of both lists, and this workgroup's place in it
   const int xcd = blockIdx.x & 7, s = blockIdx.x >> 3, W = G >> 3;
-  const int lo = (int)((int64_t)Bm * xcd / 8), hi = (int)((int64_t)Bm * (xcd + 1) / 8);
+  const XcdPart part(Bm, GM * max(ncb, 1), xcd);
   const int slo = (int)((int64_t)Ns * xcd / 8), sn = (int)((int64_t)Ns * (xcd + 1) / 8) - slo;
   bool first = true;
-  for (int p = lo + s; p < hi; p += W) {
+  for (int p = s; p < part.size; p += W) {
     // every wave has read the previous tile's epilogue staging out of LDS
     // (plain s_barrier: no wait for that epilogue's stores)
     if (!first) asm volatile("s_barrier" ::: "memory");
     first = false;
     int mt, nt;
-    sched_place(p, BR, ncb, mt, nt);
+    sched_place(part(p), BR, ncb, mt, nt);
     const int e = uni(sched_find(S.big, E, mt));
     const int row0 = uni(S.off[e] + (mt - S.big[e]) * 256);
     const int rows = min(256, uni(S.off[e + 1]) - row0);
     gemm_tile<BigTile, 256, 256, 2, 4, EPI>(a, lds, e, row0, rows, nt * 256);
   }
   if (whole) return;
-  const int odd = (hi - lo) % W;              // workgroups with one big tile more
+  const int odd = part.size % W;              // workgroups with one big tile more
   const int idle = odd > 0 ? W - odd : 0;     // ... and the rest, which start
   const int ahead = SMALL_PER_BIG * idle;
   for (int k = (idle > 0 && s >= odd) ? 0 : SMALL_PER_BIG;; ++k) {
@@ -978,11 +1004,11 @@ __global__ __launch_bounds__(TL::NT, TL::WPS * 256 / TL::NT) void gemm_kernel(Ge
   const int ncol = a.Ncols / BN;
   const int64_t T = (int64_t)BR * ncol;
   const int xcd = blockIdx.x & 7, s = blockIdx.x >> 3, W = gridDim.x >> 3;
-  const int lo = (int)(T * xcd / 8), hi = (int)(T * (xcd + 1) / 8);
-  for (int p = lo + s; p < hi; p += W) {
-    if (p != lo + s) asm volatile("s_barrier" ::: "memory");  // as above
+  const XcdPart part(T, GM * ncol, xcd);
+  for (int p = s; p < part.size; p += W) {
+    if (p != s) asm volatile("s_barrier" ::: "memory");  // as above
     int mt, nt;
-    sched_place(p, BR, ncol, mt, nt);
+    sched_place(part(p), BR, ncol, mt, nt);
     int e, row0, rend;
     if (lanes) {
       e = __popcll(__ballot(pre <= mt));  // (lanes past E hold BR > mt)

@@ -17,13 +17,13 @@ pytestmark = pytest.mark.gpu
 # K = E gives every expert all N rows: remainders of 1, 127, 128, 129, 255 and
 # 0 rows past multiples of 256; widths with and without a last 128 columns.  The
 # reductions of up to 384 run on the 128 x 128 kernel with and without the flag
-# (its own edges, 200 and 70 experts on its LDS prefixes among them), the longer
-# ones on a plan of quarter tiles.
+# (its own edges, 200 and 70 experts on its LDS prefixes and 98 row tiles in whole
+# groups per XCD among them), the longer ones on a plan of quarter tiles.
 CASES = [
     (257, 128, 2, 2, 128, 0), (383, 256, 3, 3, 128, 0), (384, 384, 2, 2, 256, 0),
     (385, 192, 2, 2, 320, 1), (511, 640, 2, 2, 384, 2), (512, 128, 1, 1, 640, 0),
     (2600, 256, 2, 2, 2048, 0), (3300, 128, 3, 3, 2560, 0), (4100, 320, 2, 2, 896, 1),
-    (1300, 256, 200, 8, 128, 0), (1500, 256, 70, 1, 256, 0),
+    (1300, 256, 200, 8, 128, 0), (1500, 256, 70, 1, 256, 0), (6200, 128, 2, 2, 256, 0),
 ]
 
 
@@ -53,7 +53,8 @@ def plan(counts, ncols, cus):
 # workgroups of one big tile more than the rest and small tiles handed to the
 # rest first; several big tiles per workgroup; the last 128 columns of an odd
 # number; big tiles of 129 and of 228 rows, remainders of 1 and 127; 70 and 200
-# experts (prefixes over several waves, some experts empty).
+# experts (prefixes over several waves, some experts empty); 108 row tiles, of
+# which the XCDs take two whole groups of 6 each in turn, then eighths of the rest.
 PLAN_CASES = [
     (2600, 512, 2, 2, 2048, 0, dict(run=256, cut=64, small=2)),
     (2600, 512, 2, 2, 1024, 0, dict(run=160, cut=0, small=2, odd=20)),
@@ -62,6 +63,8 @@ PLAN_CASES = [
     (385, 448, 2, 2, 5120, 0, dict(run=160, cut=0, small=0, partial=True)),
     (257, 448, 3, 3, 5632, 0, dict(run=132, cut=0, small=3)),
     (383, 500, 3, 3, 5632, 1, dict(run=132, cut=0, small=3)),
+    (9000, 448, 3, 3, 512, 0, dict(run=420, cut=0, small=3, deep=2, odd=20)),
+    (9001, 500, 3, 3, 384, 0, dict(run=256, cut=59, small=3)),
     (6000, 512, 70, 1, 512, 0, dict(cut=0, deep=1)),
     (1500, 512, 200, 8, 512, 0, dict(run=0, cut=0, small=200)),
 ]
