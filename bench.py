@@ -41,12 +41,12 @@ def stage_bytes(cfg) -> dict:
     N, D, E, K = cfg.N, cfg.D, cfg.E, cfg.K
     xb = 2 if cfg.dtype == "bf16" else 4
     NK = N * K
-    tiles = (N + 63) // 64
+    tiles = -(-N // (16 if N <= 16384 else 64))  # of the tiled router
     return {
         # x read, router weights, top_idx + gates + ranks written, tile partials
         "router": N * D * xb + D * E * xb + NK * 12 + tiles * E * 8,
-        # top_idx, ranks, tile bases read; perm, slot_pos written
-        "scatter": NK * 4 * 2 + NK * 4 * 2,
+        # the dispatch: tile partials, top_idx, ranks read; perm, slot_pos written
+        "scan": tiles * E * 8 + NK * 4 * 2 + NK * 4 * 2,
         # K rows of y per token, gates + idx + pos, delta written fp32
         "combine": NK * D * (2 if cfg.dtype == "bf16" else 4) + NK * 12 + N * D * 4,
     }
@@ -585,7 +585,7 @@ def main() -> int:
                    "expert": "sigmoid-GLU (swiglu)" if cfg.expert_type == 0 else str(cfg.expert_type),
                    "parallelism": "single GPU"},
         "roofline": {"bound": "mfma",
-                     "kernel": "gemm_kernel, the grouped GEMM of one forward (gate+up launch "
+                     "kernel": "gemm_sched_kernel, the grouped GEMM of one forward (gate+up launch "
                                "with GLU epilogue + down launch)",
                      "achieved": gg["tflops"], "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": gg["frac"], "traffic": gemm_traffic(cfg.name, args.flags)},

@@ -69,7 +69,11 @@ extern "C" {
  * reference (its graph keeps them implicitly). */
 #define MXM_FLAG_KEEP_FOR_BACKWARD 32
 
-/* Stages timed by mxm_moe_stage_times, in launch order. */
+/* Stages timed by mxm_moe_stage_times, in launch order.  ROUTER includes the
+ * zero-padded copy of x where D is not a multiple of 64 (the router reads it);
+ * SCAN is the dispatch (counts, offsets, permutation, aux and entropy) of the
+ * tiled router's batches, all of it: SCATTER has no launch of its own and times
+ * an empty gap. */
 #define MXM_STAGE_ROUTER 0
 #define MXM_STAGE_SCAN 1
 #define MXM_STAGE_SCATTER 2
@@ -278,15 +282,15 @@ int mxm_moe_stage_times(int64_t op, float* ms, int n);
  * than 96 routed rows per expert, not created with
  * MXM_FLAG_KEEP_FOR_BACKWARD; they hold the weights in both layouts, and
  * their backward runs on the tiles), info[1] = workspace bytes, info[2] = row-tile
- * height of the grouped GEMM, info[3] = number of router tiles, info[4] = the
+ * height that the up projection's kernel runs most rows at, info[3] = number of router tiles, info[4] = the
  * expert width the kernels run at (ffn, or ffn rounded up to the tiles: 128
  * for MFMA, 64 for the int8 kernels, with zero weights in the padding),
  * info[5] = the down
  * projection's output width (D, or D rounded up to 128 / 16), info[6] = the
  * up projection's reduction length (D, or D rounded up to 64), info[7] = how
- * the last forward routed: 0 the tiled router, scan and scatter (three
- * launches), 1 the one-launch router (a workgroup per token, the dispatch in
- * its last workgroup), 2 the decode flow of the decode kernels (int8, or
+ * the last forward routed: 0 the tiled router and the dispatch (two launches,
+ * three for many tiles), 1 the one-launch router (a workgroup per token, or per
+ * four past 256, the dispatch in its last workgroup), 2 the decode flow of the decode kernels (int8, or
  * bf16 streamed: the one-launch router's per-token results only; the expert
  * kernels find their rows from the top-k picks), -1 no forward yet.  Returns the number of entries written (at most
  * n, at most 8). */

@@ -209,12 +209,12 @@ struct MoeOp {
   // backward (fp32 flow): the experts' projections, gradients and scratch
   bool keep_probs = false, bw_ready = false;
   // set by the fp32 backward around its forward: stop after the routing
-  // (router, scan, scatter); the backward computes the experts' products itself
+  // (router, dispatch); the backward computes the experts' products itself
   bool route_only = false;
   bool up_only = false;  // the forward stops after the up projection (MFMA backward)
   // MXM_FLAG_KEEP_FOR_BACKWARD: the last call was an mxm_moe_forward, which
-  // kept its own copy of x and (MFMA backward family) its routing,
-  // probabilities and raw up projections for mxm_moe_backward_kept
+  // kept its own copy of x, its routing and probabilities and (MFMA backward
+  // family) its raw up projections for mxm_moe_backward_kept
   bool train = false, kept = false;
   DevBuf kept_xbuf;
   int kept_dtype = -1;
@@ -602,7 +602,7 @@ void run_forward(MoeOp& o, const Workspace& w, const void* x, int x_dtype, float
     da.aux_scaled = blk ? blk->aux_scaled : nullptr;
     for (int rep = 0; rep < reps; ++rep) mxm_launch_dispatch(da, o.bf16, st);
     HIPCK(hipGetLastError());
-    mark(2);  // (the scatter stage is part of the dispatch launch)
+    mark(2);  // (the scatter stage is part of the dispatch launch: an empty gap)
   }
 
   mark(3);

@@ -7,10 +7,17 @@
 
 #include "mxm_numerics.h"
 
-// Tokens per router tile; the dispatch bitmasks are two 32-bit words per
-// expert and tile, so this is fixed at 64.
+// Most tokens per tile of the tiled router (the other size is 16): a tile's
+// bitmasks are two 32-bit words per expert.
 #define MXM_ROUTER_TM 64
-// Batches of up to this many tokens take tiles of 16 on the tiled router.
+// Batches of up to this many tokens take tiles of 16 on the tiled router, where
+// the matrix cores take their rows.  Whole forwards of small experts on tiles of
+// 64 / 16, fp32: E 64 / D 2048 at 8192 tokens 296 / 277 us, 12288 343 / 333, 16384
+// 469 / 485 (256 tiles of 64: one round of the CUs), 20480 549 / 527, 24576 659
+// / 647, 32768 819 / 836; E 8 / D 512 84 / 82, 92 / 90, 118 / 120, 134 / 133, 159 /
+// 161, 194 / 201; E 256 / D 512 152 / 129, 181 / 177, 195 / 196, 237 / 223, 266 /
+// 262, 312 / 330.  Above the line tiles of 16 gain at most a few per cent on some
+// sizes and lose as much on others, for four times the histograms.
 #define MXM_ROUTER_SPLIT_N 16384
 // Largest expert count the router supports (4 experts per lane).
 #define MXM_MAX_EXPERTS 256
@@ -72,10 +79,10 @@ struct RouterArgs {
 void mxm_launch_router(const RouterArgs& a, bool bf16, hipStream_t s);
 
 // Decode-sized batches (N <= MXM_SMALL_BATCH, N*K <= MXM_SMALL_SLOTS,
-// D <= MXM_SMALL_D) route in one launch: a workgroup per token computes its
-// logits, softmax, top-k and gates, and the last workgroup to finish (an
-// atomic ticket) computes counts, offsets, row-tile prefixes, the stable
-// permutation, aux and entropy -- the work of the router, scan and scatter
+// D <= MXM_SMALL_D) route in one launch: a workgroup per token (or per four)
+// computes its logits, softmax, top-k and gates, and the last workgroup to
+// finish (an atomic ticket) computes counts, offsets, row-tile prefixes, the
+// stable permutation, aux and entropy -- the work of the router and dispatch
 // kernels of larger batches.
 #define MXM_SMALL_BATCH 1024
 #define MXM_SMALL_SLOTS 16384

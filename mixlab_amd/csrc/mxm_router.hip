@@ -18,7 +18,7 @@
 // into the stable permutation.
 //
 // Decode-sized batches take route_small_kernel instead (one launch for the
-// router, scan and scatter; see below).  Both kernels run the per-token
+// router and the dispatch; see below).  Both kernels run the per-token
 // softmax / top-k / gate code of route_token, so their routing is the same
 // bit for bit.
 #include <algorithm>
@@ -738,9 +738,9 @@ __global__ __launch_bounds__(NT) void router_kernel(RouterArgs a) {
 // lane-interleaved (each wave load is 1 KB contiguous: 16 bytes = the lane's expert's next 4 or 8 d),
 // and the next pieces are in flight while a chunk is summed.  A wave per
 // token then runs route_token and writes the token's picks, gates, probabilities and
-// entropy term.  Every workgroup then takes a ticket (wave 0: agent-scope
-// fence, atomic add); the one that takes the last ticket reads all tokens'
-// results back and computes what the scan and scatter kernels compute for
+// entropy term.  Every workgroup then takes a ticket (an agent-scope fence in
+// each wave that stored, then wave 0's atomic add); the one that takes the last ticket reads all tokens'
+// results back and computes what the dispatch kernel computes for
 // larger batches: per-expert counts (LDS histogram), offsets and row-tile
 // prefixes (wave scans), aux and entropy, and the stable permutation (per
 // 64-token chunk, the rank of a slot among the chunk's tokens on its expert
