@@ -292,22 +292,20 @@ int fenced(F&& f) {
     return MXM_ERR_OP;                                  \
   }
 
-// Whether a batch that the one-launch router can take is faster there than
-// on the tiled router + scan + scatter.  The one-launch router's time grows
-// with N (a workgroup per token, then one workgroup's dispatch of the N*K
-// slots); the three-launch path's hardly does at these sizes.  So the one
-// launch pays while each token brings enough logit work.  Measured on MI355X
-// over N = 64-1024 and D*E = 512 .. 131072 (bf16 and fp32; results are bit
-// for bit the same either way): where the tiled router's logits run on the
-// matrix cores (mf) and E <= 64 it is the faster one for every N <= 640,
-// up to N = 768 from D*E = 8192 on, up to N = 896 from D*E = 65536 on and
-// up to N = 1024 from D*E = 98304 on; for E > 64 for every N <= 512, up to
-// N = 768 from D*E = 4096 on and up to N = 1024 from D*E = 16384 on (with
-// or without the matrix-core logits: the tiled router has only N / 64
-// workgroups at these sizes); for
-// E <= 32, where the tiled router routes several tokens per wave, the
-// crossover lies near N = 200-300 for D*E = 512, ~400 for 4096, ~550 for
-// 8192 and ~700 for 16384.  The int8 decode flow is built on the one-launch
+// Whether a batch that the one-launch router can take goes there instead of to
+// the tiled router and its dispatch.  The one-launch router's time grows with N
+// (a workgroup per token or per four, then one workgroup's dispatch of the N*K
+// slots); the tiled router's hardly does at these sizes.  The lines below were
+// measured against a tiled router of 64-token tiles (logits on the matrix cores
+// for E > 32 only) with a scan and a scatter launch after it.  Against the
+// present one they hold the one launch too long: whole forwards, one launch /
+// tiled, at 64, 256 and 1024 tokens, bf16 E 8 / D 512 26.5 / 26.3, 36.0 / 27.0, 76.0
+// / 28.5 us; E 64 / D 2048 41.2 / 55.2, 51.5 / 56.6, 98.0 / 59.4; E 256 / D 1024
+// 50.8 / 75.8, 81.2 / 86.8, 177 / 93.5; fp32 E 16 / D 1024 77.1 / 75.5, 85.7 / 76.9,
+// 130 / 82.3 -- the times cross near 64 tokens for E <= 32 and between 130 and 300
+// above.  They are left where they are because the two paths sum aux and the
+// entropy in different orders (the routing is the same bit for bit) and
+// mxm_moe_info reports the path.  The decode flow is built on the one-launch
 // router and keeps it wherever it fits.
 bool small_route_pays(int N, int D, int E, bool mf) {
   const int64_t de = (int64_t)D * E;
@@ -1129,7 +1127,8 @@ int64_t mxm_moe_create(const float* float_params, int n_float_params, const int3
     const size_t F1 = (size_t)o->Kx * o->Fk, F2 = (size_t)o->Fk * o->Dk;  // padded matrices
     o->router.alloc(DE * (o->bf16 ? 2 : 4));
     if (const char* v = std::getenv("MXM_ROUTER_MFMA")) o->mf_router = std::atoi(v) != 0;
-    // (the launcher also wants x 16-byte aligned; D decides it for the choice)
+    // (of the choice's lines; the tiled router itself takes its logits on the
+    // matrix cores for every E)
     const bool mf_logits =
         o->mf_router && o->E > 32 && o->D % (o->bf16 ? 8 : 4) == 0 && o->D <= (1 << 24);
     o->small_route = mxm_route_small_fits(o->N, o->D, o->E, o->K) &&

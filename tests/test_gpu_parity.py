@@ -244,10 +244,9 @@ def test_mfma_family_auto(gpu_lib, N, D, F, bm):
 @pytest.mark.parametrize("N", [1100, 2049])
 @pytest.mark.parametrize("bf16", [False, True])
 def test_tiled_scan_few_experts(gpu_lib, E, K, N, bf16):
-    """The tiled router and the scan's one workgroup per expert at the
-    smallest expert counts (E = 1: the only expert workgroup is also the
-    last ticket), a ragged last token tile, and two calls on one op (the last
-    workgroup resets the ticket for the next call)."""
+    """The tiled router and its dispatch at the smallest expert counts (E = 1:
+    every slot on one expert), a ragged last token tile, and two calls on one
+    op (neither leaves anything that the next one reads)."""
     from mixlab_amd.op import MoEFeedForward
 
     D, F = 128, 128
@@ -861,7 +860,7 @@ def test_decode_router_shapes(gpu_lib, monkeypatch, N, D, E, K, bf16):
 
 
 # (N, D, E, K, dtype, int8, the router the library picks): 0 tiled router +
-# scan + scatter, 1 the one-launch router, 2 the int8 decode flow
+# dispatch, 1 the one-launch router, 2 the int8 decode flow
 ROUTER_CHOICE = [
     # E <= 32 (the tiled router takes several tokens per wave)
     (1024, 128, 4, 2, "fp32", False, 0),    # C1, the reference's moe_tiny scale: D*E = 512
