@@ -1494,7 +1494,7 @@ def test_stage_profiling_repeats(gpu_lib, T):
     """Profiled forwards that launch each stage several times between its
     events (mxm_moe_set_profiling with R > 1) leave the outputs unchanged:
     every stage is idempotent, on the one-launch router (T=64) and on the
-    tiled router + scan + scatter (T=1536)."""
+    tiled router and its dispatch (T=1536)."""
     from mixlab_amd.op import MoEFeedForward
 
     D, E, K, F = 256, 8, 2, 256
